@@ -50,6 +50,26 @@ def test_elasticity_operator_parity(dim, p, n):
     assert rel_err(host(y32), ref.operator(x.astype(np.float32).astype(np.float64))) < 1e-6
 
 
+# cells per block: 64 / (p+1)^(dim-1); last blocks with one cell, full ones, fewer cells
+# than a block, cells with boundary faces on both sides of a direction
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 2), (2, 3, 4), (2, 4, 5), (2, 2, 2), (3, 1, 2),
+                                     (3, 2, 2), (3, 1, 5), (3, 3, 2), (3, 4, 2), (3, 2, 7)])
+def test_elasticity_operator_block_edges(dim, p, n):
+    t = _tpss()
+    ref = o.Smoother(dim, p, n, ip=3.0, elasticity=(0.7, 2.5))
+    x, b = o.splitmix_uniform(3, ref.N), o.splitmix_uniform(4, ref.N)
+    for prec, dt, bar in ((t.F64, np.float64, 1e-12), (t.F32, np.float32, 1e-6)):
+        lv = t.Level(dim, p, n, ip_factor=3.0, elasticity=(0.7, 2.5), precision=prec)
+        xs, bs = x.astype(dt), b.astype(dt)
+        Ax = ref.operator(xs.astype(np.float64))
+        y = dev(np.full(ref.N + 8, 7.0, dt))  # guard values behind the output
+        lv.vmult(y, dev(xs))
+        assert rel_err(host(y)[:ref.N], Ax) < bar
+        assert (host(y)[ref.N:] == 7.0).all()
+        lv.residual(y, dev(bs), dev(xs))
+        assert rel_err(host(y)[:ref.N], bs - Ax) < bar
+
+
 @pytest.mark.parametrize("dim,p,n", [(2, 2, 6), (3, 2, 4)])
 def test_elasticity_index_tables_bit_exact(dim, p, n):
     t = _tpss()

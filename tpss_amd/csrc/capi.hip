@@ -46,36 +46,61 @@ constexpr int cells_per_block()
   return ndc >= 256 ? 1 : 256 / ndc;
 }
 
-// y = A x (or y = b - A x), optionally only on a list of cells; vectors of type VT
+// the 1D matrices of k_elasticity, formed in FP64
 template<int NP, typename T>
 ElastTab<NP, T> make_elast_tab(const tpss_level *lv)
 {
   ElastTab<NP, T> tab;
   const Basis1D bs = make_basis(NP - 1);
-  const double h = lv->h;
-  for(int q = 0; q < NP; ++q)
-  {
-    tab.w[q] = T(h * bs.qw[q]);
-    for(int i = 0; i < NP; ++i)
-    {
-      tab.V[q * NP + i] = T(bs.val[i * NP + q]);
-      tab.G[q * NP + i] = T(bs.grad[i * NP + q] / h);
-    }
-  }
-  for(int f = 0; f < 2; ++f)
-    for(int i = 0; i < NP; ++i)
-    {
-      tab.f[f][i] = T(bs.fval[i * 2 + f]);
-      tab.fd[f][i] = T(bs.fgrad[i * 2 + f] / h);
-    }
+  const double h = lv->h, mu = lv->mu, la = lv->lambda;
   const int p = NP - 1;
-  const double gamma = p == 0 ? 1.0 : double(p) * (p + 1);
-  tab.mu = T(lv->mu);
-  tab.lambda = T(lv->lambda);
-  tab.sigma = T(lv->ip * gamma / h);  // Laplace::compute_penalty of two cells of size h
+  const double sigma = lv->ip * (p == 0 ? 1.0 : double(p) * (p + 1)) / h;
+  const double aA = 2.0 * mu + la, aB = mu, pA = (2.0 * mu + la) * sigma, pB = 2.0 * mu * sigma;
+  for(int i = 0; i < NP; ++i)
+    for(int j = 0; j < NP; ++j)
+    {
+      double m = 0, st = 0, gij = 0, gji = 0;
+      for(int q = 0; q < NP; ++q)
+      {
+        const double vi = bs.val[i * NP + q], vj = bs.val[j * NP + q];
+        const double gi = bs.grad[i * NP + q], gj = bs.grad[j * NP + q];
+        m += vi * vj * h * bs.qw[q];
+        st += gi * gj / h * bs.qw[q];
+        gij += vi * gj * bs.qw[q];
+        gji += vj * gi * bs.qw[q];
+      }
+      // the cell's own half of its two interior faces: sides 0 (s = +1) and 1 (s = -1)
+      double cons = 0;
+      for(int f = 0; f < 2; ++f)
+      {
+        const double vi = bs.fval[i * 2 + f], vj = bs.fval[j * 2 + f];
+        const double gi = bs.fgrad[i * 2 + f] / h, gj = bs.fgrad[j * 2 + f] / h;
+        cons += (f == 0 ? 0.5 : -0.5) * (vi * gj + gi * vj);
+      }
+      tab.M[i * NP + j] = T(m);
+      tab.K[i * NP + j] = T(0.5 * (gij - gji));
+      tab.LA[i * NP + j] = T(aA * (st + cons));
+      tab.LB[i * NP + j] = T(aB * (st + cons));
+    }
+  for(int f = 0; f < 2; ++f)
+    for(int i = 0; i < NP; ++i) tab.g[f][i] = T(bs.fgrad[i * 2 + f] / h);
+  tab.aA = T(0.5 * aA);
+  tab.aB = T(0.5 * aB);
+  tab.pA = T(pA);
+  tab.pB = T(pB);
+  for(int k = 0; k < 2; ++k)
+  {
+    const double e = k == 0 ? 1.0 : -1.0;
+    tab.h1K[k] = T(0.5 * (e * la + mu));
+    tab.h1B[k] = T(0.25 * (e * la - mu));
+    tab.h2K[k] = T(0.5 * (e * mu + la));
+    tab.h2B[k] = T(0.25 * (e * mu - la));
+  }
+  tab.kappa = T(-(mu + la));
   return tab;
 }
 
+// y = A x (or y = b - A x), optionally only on a list of cells; vectors of type VT
 template<typename VT>
 void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const uint32_t *cells,
                     int64_t n_list, hipStream_t s)
@@ -84,20 +109,17 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
   {
     dispatch_dim_np(lv->dim, lv->np, [&](auto D, auto NPc) {
       constexpr int DIM = decltype(D)::value, NP = decltype(NPc)::value;
-      constexpr int NDC = cpow(NP, DIM);
-      const auto tab = make_elast_tab<NP, VT>(lv);
       const int64_t count = cells ? n_list : lv->ncell;
       if(count == 0) return;
-      (void)NDC;
-      constexpr int CPB = elasticity_cells_per_block<DIM, NP>();
-      const unsigned threads = unsigned(elasticity_threads<DIM, NP>());
-      const unsigned grid = blocks_for(count, CPB);
+      // eight equal shares of blocks, one per XCD
+      const auto tab = make_elast_tab<NP, VT>(lv);
+      const unsigned grid = (blocks_for(count, elasticity_cells_per_block<DIM, NP>()) + 7) / 8 * 8;
       if(b)
-        hipLaunchKernelGGL((k_elasticity<DIM, NP, VT, true>), dim3(grid), dim3(threads), 0, s, x,
-                           y, b, tab, lv->n, lv->Ns, cells, count);
+        hipLaunchKernelGGL((k_elasticity<DIM, NP, VT, true>), dim3(grid), dim3(64), 0, s, x, y, b,
+                           tab, lv->n, lv->Ns, cells, count);
       else
-        hipLaunchKernelGGL((k_elasticity<DIM, NP, VT, false>), dim3(grid), dim3(threads), 0, s, x,
-                           y, b, tab, lv->n, lv->Ns, cells, count);
+        hipLaunchKernelGGL((k_elasticity<DIM, NP, VT, false>), dim3(grid), dim3(64), 0, s, x, y, b,
+                           tab, lv->n, lv->Ns, cells, count);
       TPSS_HIP(hipGetLastError());
     });
     return;

@@ -9,21 +9,10 @@
 //             grad u_out = grad u_in (penalty 2 sigma, Dirichlet u = 0)
 // sigma = ip * gamma / h, gamma = p (p + 1).
 //
-// Vectors are component-blocked: x[c * Ns + cell * NDC + local].  CPB cells per
-// block (64 / NDC for small cells), one thread per cell DoF / quadrature point
-// (QGauss(p+1)) handling all components; arithmetic in the vector type.
-//   cell term: the gradients of all components by sum factorisation (x, y, z
-//     stages sharing their 1D interpolations), the stress times JxW, and its
-//     integration against the test gradients (z, y, x stages);
-//   faces, one direction at a time (both faces of the cell): traces of both
-//     sides contracted along the normal (the neighbour's straight from global
-//     memory; the face neighbours' cell indices are formed once per block),
-//     fluxes per face point, fluxes projected on the tangential test
-//     functions (3D: sum-factorised, one tangential direction after the other,
-//     through the cell-stage arrays, which the faces leave free), and every
-//     thread adds the terms of its test function.
-// Faces are evaluated element-centrically (every output entry is written by
-// exactly one thread).
+// Vectors are component-blocked: x[c * Ns + cell * NDC + local]; arithmetic in the
+// vector type.  On uniform cells QGauss(p+1) integrates every term exactly, so the
+// form is evaluated as a sum of Kronecker products of 1D matrices, element-centrically
+// (every output entry is written by exactly one lane).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -35,511 +24,503 @@
 
 namespace tpss
 {
+// Per direction d, with K = 1/2 (G - G^T), G = int phi_i phi_j',
+// B = diag(-1, 0, .., 0, 1), M the mass and L_a the SIPG line matrix of a cell
+// (stiffness and its half of the consistency terms, without penalty) for the
+// stiffness factor a (2 mu + lambda along the component, mu across; penalty factors
+// pi = 2 mu + lambda and 2 mu):
+//   own cell    y_c += sum_d L_d M M u_c,   y_a += -(mu + lambda) M (K_a K_c + 1/4 B_a B_c) u_c
+//   face (d, side) with the neighbour's trace (v, v'), s = +1 (left) or -1:
+//     y_c += (e_i P + (-s/2 a g_i) v) M M,  P = pi sigma (u - v) + s/2 a v'
+//     y_d += e_i s M H1 u_c,  H1 = h1K K + h1B B   (tangential direction c)
+//     y_a += e_i s M H2 u_d,  H2 = h2K K + h2B B   (tangential direction a)
+// (e_i: 1 at the node on the face; g_i = phi_i' there; the penalty acts on the jump
+// u - v, whose cancellation in FP32 a penalty inside L_a would lose).  A boundary face takes the
+// odd reflection of the cell as its neighbour (v = -u, v' = u'); only the
+// average of the mixed terms is even there, which flips one sign in the h's.  The
+// trace of a neighbour is its node value on the face (Gauss-Lobatto nodes) and one
+// NP-term product for the derivative.  (3D written out; 2D has no third mass factor.)
 template<int NP, typename T>
 struct ElastTab
 {
-  T V[NP * NP];   // V[q*NP + i] = phi_i(x_q)
-  T G[NP * NP];   // G[q*NP + i] = phi_i'(x_q) / h
-  T f[2][NP];     // phi_i(0), phi_i(1)
-  T fd[2][NP];    // phi_i'(0) / h, phi_i'(1) / h
-  T w[NP];        // h * Gauss weight
-  T mu, lambda, sigma;
+  T M[NP * NP], K[NP * NP];
+  T LA[NP * NP], LB[NP * NP];  // L along the component / across it
+  T g[2][NP];                  // phi_i'(0) / h, phi_i'(1) / h
+  T aA, aB;                    // 1/2 stiffness factor along / across
+  T pA, pB;                    // penalty factor times sigma
+  T h1K[2], h1B[2], h2K[2], h2B[2];  // [0] interior face, [1] boundary face
+  T kappa;                     // -(mu + lambda)
+};
+
+// Rows of N values moved through LDS in 16-byte chunks: chunk k of the row of lane
+// l sits at (k * LANES + l), so that the lanes' accesses are free of bank conflicts.
+template<int N, int LANES, typename T>
+struct LaneRows
+{
+  static constexpr int CW = 16 / int(sizeof(T)), NC = (N + CW - 1) / CW;
+  static constexpr int SIZE = NC * LANES * CW;
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  static __device__ __forceinline__ void put(T *buf, int lane, const T *v)
+  {
+#pragma unroll
+    for(int k = 0; k < NC; ++k)
+    {
+      vec w;
+#pragma unroll
+      for(int e = 0; e < CW; ++e) w[e] = k * CW + e < N ? v[k * CW + e] : T(0);
+      reinterpret_cast<vec *>(buf)[k * LANES + lane] = w;
+    }
+  }
+  static __device__ __forceinline__ void get(const T *buf, int lane, T *v)
+  {
+#pragma unroll
+    for(int k = 0; k < NC; ++k)
+    {
+      const vec w = reinterpret_cast<const vec *>(buf)[k * LANES + lane];
+#pragma unroll
+      for(int e = 0; e < CW; ++e)
+        if(k * CW + e < N) v[k * CW + e] = w[e];
+    }
+  }
 };
 
 template<int DIM, int NP>
 constexpr int elasticity_cells_per_block()
 {
-  return cpow(NP, DIM) >= 64 ? 1 : 64 / cpow(NP, DIM);
+  return 64 / cpow(NP, DIM - 1);
 }
 
-template<int DIM, int NP>
-constexpr int elasticity_threads()
+// Waves per SIMD the register allocation must allow (64^3 Q2: FP32 129 us unbounded,
+// 106 us with 3; FP64 290 us unbounded, 231 us with 2).  Longer lines would spill:
+// 3D Q3 FP32 24^3 15.1 us unbounded, 15.8 us with 3.
+template<int NP, typename T>
+constexpr int elasticity_min_waves()
 {
-  return ((elasticity_cells_per_block<DIM, NP>() * cpow(NP, DIM) + 63) / 64) * 64;
+  return std::is_same<T, float>::value ? (NP <= 3 ? 3 : 2) : (NP <= 4 ? 2 : 1);
 }
 
+// One lane per x-line (ly, lz) of a cell, 64 / NP^(DIM-1) cells per single-wave block
+// (its barriers cost nothing).  A lane holds its line of all components; the x
+// products run in registers.  The y products read the cell's lines from LDS, each
+// extended by the x-face traces of its lane (v, P on both sides), so that the x
+// faces need no exchange of their own; in 3D nine mixed rows per lane pass through
+// LDS for the z products.  The y- and z-face traces are formed by lanes that own a
+// tangential point (lines of the neighbour along the face normal), the z-face ones
+// contracted along y before the lanes of the lines read them as rows.
+// Blocks of one eighth of the launch run on one XCD, so that neighbours in y and z
+// are mostly found in its L2 (64^3 Q2 FP64 309 -> 290 us).
+// Bound by instruction issue and LDS together: 64^3 Q2 (21.2M DoFs, 170 MB in FP32)
+// FP32 106 us, FP64 231 us per apply; the quadrature form of the same operator
+// (tensor interpolation to Gauss points, fluxes per face point) took 618 / 1278 us.
 template<int DIM, int NP, typename VT, bool RESIDUAL>
-__global__ void __launch_bounds__((elasticity_threads<DIM, NP>()))
+__global__ void __launch_bounds__(64, (elasticity_min_waves<NP, VT>()))
 k_elasticity(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
              const ElastTab<NP, VT> tab, const int n, const int64_t Ns,
              const uint32_t *__restrict__ cells, const int64_t count)
 {
   using T = VT;
-  constexpr int NDC = cpow(NP, DIM);
-  constexpr int NF = cpow(NP, DIM - 1);
+  constexpr bool D3 = DIM == 3;
+  constexpr int NL = cpow(NP, DIM - 1), NDC = NL * NP, P = NP - 1;
   constexpr int CPB = elasticity_cells_per_block<DIM, NP>();
-  constexpr int NT = elasticity_threads<DIM, NP>();
-  constexpr int ST[3] = {1, NP, NP * NP};
-  constexpr int NS = DIM * DIM;  // stage arrays per cell
-  __shared__ T U[CPB][DIM][NDC];
-  __shared__ T R1[CPB][NS][NDC], R2[CPB][NS][NDC];  // stage arrays, used in turn
-  // normal traces [face side][cell side][component][tangential node]; later the
-  // projections of the fluxes on the tangential test functions ([.][0][.][.])
-  __shared__ T PA[CPB][2][2][DIM][NF], PB[CPB][2][2][DIM][NF];
-  __shared__ T FA[CPB][2][DIM][NF], FB[CPB][2][DIM][DIM][NF];
-  __shared__ int64_t nbc[CPB][2 * DIM];  // face neighbours [2 D + side] (-1: boundary face)
-  __shared__ ElastTab<NP, T> tl;
+  constexpr int NX = NP + 4;  // extended line: values, then v, P of the left and right x-face
+  using Ext = LaneRows<NX, 64, T>;
+  using Row = LaneRows<NP, 64, T>;
+  // face rows: entry lx of row (cell slot, tangential line); slots for idle lanes too
+  constexpr int FL = D3 ? NP : 1, FR = ((64 + NL - 1) / NL) * FL, NF = 4 * DIM;
+  using Face = LaneRows<NP, FR, T>;
+  constexpr int CW = Face::CW;
+  constexpr int S1 = DIM * Ext::SIZE + NF * Face::SIZE, S2 = D3 ? 9 * Row::SIZE : 0;
+  __shared__ __align__(16) T buf[S1 > S2 ? S1 : S2];  // y stage; then the z stage's rows
+  __shared__ __align__(16) T fz[D3 ? NF * Face::SIZE : 1];     // z-face traces, then contracted along y
+  constexpr int NTAB = int(sizeof(ElastTab<NP, T>) / sizeof(T));
+  __shared__ T tl[NTAB];
+  T *ext = buf, *fy = buf + DIM * Ext::SIZE;
+  // entry e of the line of lane l, component c
+  auto eidx = [](int c, int l, int e) { return c * Ext::SIZE + ((e / CW) * 64 + l) * CW + e % CW; };
+  // entry e of face row r in plane k; planes of the values v and of P
+  auto pv = [](int side, int c) { return side * 2 * DIM + c; };
+  auto pp = [](int side, int c) { return side * 2 * DIM + DIM + c; };
+  auto fidx = [](int k, int r, int e) { return k * Face::SIZE + ((e / CW) * FR + r) * CW + e % CW; };
 
-  const int t = threadIdx.x;
-  const int cs = t / NDC, ts0 = t % NDC;
-  const int64_t slot = int64_t(blockIdx.x) * CPB + cs;
+  const int t = threadIdx.x, cs = t / NL, q = t % NL;
+  const int cr = min(cs, CPB - 1);  // lanes beyond the last cell read its lines
+  const int q0 = q % NP, q1 = q / NP;  // (ly, lz) of the line; (lx, lz) / (lx, ly) of a face point
+  const int64_t nblk = gridDim.x, per = nblk / 8;  // the grid is a multiple of eight blocks
+  const int64_t blk = int64_t(blockIdx.x % 8) * per + blockIdx.x / 8;
+  const int64_t slot = blk * CPB + cs;
   const bool act = cs < CPB && slot < count;
-  const int c0 = cs < CPB ? cs : 0;  // LDS slot of this thread (idle threads alias slot 0)
-  const int ts = act ? ts0 : 0;
-  auto cell_of = [&](int s) -> int64_t {
-    const int64_t sl = int64_t(blockIdx.x) * CPB + s;
-    return sl < count ? (cells ? int64_t(cells[sl]) : sl) : int64_t(-1);
+  const int64_t sl = act ? slot : 0;
+  const int64_t cell = cells ? int64_t(cells[sl]) : sl;
+  const int ci = int(cell);
+  const int cx = ci % n, cy = (ci / n) % n, cz = D3 ? ci / (n * n) : 0;
+  const bool has[3][2] = {{cx > 0, cx < n - 1}, {cy > 0, cy < n - 1}, {cz > 0, cz < n - 1}};
+  const int64_t nn = int64_t(n) * n;
+  const T *xc = x + cell * NDC;
+
+  for(int i = t; i < NTAB; i += 64) tl[i] = reinterpret_cast<const T *>(&tab)[i];
+  // ---- loads: the lane's lines, the x-neighbours' lines and the neighbours' lines
+  // along y and z at the lane's tangential point
+  T u[DIM][NP], nx[2][DIM][NP], fl[DIM - 1][2][DIM][NP];
+#pragma unroll
+  for(int c = 0; c < DIM; ++c)
+  {
+    load_row<NP>(xc + c * Ns + NP * q, u[c]);
+    load_row<NP>(xc + c * Ns + NP * q + (has[0][0] ? -NDC : 0), nx[0][c]);
+    load_row<NP>(xc + c * Ns + NP * q + (has[0][1] ? NDC : 0), nx[1][c]);
+  }
+#pragma unroll
+  for(int d = 1; d < DIM; ++d)
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool in = has[d][side];
+      const int st = d == 1 ? NP : NP * NP;
+      const int64_t shift = (d == 1 ? int64_t(n) : nn) * NDC;
+      const int at = d == 1 ? q0 + NP * NP * q1 : q0 + NP * q1;
+      // absent neighbour: the cell's own line, reversed
+      const T *src = xc + (in ? (side ? shift : -shift) : 0) + at + (in ? 0 : P * st);
+      const int sst = in ? st : -st;
+#pragma unroll
+      for(int c = 0; c < DIM; ++c)
+#pragma unroll
+        for(int j = 0; j < NP; ++j) fl[d - 1][side][c][j] = src[c * Ns + j * sst];
+    }
+
+  // trace (v, P) of a neighbour line r on this cell's face `side`; sg: -1 for the
+  // reflection; w: the cell's own value there
+  auto trace = [&](const T *r, int side, bool along, T sg, T w, T &v, T &jp) {
+    T d = 0;
+#pragma unroll
+    for(int j = 0; j < NP; ++j) d += tab.g[1 - side][j] * r[j];
+    v = sg * (side ? r[0] : r[P]);
+    const T a = along ? tab.aA : tab.aB, pn = along ? tab.pA : tab.pB;
+    jp = (side ? -a : a) * (sg * d) + pn * (w - v);
   };
-  const int64_t cell = act ? cell_of(cs) : 0;
-  // slot s of the block holds a cell (no load of the cell list)
-  auto has_cell = [&](int s) { return int64_t(blockIdx.x) * CPB + s < count; };
-  const int ix = ts % NP, iy = (ts / NP) % NP, iz = DIM == 3 ? ts / (NP * NP) : 0;
-  const int ti[3] = {ix, iy, iz};
-
+  T vx[2][DIM];  // x-face values of this lane's line
   {
-    const T *src = reinterpret_cast<const T *>(&tab);
-    T *dst = reinterpret_cast<T *>(&tl);
-    constexpr int NTAB = int(sizeof(ElastTab<NP, T>) / sizeof(T));
-    for(int i = t; i < NTAB; i += NT) dst[i] = src[i];
-  }
-  if(t < CPB * 2 * DIM)
-  {
-    const int s = t / (2 * DIM), f = t % (2 * DIM), D = f >> 1, side = f & 1;
-    const int64_t ce = cell_of(s);
-    int64_t nb = -1;
-    if(ce >= 0)
-    {
-      const int64_t cstride = D == 0 ? int64_t(1) : D == 1 ? int64_t(n) : int64_t(n) * n;
-      const int cd = int((ce / cstride) % n);
-      if(side == 1 ? cd < n - 1 : cd > 0) nb = side == 1 ? ce + cstride : ce - cstride;
-    }
-    nbc[s][f] = nb;
-  }
-  if(act)
-#pragma unroll
-    for(int c = 0; c < DIM; ++c) U[c0][c][ts] = x[c * Ns + cell * NDC + ts];
-  __syncthreads();
-
-  // ---------------- cell term
-  T acc[DIM];
-#pragma unroll
-  for(int c = 0; c < DIM; ++c) acc[c] = T(0);
-  {
-    // x-stage: R1[2c] = V_x u_c, R1[2c+1] = G_x u_c
-    if(act)
-    {
-      const int base = ts - ix;
-#pragma unroll
-      for(int c = 0; c < DIM; ++c)
-      {
-        T v = 0, g = 0;
-#pragma unroll
-        for(int j = 0; j < NP; ++j)
-        {
-          const T u = U[c0][c][base + j];
-          v += tl.V[ix * NP + j] * u;
-          g += tl.G[ix * NP + j] * u;
-        }
-        R1[c0][2 * c][ts] = v;
-        R1[c0][2 * c + 1][ts] = g;
-      }
-    }
-    __syncthreads();
-    T g[DIM][DIM];  // g[c][a] = d u_c / d x_a at the quadrature point ts
-    if constexpr(DIM == 3)
-    {
-      // y-stage: R2[3c] = V_y G_x u_c, R2[3c+1] = G_y V_x u_c, R2[3c+2] = V_y V_x u_c
-      if(act)
-      {
-        const int base = ts - iy * NP;
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-        {
-          T s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-          for(int j = 0; j < NP; ++j)
-          {
-            const T av = R1[c0][2 * c][base + j * NP], ag = R1[c0][2 * c + 1][base + j * NP];
-            const T vy = tl.V[iy * NP + j];
-            s0 += vy * ag;
-            s1 += tl.G[iy * NP + j] * av;
-            s2 += vy * av;
-          }
-          R2[c0][3 * c][ts] = s0;
-          R2[c0][3 * c + 1][ts] = s1;
-          R2[c0][3 * c + 2][ts] = s2;
-        }
-      }
-      __syncthreads();
-      // z-stage into registers
-      const int base = ts - iz * NP * NP;
-#pragma unroll
-      for(int c = 0; c < DIM; ++c)
-      {
-        T s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-        for(int j = 0; j < NP; ++j)
-        {
-          const T vz = tl.V[iz * NP + j];
-          s0 += vz * R2[c0][3 * c][base + j * NP * NP];
-          s1 += vz * R2[c0][3 * c + 1][base + j * NP * NP];
-          s2 += tl.G[iz * NP + j] * R2[c0][3 * c + 2][base + j * NP * NP];
-        }
-        g[c][0] = s0;
-        g[c][1] = s1;
-        g[c][2] = s2;
-      }
-    }
-    else
-    {
-      const int base = ts - iy * NP;
-#pragma unroll
-      for(int c = 0; c < DIM; ++c)
-      {
-        T s0 = 0, s1 = 0;
-#pragma unroll
-        for(int j = 0; j < NP; ++j)
-        {
-          s0 += tl.V[iy * NP + j] * R1[c0][2 * c + 1][base + j * NP];
-          s1 += tl.G[iy * NP + j] * R1[c0][2 * c][base + j * NP];
-        }
-        g[c][0] = s0;
-        g[c][1] = s1;
-      }
-    }
-    // stress times JxW: mu (grad u + grad u^T) + lambda div u I, into the array
-    // not read in the last stage (3D: R1, 2D: R2)
-    {
-      T w = T(1), div = T(0);
-#pragma unroll
-      for(int e = 0; e < DIM; ++e) w *= tl.w[ti[e]];
-#pragma unroll
-      for(int c = 0; c < DIM; ++c) div += g[c][c];
-      T(*SG)[NDC] = DIM == 3 ? R1[c0] : R2[c0];
-      if(act)
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-#pragma unroll
-          for(int a = 0; a < DIM; ++a)
-            SG[c * DIM + a][ts] =
-              w * (tl.mu * (g[c][a] + g[a][c]) + (c == a ? tl.lambda * div : T(0)));
-    }
-    __syncthreads();
-    if constexpr(DIM == 3)
-    {
-      // z-integration: R2[3c] = V_z^T s_c0, R2[3c+1] = V_z^T s_c1, R2[3c+2] = G_z^T s_c2
-      if(act)
-      {
-        const int base = ts - iz * NP * NP;
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-        {
-          T s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-          for(int q = 0; q < NP; ++q)
-          {
-            const T vz = tl.V[q * NP + iz];
-            s0 += vz * R1[c0][c * 3][base + q * NP * NP];
-            s1 += vz * R1[c0][c * 3 + 1][base + q * NP * NP];
-            s2 += tl.G[q * NP + iz] * R1[c0][c * 3 + 2][base + q * NP * NP];
-          }
-          R2[c0][3 * c][ts] = s0;
-          R2[c0][3 * c + 1][ts] = s1;
-          R2[c0][3 * c + 2][ts] = s2;
-        }
-      }
-      __syncthreads();
-      // y-integration: R1[2c] = V_y^T (.)0, R1[2c+1] = G_y^T (.)1 + V_y^T (.)2
-      if(act)
-      {
-        const int base = ts - iy * NP;
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-        {
-          T s0 = 0, s1 = 0;
-#pragma unroll
-          for(int q = 0; q < NP; ++q)
-          {
-            const T vy = tl.V[q * NP + iy];
-            s0 += vy * R2[c0][3 * c][base + q * NP];
-            s1 += tl.G[q * NP + iy] * R2[c0][3 * c + 1][base + q * NP] +
-                  vy * R2[c0][3 * c + 2][base + q * NP];
-          }
-          R1[c0][2 * c][ts] = s0;
-          R1[c0][2 * c + 1][ts] = s1;
-        }
-      }
-    }
-    else
-    {
-      // y-integration: R1[2c] = V_y^T s_c0, R1[2c+1] = G_y^T s_c1
-      if(act)
-      {
-        const int base = ts - iy * NP;
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-        {
-          T s0 = 0, s1 = 0;
-#pragma unroll
-          for(int q = 0; q < NP; ++q)
-          {
-            s0 += tl.V[q * NP + iy] * R2[c0][c * 2][base + q * NP];
-            s1 += tl.G[q * NP + iy] * R2[c0][c * 2 + 1][base + q * NP];
-          }
-          R1[c0][2 * c][ts] = s0;
-          R1[c0][2 * c + 1][ts] = s1;
-        }
-      }
-    }
-    __syncthreads();
-    // x-integration
-    if(act)
-    {
-      const int base = ts - ix;
-#pragma unroll
-      for(int c = 0; c < DIM; ++c)
-      {
-        T s = 0;
-#pragma unroll
-        for(int q = 0; q < NP; ++q)
-          s += tl.G[q * NP + ix] * R1[c0][2 * c][base + q] +
-               tl.V[q * NP + ix] * R1[c0][2 * c + 1][base + q];
-        acc[c] = s;
-      }
-    }
-  }
-
-  // ---------------- faces, direction D fixed at compile time (both faces)
-  auto face_dir = [&](auto Dc) {
-    constexpr int D = decltype(Dc)::value;
-    constexpr int E1 = D == 0 ? 1 : 0;
-    constexpr int E2 = DIM == 3 ? (D == 2 ? 1 : 2) : E1;
-    __syncthreads();  // PA / PB of the previous direction have been read
-    // traces along the normal: value (PA) and normal derivative (PB) of both
-    // cell sides for every component and tangential node; the cell's own side
-    // (from LDS) and the neighbour's (from global memory) in separate passes, so
-    // that a wave runs one of the two branches per iteration
-#pragma unroll
-    for(int sd = 0; sd < 2; ++sd)
-      for(int o = t; o < CPB * 2 * DIM * NF; o += NT)
-      {
-        const int s = o / (2 * DIM * NF), side = (o / (DIM * NF)) % 2;
-        const int c = (o / NF) % DIM, m = o % NF;
-        if(!has_cell(s)) continue;
-        const bool inner = nbc[s][2 * D + side] >= 0;
-        if(sd == 1 && !inner) continue;
-        const int i1 = m % NP, i2 = DIM == 3 ? m / NP : 0;
-        const int base = i1 * ST[E1] + (DIM == 3 ? i2 * ST[E2] : 0);
-        const int fs = sd == 0 ? side : 1 - side;
-        T a = 0, bs = 0;
-        if(sd == 0)
-        {
-#pragma unroll
-          for(int id = 0; id < NP; ++id)
-          {
-            const T u = U[s][c][base + id * ST[D]];
-            a += tl.f[fs][id] * u;
-            bs += tl.fd[fs][id] * u;
-          }
-        }
-        else
-        {
-          const VT *src = x + c * Ns + nbc[s][2 * D + side] * NDC + base;
-#pragma unroll
-          for(int id = 0; id < NP; ++id)
-          {
-            const T u = src[id * ST[D]];
-            a += tl.f[fs][id] * u;
-            bs += tl.fd[fs][id] * u;
-          }
-        }
-        PA[s][side][sd][c][m] = a;
-        PB[s][side][sd][c][m] = bs;
-      }
-    __syncthreads();
-    // fluxes at every face point
-    for(int o = t; o < CPB * 2 * NF; o += NT)
-    {
-      const int s = o / (2 * NF), side = (o / NF) % 2, l = o % NF;
-      if(!has_cell(s)) continue;
-      const bool inner = nbc[s][2 * D + side] >= 0;
-      const int l1 = l % NP, l2 = DIM == 3 ? l / NP : 0;
-      // traces and physical gradients of this cell (o) and the exterior state (x)
-      T uo[DIM], go[DIM][DIM], ux[DIM], gx[DIM][DIM];
-#pragma unroll
-      for(int c = 0; c < DIM; ++c)
-      {
-        uo[c] = ux[c] = T(0);
-#pragma unroll
-        for(int a = 0; a < DIM; ++a) go[c][a] = gx[c][a] = T(0);
-      }
-#pragma unroll
-      for(int m = 0; m < NF; ++m)
-      {
-        const int i1 = m % NP, i2 = DIM == 3 ? m / NP : 0;
-        const T t1v = tl.V[l1 * NP + i1], t1d = tl.G[l1 * NP + i1];
-        const T t2v = DIM == 3 ? tl.V[l2 * NP + i2] : T(1);
-        const T t2d = DIM == 3 ? tl.G[l2 * NP + i2] : T(0);
-        const T wvv = t1v * t2v, wdv = t1d * t2v, wvd = t1v * t2d;
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-        {
-          const T a = PA[s][side][0][c][m];
-          uo[c] += wvv * a;
-          go[c][D] += wvv * PB[s][side][0][c][m];
-          go[c][E1] += wdv * a;
-          if(DIM == 3) go[c][E2] += wvd * a;
-          if(inner)
-          {
-            const T a1 = PA[s][side][1][c][m];
-            ux[c] += wvv * a1;
-            gx[c][D] += wvv * PB[s][side][1][c][m];
-            gx[c][E1] += wdv * a1;
-            if(DIM == 3) gx[c][E2] += wvd * a1;
-          }
-        }
-      }
-      if(!inner)
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-        {
-          ux[c] = -uo[c];
-#pragma unroll
-          for(int a = 0; a < DIM; ++a) gx[c][a] = go[c][a];
-        }
-      const T nrm = side == 1 ? T(1) : T(-1);
-      const T dS = tl.w[l1] * (DIM == 3 ? tl.w[l2] : T(1));
-      T J[DIM], divo = 0, divx = 0;
-#pragma unroll
-      for(int c = 0; c < DIM; ++c)
-      {
-        J[c] = uo[c] - ux[c];
-        divo += go[c][c];
-        divx += gx[c][c];
-      }
-      const T hm = T(-0.5) * tl.mu * nrm, hl = T(-0.5) * tl.lambda * nrm;
-#pragma unroll
-      for(int c = 0; c < DIM; ++c)
-      {
-        // {2 mu eps(u) n + lambda div(u) n}_c
-        const T fo = tl.mu * (go[c][D] + go[D][c]) + (c == D ? tl.lambda * divo : T(0));
-        const T fx = tl.mu * (gx[c][D] + gx[D][c]) + (c == D ? tl.lambda * divx : T(0));
-        const T F = T(0.5) * (fo + fx) * nrm;
-        FA[s][side][c][l] = dS * (-F + T(2) * tl.mu * tl.sigma * J[c] +
-                                  (c == D ? tl.lambda * tl.sigma * J[D] : T(0)));
-        // -1/2 (2 mu eps(v) n . [u] + lambda div v [u].n)
-        T fb[DIM];
-#pragma unroll
-        for(int a = 0; a < DIM; ++a) fb[a] = T(0);
-        fb[D] += hm * J[c];
-        if(c == D)
-#pragma unroll
-          for(int a = 0; a < DIM; ++a) fb[a] += hm * J[a];
-        fb[c] += hl * J[D];
-#pragma unroll
-        for(int a = 0; a < DIM; ++a) FB[s][side][c][a][l] = dS * fb[a];
-      }
-    }
-    __syncthreads();
-    // projections on the tangential test functions (into PA / PB [.][0])
-    if constexpr(DIM == 3)
-    {
-      // sum-factorised: along e1 into the cell-stage arrays (free during the faces),
-      // SA = sum_l1 phi_i1 FA + phi'_i1 FB_E1, SB = sum_l1 phi_i1 FB_E2,
-      // SC = sum_l1 phi_i1 FB_D at (i1, l2); then along e2
-      constexpr int NQ = CPB * 2 * DIM * NF;
-      static_assert(3 * NQ <= CPB * NS * NDC, "projection stage fits the stage arrays");
-      T *SA = &R2[0][0][0], *SB = SA + NQ, *SC = SA + 2 * NQ;
-      for(int o = t; o < NQ; o += NT)
-      {
-        const int s = o / (2 * DIM * NF), side = (o / (DIM * NF)) % 2;
-        const int c = (o / NF) % DIM, m = o % NF;
-        if(!has_cell(s)) continue;
-        const int i1 = m % NP, l2 = m / NP;
-        T sa = 0, sb = 0, sc = 0;
-#pragma unroll
-        for(int l1 = 0; l1 < NP; ++l1)
-        {
-          const int l = l1 + NP * l2;
-          const T v = tl.V[l1 * NP + i1], g = tl.G[l1 * NP + i1];
-          sa += v * FA[s][side][c][l] + g * FB[s][side][c][E1][l];
-          sb += v * FB[s][side][c][E2][l];
-          sc += v * FB[s][side][c][D][l];
-        }
-        SA[o] = sa;
-        SB[o] = sb;
-        SC[o] = sc;
-      }
-      __syncthreads();
-      for(int o = t; o < NQ; o += NT)
-      {
-        const int s = o / (2 * DIM * NF), side = (o / (DIM * NF)) % 2;
-        const int c = (o / NF) % DIM, m = o % NF;
-        if(!has_cell(s)) continue;
-        const int i1 = m % NP, i2 = m / NP, base = o - m;
-        T pv = 0, pd = 0;
-#pragma unroll
-        for(int l2 = 0; l2 < NP; ++l2)
-        {
-          const int r = base + i1 + NP * l2;
-          const T v = tl.V[l2 * NP + i2], g = tl.G[l2 * NP + i2];
-          pv += v * SA[r] + g * SB[r];
-          pd += v * SC[r];
-        }
-        PA[s][side][0][c][m] = pv;
-        PB[s][side][0][c][m] = pd;
-      }
-    }
-    else
-    {
-      // 2D: one tangential direction (NF = NP)
-      for(int o = t; o < CPB * 2 * DIM * NF; o += NT)
-      {
-        const int s = o / (2 * DIM * NF), side = (o / (DIM * NF)) % 2;
-        const int c = (o / NF) % DIM, i1 = o % NF;
-        if(!has_cell(s)) continue;
-        T pv = 0, pd = 0;
-#pragma unroll
-        for(int l = 0; l < NF; ++l)
-        {
-          const T v = tl.V[l * NP + i1];
-          pv += v * FA[s][side][c][l] + tl.G[l * NP + i1] * FB[s][side][c][E1][l];
-          pd += v * FB[s][side][c][D][l];
-        }
-        PA[s][side][0][c][i1] = pv;
-        PB[s][side][0][c][i1] = pd;
-      }
-    }
-    __syncthreads();
-    if(act)
-    {
-      // test functions of this cell: phi_i = f(i_D) * tangential factors
-      const int id = ti[D];
-      const int m = ti[E1] + (DIM == 3 ? NP * ti[E2] : 0);
-#pragma unroll
-      for(int side = 0; side < 2; ++side)
-      {
-        const T fv = tl.f[side][id], fdv = tl.fd[side][id];
-#pragma unroll
-        for(int c = 0; c < DIM; ++c)
-          acc[c] += fv * PA[c0][side][0][c][m] + fdv * PB[c0][side][0][c][m];
-      }
-    }
-  };
-  face_dir(std::integral_constant<int, 0>{});
-  face_dir(std::integral_constant<int, 1>{});
-  if constexpr(DIM == 3) face_dir(std::integral_constant<int, DIM == 3 ? 2 : 1>{});
-
-  if(act)
+    T e[DIM][NX];
 #pragma unroll
     for(int c = 0; c < DIM; ++c)
     {
-      const int64_t i = c * Ns + cell * NDC + ts;
-      if(RESIDUAL)
-        y[i] = b[i] - acc[c];
-      else
-        y[i] = acc[c];
+#pragma unroll
+      for(int i = 0; i < NP; ++i) e[c][i] = u[c][i];
+#pragma unroll
+      for(int side = 0; side < 2; ++side)
+      {
+        T r[NP];
+#pragma unroll
+        for(int j = 0; j < NP; ++j) r[j] = has[0][side] ? nx[side][c][j] : -u[c][P - j];
+        trace(r, side, c == 0, T(1), u[c][side ? P : 0], vx[side][c], e[c][NP + 2 * side + 1]);
+        e[c][NP + 2 * side] = vx[side][c];
+      }
+      Ext::put(ext + c * Ext::SIZE, t, e[c]);
     }
+  }
+  __syncthreads();  // the lines are staged
+#pragma unroll
+  for(int side = 0; side < 2; ++side)
+#pragma unroll
+    for(int c = 0; c < DIM; ++c)
+    {
+      T v, jp;
+      const int r = cs * FL + q1, e = side ? P : 0;
+      trace(fl[0][side][c], side, c == 1, has[1][side] ? T(1) : T(-1),
+            ext[eidx(c, cr * NL + e + NP * q1, q0)], v, jp);
+      fy[fidx(pv(side, c), r, q0)] = v;
+      fy[fidx(pp(side, c), r, q0)] = jp;
+      if constexpr(D3)
+      {
+        trace(fl[DIM - 2][side][c], side, c == 2, has[2][side] ? T(1) : T(-1),
+              ext[eidx(c, cr * NL + q1 + NP * e, q0)], v, jp);
+        fz[fidx(pv(side, c), r, q0)] = v;
+        fz[fidx(pp(side, c), r, q0)] = jp;
+      }
+    }
+  __syncthreads();
+
+  // lane-indexed rows of the 1D tables
+  const T *tM = tl, *tK = tl + NP * NP, *tLA = tl + 2 * NP * NP, *tLB = tl + 3 * NP * NP;
+  const T *tg = tl + 4 * NP * NP;
+  const T b0 = q0 == 0 ? T(-1) : q0 == P ? T(1) : T(0);
+  const T b1 = q1 == 0 ? T(-1) : q1 == P ? T(1) : T(0);
+  const T kappa = tab.kappa, kq = T(0.25) * tab.kappa;
+  T M1[NP], K1[NP];  // rows of index q1
+  // ---- z-face traces contracted along y by the lanes (lx, ly) = (q0, q1):
+  // M v, M P with the tangential mixed terms along y added to P
+  T zt[2][2 * DIM];
+  if constexpr(D3)
+  {
+#pragma unroll
+    for(int j = 0; j < NP; ++j)
+    {
+      M1[j] = tM[q1 * NP + j];
+      K1[j] = tK[q1 * NP + j];
+    }
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      T kv[3];
+#pragma unroll
+      for(int k = 0; k < 2 * DIM; ++k)
+      {
+        T m = 0, kk = 0;
+#pragma unroll
+        for(int j = 0; j < NP; ++j)
+        {
+          const T w = fz[fidx(side * 2 * DIM + k, cs * NP + j, q0)];
+          m += M1[j] * w;
+          if(k == 1 || k == 2) kk += K1[j] * w;
+        }
+        zt[side][k] = m;
+        if(k == 1 || k == 2)
+        {
+          const T w = fz[fidx(pv(side, k), cs * NP + q1, q0)];
+          const int bf = has[2][side] ? 0 : 1;
+          const T hK = k == 1 ? tab.h1K[bf] : tab.h2K[bf], hB = k == 1 ? tab.h1B[bf] : tab.h2B[bf];
+          kv[k] = (side ? T(-1) : T(1)) * (hK * kk + hB * b1 * w);
+        }
+      }
+      zt[side][DIM + 1] += kv[2];  // component 1: H2 along y of u_2
+      zt[side][DIM + DIM - 1] += kv[1];  // component 2: H1 along y of u_1
+    }
+  }
+
+  // ---- y stage: M, L and K along y of the extended lines, with the y faces
+  T My[DIM][NX], Ly[DIM][NP], Ky[DIM][NP], KyV[DIM][2], Q[DIM][NP];
+  {
+    T M0[NP], K0[NP], LA0[NP], LB0[NP];
+#pragma unroll
+    for(int j = 0; j < NP; ++j)
+    {
+      M0[j] = tM[q0 * NP + j];
+      K0[j] = tK[q0 * NP + j];
+      LA0[j] = tLA[q0 * NP + j];
+      LB0[j] = tLB[q0 * NP + j];
+    }
+    T gs[2], es[2];
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      gs[side] = (side ? T(1) : T(-1)) * tg[side * NP + q0];
+      es[side] = q0 == (side ? P : 0) ? T(1) : T(0);
+    }
+#pragma unroll
+    for(int c = 0; c < DIM; ++c)
+    {
+#pragma unroll
+      for(int i = 0; i < NX; ++i) My[c][i] = 0;
+#pragma unroll
+      for(int i = 0; i < NP; ++i) Ly[c][i] = Ky[c][i] = 0;
+      KyV[c][0] = KyV[c][1] = 0;
+#pragma unroll
+      for(int j = 0; j < NP; ++j)
+      {
+        T r[NX];
+        Ext::get(ext + c * Ext::SIZE, cr * NL + j + NP * q1, r);
+        const T l = c == 1 ? LA0[j] : LB0[j];
+#pragma unroll
+        for(int i = 0; i < NX; ++i) My[c][i] += M0[j] * r[i];
+#pragma unroll
+        for(int i = 0; i < NP; ++i)
+        {
+          Ly[c][i] += l * r[i];
+          Ky[c][i] += K0[j] * r[i];
+        }
+        KyV[c][0] += K0[j] * r[NP];
+        KyV[c][1] += K0[j] * r[NP + 2];
+      }
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+      {
+        Ky[c][i] *= kappa;
+        Q[c][i] = kq * b0 * u[c][i];
+      }
+      const T a = c == 1 ? tab.aA : tab.aB;
+#pragma unroll
+      for(int side = 0; side < 2; ++side)
+      {
+        T v[NP], jp[NP];
+        Face::get(fy + pv(side, c) * Face::SIZE, cs * FL + q1, v);
+        Face::get(fy + pp(side, c) * Face::SIZE, cs * FL + q1, jp);
+        const int bf = has[1][side] ? 0 : 1;
+        const T sg = side ? -es[side] : es[side];
+        const T hK = sg * (c == 1 ? tab.h2K[bf] : tab.h1K[bf]);
+        const T hB = sg * (c == 1 ? tab.h2B[bf] : tab.h1B[bf]);
+        const T cv = a * gs[side];
+#pragma unroll
+        for(int i = 0; i < NP; ++i)
+        {
+          Ly[c][i] += cv * v[i] + es[side] * jp[i];
+          Ky[c][i] += hK * v[i];
+          Q[c][i] += hB * v[i];
+        }
+      }
+    }
+  }
+  __syncthreads();  // the lines, the y-face rows and the z-face traces are read
+
+  if constexpr(D3)
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+#pragma unroll
+      for(int k = 0; k < 2 * DIM; ++k) fz[fidx(side * 2 * DIM + k, cs * NP + q1, q0)] = zt[side][k];
+
+  // ---- x products in registers
+  auto xprod = [&](const T *A, const T *r, T *o, T f) {
+#pragma unroll
+    for(int i = 0; i < NP; ++i)
+    {
+      T s = 0;
+#pragma unroll
+      for(int j = 0; j < NP; ++j) s += A[i * NP + j] * r[j];
+      o[i] += f * s;
+    }
+  };
+  auto clear = [&](T *o) {
+#pragma unroll
+    for(int i = 0; i < NP; ++i) o[i] = 0;
+  };
+  T I[DIM][NP];
+  T *zb = buf;
+#pragma unroll
+  for(int c = 0; c < DIM; ++c)
+  {
+    T zm[NP], zl[NP], zk[NP];
+    // L along x with the x faces; M along x of the y-line products
+    const T a = c == 0 ? tab.aA : tab.aB;
+#pragma unroll
+    for(int i = 0; i < NP; ++i)
+      zm[i] = -a * tab.g[0][i] * My[c][NP] + a * tab.g[1][i] * My[c][NP + 2];
+    zm[0] += My[c][NP + 1];
+    zm[P] += My[c][NP + 3];
+    xprod(c == 0 ? tab.LA : tab.LB, My[c], zm, T(1));
+    xprod(tab.M, Ly[c], zm, T(1));
+    // the mixed terms
+    if(c < 2)
+    {
+      const int o = 1 - c;
+      xprod(tab.K, Ky[o], zm, T(1));
+      zm[0] -= Q[o][0];
+      zm[P] += Q[o][P];
+    }
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const int bf = has[0][side] ? 0 : 1;
+      const T s = side ? T(-1) : T(1);
+      if(c < 2)
+        zm[side ? P : 0] += s * ((c == 0 ? tab.h1K[bf] : tab.h2K[bf]) * KyV[1 - c][side] +
+                                 (c == 0 ? tab.h1B[bf] : tab.h2B[bf]) * b0 * vx[side][1 - c]);
+    }
+    if constexpr(D3)
+    {
+      clear(zl);
+      xprod(tab.M, My[c], zl, T(1));
+      clear(zk);
+      clear(I[c]);
+      if(c == 1) xprod(tab.M, Ky[DIM - 1], zk, T(1));
+      if(c == 2) xprod(tab.M, Ky[1], zk, T(1));
+      if(c != 1)
+      {
+        const int o = 2 - c;
+        xprod(tab.K, My[o], zk, kappa);
+#pragma unroll
+        for(int side = 0; side < 2; ++side)
+        {
+          const int i = side ? P : 0, bf = has[0][side] ? 0 : 1;
+          const T s = side ? T(-1) : T(1);
+          zk[i] += s * (c == 0 ? tab.h1K[bf] : tab.h2K[bf]) * My[o][NP + 2 * side];
+          I[c][i] += b1 * s *
+                     ((c == 0 ? tab.h1B[bf] : tab.h2B[bf]) * My[o][NP + 2 * side] - kq * My[o][i]);
+        }
+      }
+      if(c > 0) xprod(tab.M, Q[3 - c], I[c], b1);
+      Row::put(zb + (3 * c + 0) * Row::SIZE, t, zm);
+      Row::put(zb + (3 * c + 1) * Row::SIZE, t, zl);
+      Row::put(zb + (3 * c + 2) * Row::SIZE, t, zk);
+    }
+    else
+#pragma unroll
+      for(int i = 0; i < NP; ++i) I[c][i] = zm[i];
+  }
+  // ---- z stage and the z faces
+  if constexpr(D3)
+  {
+    __syncthreads();
+    T LA1[NP], LB1[NP];
+#pragma unroll
+    for(int j = 0; j < NP; ++j)
+    {
+      LA1[j] = tLA[q1 * NP + j];
+      LB1[j] = tLB[q1 * NP + j];
+    }
+#pragma unroll
+    for(int c = 0; c < DIM; ++c)
+#pragma unroll
+      for(int k = 0; k < NP; ++k)
+      {
+        T zm[NP], zl[NP], zk[NP];
+        const int ln = cr * NL + q0 + NP * k;
+        Row::get(zb + (3 * c + 0) * Row::SIZE, ln, zm);
+        Row::get(zb + (3 * c + 1) * Row::SIZE, ln, zl);
+        Row::get(zb + (3 * c + 2) * Row::SIZE, ln, zk);
+        const T l = c == 2 ? LA1[k] : LB1[k];
+#pragma unroll
+        for(int i = 0; i < NP; ++i) I[c][i] += M1[k] * zm[i] + l * zl[i] + K1[k] * zk[i];
+      }
+    T tz[DIM][NP], w0[NP], w2[NP];
+#pragma unroll
+    for(int c = 0; c < DIM; ++c) clear(tz[c]);
+    clear(w0);
+    clear(w2);
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const T gz = (side ? T(1) : T(-1)) * tg[side * NP + q1];
+      const T ez = q1 == (side ? P : 0) ? T(1) : T(0);
+      const int bf = has[2][side] ? 0 : 1;
+      const T sg = side ? -ez : ez;
+#pragma unroll
+      for(int c = 0; c < DIM; ++c)
+      {
+        T v[NP], jp[NP];
+        Face::get(fz + pv(side, c) * Face::SIZE, cs * NP + q0, v);
+        Face::get(fz + pp(side, c) * Face::SIZE, cs * NP + q0, jp);
+        const T cv = (c == 2 ? tab.aA : tab.aB) * gz;
+#pragma unroll
+        for(int i = 0; i < NP; ++i) tz[c][i] += cv * v[i] + ez * jp[i];
+        if(c != 1)
+        {
+          // H2 along x of u_2 into component 0, H1 along x of u_0 into component 2
+          const T hK = sg * (c == 2 ? tab.h2K[bf] : tab.h1K[bf]);
+          const T hB = sg * (c == 2 ? tab.h2B[bf] : tab.h1B[bf]);
+          T *w = c == 2 ? w0 : w2, *o = c == 2 ? I[0] : I[DIM - 1];
+#pragma unroll
+          for(int i = 0; i < NP; ++i) w[i] += hK * v[i];
+          o[0] -= hB * v[0];
+          o[P] += hB * v[P];
+        }
+      }
+    }
+    xprod(tab.K, w0, I[0], T(1));
+    xprod(tab.K, w2, I[DIM - 1], T(1));
+#pragma unroll
+    for(int c = 0; c < DIM; ++c) xprod(tab.M, tz[c], I[c], T(1));
+  }
+  if(!act) return;
+#pragma unroll
+  for(int c = 0; c < DIM; ++c)
+  {
+    const int64_t at = c * Ns + cell * NDC + NP * q;
+    if(RESIDUAL)
+    {
+      T bv[NP];
+      load_row<NP>(b + at, bv);
+#pragma unroll
+      for(int i = 0; i < NP; ++i) I[c][i] = bv[i] - I[c][i];
+    }
+    store_row<NP>(y + at, I[c]);
+  }
 }
 
 }  // namespace tpss
