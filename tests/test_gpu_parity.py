@@ -286,6 +286,27 @@ def test_distorted_operator_parity_f32(dim, p, n):
     assert rel_err(host(y), b - ref.operator(x)) < 1e-5
 
 
+# cells per block: 64 / (p+1)^(dim-1); last blocks with one cell, full ones, fewer cells
+# than a block, cells with boundary faces on both sides of a direction
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 2), (2, 1, 9), (2, 2, 5), (2, 3, 8), (2, 4, 7), (3, 1, 2),
+                                     (3, 1, 5), (3, 2, 2), (3, 2, 6), (3, 3, 2), (3, 3, 5), (3, 4, 2)])
+def test_distorted_operator_block_edges(dim, p, n):
+    t = _tpss()
+    V = o.distorted_vertices(dim, n, 0.2, seed=5)
+    ref = o.Smoother(dim, p, n, ip=2.0, vertices=V)
+    x, b = o.splitmix_uniform(3, ref.N), o.splitmix_uniform(4, ref.N)
+    for prec, dt, bar in ((t.F64, np.float64, 1e-12), (t.F32, np.float32, 1e-5)):
+        lv = t.Level(dim, p, n, ip_factor=2.0, vertices=V, precision=prec)
+        xs, bs = x.astype(dt), b.astype(dt)
+        Ax = ref.operator(xs.astype(np.float64))
+        y = dev(np.full(ref.N + 8, 7.0, dt), prec)  # guard values behind the output
+        lv.vmult(y, dev(xs, prec))
+        assert rel_err(host(y)[:ref.N], Ax) < bar
+        assert (host(y)[ref.N:] == 7.0).all()
+        lv.residual(y, dev(bs, prec), dev(xs, prec))
+        assert rel_err(host(y)[:ref.N], bs - Ax) < bar
+
+
 @pytest.mark.parametrize("dim,p,n,variant", [(2, 3, 6, 0), (3, 3, 4, 0), (3, 2, 5, 1), (3, 4, 3, 0)])
 def test_distorted_smoother_parity(dim, p, n, variant):
     V = o.distorted_vertices(dim, n, 0.15, seed=3)

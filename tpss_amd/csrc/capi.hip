@@ -142,22 +142,29 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
         }
       }
       for(int f = 0; f < 2; ++f)
-        for(int i = 0; i < NP; ++i)
+        for(int i = 0; i < NP; ++i) tab.fd[f][i] = VT(bs.fgrad[i * 2 + f]);
+      for(int q = 0; q < NP; ++q)
+        for(int r = 0; r < NP; ++r)
         {
-          tab.f[f][i] = VT(bs.fval[i * 2 + f]);
-          tab.fd[f][i] = VT(bs.fgrad[i * 2 + f]);
+          const int i = (q + r) % NP, at = q * NP + r;
+          tab.R[0][at] = tab.V[q * NP + i];
+          tab.R[1][at] = tab.Dv[q * NP + i];
+          tab.R[2][at] = tab.V[i * NP + q];
+          tab.R[3][at] = tab.Dv[i * NP + q];
         }
       const int64_t count = cells ? n_list : lv->ncell;
       if(count == 0) return;
-      const unsigned threads = NDC <= 64 ? 64u : 128u;
-      if(b)
-        hipLaunchKernelGGL((k_sipg_general<DIM, NP, VT, true>), dim3(unsigned(count)),
-                           dim3(threads), 0, s, x, y, b, lv->d_vertices.ptr, tab, lv->n, lv->ip,
-                           NP - 1, cells);
+      // eight equal shares of blocks, one per XCD
+      const unsigned grid = (blocks_for(count, moved_cells_per_block<DIM, NP>()) + 7) / 8 * 8;
+      const VT ipg = VT(lv->ip * double(NP - 1) * NP);
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, s, x, y, b, lv->d_vertices.ptr, tab,
+                           lv->n, ipg, cells, count);
+      };
+      if constexpr(DIM == 3)
+        b ? launch(k_sipg_moved<NP, VT, true>) : launch(k_sipg_moved<NP, VT, false>);
       else
-        hipLaunchKernelGGL((k_sipg_general<DIM, NP, VT, false>), dim3(unsigned(count)),
-                           dim3(threads), 0, s, x, y, b, lv->d_vertices.ptr, tab, lv->n, lv->ip,
-                           NP - 1, cells);
+        b ? launch(k_sipg_moved_2d<NP, VT, true>) : launch(k_sipg_moved_2d<NP, VT, false>);
       TPSS_HIP(hipGetLastError());
     });
     return;

@@ -1,44 +1,37 @@
 // kernels_general.hpp -- SIPG Poisson operator on meshes with moved vertices
 // ((bi/tri)linear cells), matrix-free with QGauss(p+1) on cells and faces:
 // Laplace::DG::MF::Operator::{apply_cell, apply_face, apply_boundary}
-// (apps/laplace_integrator.h:613-743).  The geometry (Jacobians at quadrature
-// points) is recomputed on the fly from the multilinear coefficients of each
-// cell's map, so the only HBM traffic is the vectors and the (n+1)^dim vertex
-// array.
+// (apps/laplace_integrator.h:613-743).  The geometry is recomputed on the fly from
+// the multilinear coefficients of each cell's map, so the only HBM traffic is the
+// vectors and the (n+1)^dim vertex array.  Arithmetic in the vector type (the map
+// coefficients are formed in FP64 from the vertices).  Faces are evaluated
+// element-centrically: every cell integrates its own test functions against the
+// flux of each of its 2*dim faces (interior faces are evaluated from both sides,
+// which keeps the kernels free of write races).
 //
-// One block per cell, one thread per cell DoF / quadrature point (nq = np);
-// arithmetic in the vector type (FP32 levels compute in FP32, FP64 levels in
-// FP64; the map coefficients are formed in FP64 from the vertices).  Faces are
-// evaluated element-centrically: every cell integrates its own test functions
-// against the flux of each of its 2*dim faces (interior faces are evaluated
-// from both sides, which keeps the kernel free of write races).
+// One lane per line.  A cell is NP^(DIM-1) lanes of one wave; in 3D lane (q0, q1)
+// holds the x-line (y, z) = (q0, q1) of the cell and, for the faces of direction d,
+// the line along d at the tangential node (e1, e2) = (q0, q1) of the cell and of its
+// neighbours (in 2D the one lane index q0).  Products along the lane's own line run
+// in registers; products along a lane index take the other lines' values from the
+// lanes that hold them, rotated (lane (q + r) mod NP with coefficient row q of the
+// matrix started at column q), for NP = 4 by DPP (in 3D a cell is a DPP row, its
+// quads the first lane index) and by ds_bpermute otherwise; only the contributions
+// of the y- and z-faces pass through LDS once.
 //
-// Every contraction is sum-factorised, and independent work shares barriers:
-//   P0 load u, the face neighbours, the corners of the cell and the far corners
-//      of the face neighbours
-//   P1 x-interpolation of u (value, derivative); map coefficients of the cell;
-//      per face the tangent and normal-direction derivatives of both maps as
-//      polynomials in the face coordinates
-//   P2 y-interpolation; face traces along the normals (value, normal derivative)
-//   P3 z-interpolation -> reference gradient -> geometry -> reference flux;
-//      face traces along the first tangential direction
-//   P4 z-integration; face traces along the second tangential direction,
-//      face geometry and fluxes per face point
-//   P5 y-integration; face fluxes projected on the tangential test functions
-//      (3D: sum-factorised, first along e1, then -- after a barrier -- along e2)
-//   P6 x-integration; add the face contributions of this test function
+// Geometry from the map coefficients A_S.  The two cells of a face share its
+// tangents t1, t2; with w = t1 x t2, a normal-direction Jacobian column J_d of
+// either cell, g_ij = t_i . t_j and r_i = t_i . J_d,
+//   dS J^{-1} n = +-(w.w, g12 r2 - g22 r1, g12 r1 - g11 r2) / |J_d . w|
+// in the face frame (d, e1, e2) (2D: w = t1 turned, +-(w.w, -r1) / |J_d . w|), and
+// dS = |w|: one reciprocal per cell side and one square root.  At a cell point the
+// reference flux is C^T C grad / |det J| with the adjugate C of J.
 //
-// Face geometry without 3x3 inverses.  The two cells of a face share the face's
-// vertices, so on the face their maps have the same tangent vectors t1, t2 (the
-// Jacobian columns of the tangential directions) and differ only in the column
-// J_d of the normal direction.  With w = t1 x t2 (2D: t1 turned by 90 degrees),
-// the outward unit normal is n = +-w/|w| (the sign makes n . J_d point away from
-// the cell), the surface element is |det J| |J^{-T} e_d| = |w|, and the
-// reference-gradient coefficients c = J^{-1} n of the normal derivative follow
-// from J c = n: c_d = 1/(J_d . n) (n is orthogonal to t1, t2), and the tangential
-// part solves the 2x2 Gram system G c_t = -c_d (t1 . J_d, t2 . J_d), G = (ti . tj);
-// the neighbour's coefficients use its own J_d with the same t1, t2, n and G.
-// The penalty length h = 1/|c_d| = |J_d . n| needs no division.
+// Bound by VALU issue (3D Q3 FP32: 2471 VALU instructions per wave of four cells).
+// 64^3 Q3 apply: FP32 221 us, FP64 412 us (590 / 1240 us with one thread per node
+// and every product through LDS); 40^3 Q4 283 / 576 us (296 / 640), 60^3 Q2
+// 132 / 244 us (326 / 618), 80^3 Q1 155 / 237 us (578 / 1039).  2D: 300^2 Q3 FP64
+// 17 us (123), 700^2 Q1 FP32 21 us (292).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -55,43 +48,11 @@ struct GeneralTab
   T V[NP * NP];   // V[q*NP + i]  = phi_i(x_q), Gauss points x_q
   T Dv[NP * NP];  // Dv[q*NP + i] = phi_i'(x_q)
   T qx[NP], qw[NP];
-  T f[2][NP];     // phi_i(0), phi_i(1)
   T fd[2][NP];    // phi_i'(0), phi_i'(1)
+  // rows of V, Dv and of their transposes rotated to start at the diagonal:
+  // R[m][q*NP + r] = entry (q, (q + r) mod NP)
+  T R[4][NP * NP];
 };
-
-// Jacobian J[a][b] = d x_a / d xi_b of the multilinear map
-//   x(xi) = sum_S A[S] prod_{e in S} xi_e   (S: subsets of the directions, bit masks)
-template<int DIM, typename T>
-__device__ __forceinline__ void coef_jacobian(const T (*A)[3], const T *xi, T (*J)[3])
-{
-#pragma unroll
-  for(int a = 0; a < DIM; ++a)
-#pragma unroll
-    for(int b = 0; b < DIM; ++b) J[a][b] = T(0);
-#pragma unroll
-  for(int S = 1; S < (1 << DIM); ++S)
-#pragma unroll
-    for(int b = 0; b < DIM; ++b)
-    {
-      if(!((S >> b) & 1)) continue;
-      T w = T(1);
-#pragma unroll
-      for(int e = 0; e < DIM; ++e)
-        if(e != b && ((S >> e) & 1)) w *= xi[e];
-#pragma unroll
-      for(int a = 0; a < DIM; ++a) J[a][b] += w * A[S][a];
-    }
-}
-
-// 1/a: the hardware reciprocal in FP32 (1 ulp), an exact division in FP64
-template<typename T>
-__device__ __forceinline__ T recip(T a)
-{
-  if constexpr(std::is_same<T, float>::value)
-    return __builtin_amdgcn_rcpf(a);
-  else
-    return T(1) / a;
-}
 
 template<typename T>
 __device__ __forceinline__ T root(T a)
@@ -102,664 +63,671 @@ __device__ __forceinline__ T root(T a)
     return sqrt(a);
 }
 
-// Ji = J^{-1}, returns det J
-template<int DIM, typename T>
-__device__ __forceinline__ T invert(const T (*J)[3], T (*Ji)[3])
+template<int DIM, int NP>
+constexpr int moved_cells_per_block()
 {
-  if constexpr(DIM == 2)
-  {
-    const T det = J[0][0] * J[1][1] - J[0][1] * J[1][0];
-    const T id = recip(det);
-    Ji[0][0] = J[1][1] * id;
-    Ji[0][1] = -J[0][1] * id;
-    Ji[1][0] = -J[1][0] * id;
-    Ji[1][1] = J[0][0] * id;
-    return det;
-  }
-  else
-  {
-    const T c00 = J[1][1] * J[2][2] - J[1][2] * J[2][1];
-    const T c01 = J[1][2] * J[2][0] - J[1][0] * J[2][2];
-    const T c02 = J[1][0] * J[2][1] - J[1][1] * J[2][0];
-    const T det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
-    const T id = recip(det);
-    Ji[0][0] = c00 * id;
-    Ji[0][1] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-    Ji[0][2] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-    Ji[1][0] = c01 * id;
-    Ji[1][1] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-    Ji[1][2] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-    Ji[2][0] = c02 * id;
-    Ji[2][1] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-    Ji[2][2] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
-    return det;
-  }
+  return 64 / cpow(NP, DIM - 1);
 }
 
-template<int DIM, int NP, typename VT, bool RESIDUAL>
-__global__ void __launch_bounds__((cpow(NP, DIM) <= 64 ? 64 : 128), (std::is_same<VT, float>::value ? 5 : 1))
-k_sipg_general(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
-               const double *__restrict__ vert, const GeneralTab<NP, VT> tab, const int n,
-               const double ip, const int p, const uint32_t *__restrict__ cells)
+// value of lane (q + r) mod NP along the first (AX = 0) or second (AX = 1) lane
+// index of the cell; addr: byte address of that lane for ds_bpermute (NP != 4)
+template<int NP, int AX, int R, typename T>
+__device__ __forceinline__ T lane_rot(T v, const int *addr)
+{
+  if constexpr(R == 0)
+    return v;
+  else if constexpr(NP == 4)
+  {
+    // quad_perm (i + R) mod 4; row_ror by 16 - 4 R
+    constexpr int CTRL = AX == 0 ? ((R & 3) | (((1 + R) & 3) << 2) | (((2 + R) & 3) << 4) | (((3 + R) & 3) << 6))
+                                 : 0x120 + 16 - 4 * R;
+    if constexpr(sizeof(T) == 4)
+      return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+    else
+      return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true),
+                              __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true));
+  }
+  else if constexpr(sizeof(T) == 4)
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr[R], __float_as_int(v)));
+  else
+    return __hiloint2double(__builtin_amdgcn_ds_bpermute(addr[R], __double2hiint(v)),
+                            __builtin_amdgcn_ds_bpermute(addr[R], __double2loint(v)));
+}
+
+template<int NP, int AX, typename T>
+__device__ __forceinline__ void lane_gather(T v, const int *addr, T *o)
+{
+  o[0] = v;
+  o[1] = lane_rot<NP, AX, 1>(v, addr);
+  if constexpr(NP > 2) o[2] = lane_rot<NP, AX, 2>(v, addr);
+  if constexpr(NP > 3) o[3] = lane_rot<NP, AX, 3>(v, addr);
+  if constexpr(NP > 4) o[4] = lane_rot<NP, AX, 4>(v, addr);
+}
+
+template<int NP, typename T>
+__device__ __forceinline__ T dotn(const T *a, const T *b)
+{
+  T s = 0;
+#pragma unroll
+  for(int r = 0; r < NP; ++r) s += a[r] * b[r];
+  return s;
+}
+
+// 1/a: the hardware reciprocal, in FP64 refined by two Newton steps (within an ulp
+// or two of the correctly rounded quotient)
+__device__ __forceinline__ float fast_recip(float a) { return __builtin_amdgcn_rcpf(a); }
+__device__ __forceinline__ double fast_recip(double a)
+{
+  double r = __builtin_amdgcn_rcp(a);
+  r = fma(r, fma(-a, r, 1.0), r);
+  return fma(r, fma(-a, r, 1.0), r);
+}
+
+template<int NP, typename VT, bool RESIDUAL>
+__global__ void __launch_bounds__(64, (std::is_same<VT, float>::value ? 3 : 2))
+k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
+             const double *__restrict__ vert, const GeneralTab<NP, VT> tab, const int n,
+             const VT ipg, const uint32_t *__restrict__ cells, const int64_t count)
 {
   using T = VT;
-  constexpr int NDC = cpow(NP, DIM);
-  constexpr int NF = cpow(NP, DIM - 1);
-  constexpr int NFACE = 2 * DIM;
-  constexpr int NCORN = 1 << DIM;
-  constexpr int NT = NDC <= 64 ? 64 : 128;  // block size
-  // lexicographic stride of direction e (by selection: a constant array indexed at
-  // run time would be read from memory)
-  auto stride = [](int e) { return e == 0 ? 1 : (e == 1 ? NP : NP * NP); };
-  constexpr int NP2 = DIM == 3 ? NP : 1;    // tangential nodes along the second face direction
+  constexpr int NL = NP * NP, NDC = NL * NP, CPB = moved_cells_per_block<3, NP>(), P = NP - 1;
+  constexpr int CSL = (64 + NL - 1) / NL;  // cell slots, idle lanes included
+  constexpr int NTAB = int(sizeof(GeneralTab<NP, T>) / sizeof(T));
+  __shared__ __align__(16) T tl[NTAB];
+  __shared__ double X[CSL][32][3];       // corners; far corners of the face neighbours
+  __shared__ T A_[CSL][8][3];            // map coefficients
+  __shared__ T N_[CSL][6][4][3];         // normal columns of the neighbours' maps on the faces
+  __shared__ __align__(16) T L1[CSL][NDC], L2[CSL][NDC];  // y- and z-face contributions
 
-  __shared__ T U[NDC];
-  __shared__ T A0[NDC], A1[NDC], A2[NDC];   // x-stage (gradient) / F (flux) / y-stage (integration)
-  __shared__ T B0[NDC], B1[NDC], B2[NDC];   // y-stage (gradient) / z-stage (integration)
-  __shared__ T PA[NFACE][2][NF], PB[NFACE][2][NF];  // normal traces; later the projections
-  constexpr int NHC = NCORN / 2;            // corners per face
-  constexpr int NFV = DIM == 3 ? 11 : 5;    // face polynomials per face
-  __shared__ T C[NCORN][3];                 // map coefficients of the cell
-  // per face: tangents (3D: t1 = [0] + q2 [2], t2 = [1] + q1 [2]; 2D: t1 = [0]) and
-  // the normal-direction Jacobian columns of the cell (3D [3..6], 2D [1..2]) and of
-  // the neighbour (3D [7..10], 2D [3..4]) as bilinear (2D: linear) polynomials in
-  // the face coordinates (q1, q2)
-  __shared__ T FG[NFACE][NFV][3];
-  __shared__ T HI[NFACE][2];                // 1/h of the cell and of the neighbour
-  __shared__ GeneralTab<NP, T> tl;
-  // storage shared by arrays with disjoint lifetimes: the face neighbours (P0-P2)
-  // with the face fluxes (P4-P5); the corners (P0-P1) with the tangential traces (P3-P4)
-  constexpr int NUN = NFACE * NDC, NFLUX = NFACE * NF * (2 + DIM);
-  constexpr int NTR = 3 * NFACE * 2 * NF, NXD = (NCORN + NFACE * NHC) * 3;
-  __shared__ T RU[NUN > NFLUX ? NUN : NFLUX];
-  __shared__ double RX[(NTR * int(sizeof(T)) + 7) / 8 > NXD ? (NTR * int(sizeof(T)) + 7) / 8 : NXD];
-  T(*UN)[NDC] = reinterpret_cast<T(*)[NDC]>(RU);
-  T(*JV)[NF] = reinterpret_cast<T(*)[NF]>(RU);
-  T(*AV)[NF] = reinterpret_cast<T(*)[NF]>(RU + NFACE * NF);
-  T(*FH)[DIM][NF] = reinterpret_cast<T(*)[DIM][NF]>(RU + 2 * NFACE * NF);
-  // X[c]: corner c of the cell (c < NCORN), X[NCORN + f * NHC + c']: the corner of
-  // the neighbour across face f opposite face corner c'
-  double(*X)[3] = reinterpret_cast<double(*)[3]>(RX);
-  T(*VA)[2][NF] = reinterpret_cast<T(*)[2][NF]>(RX);
-  T(*DA)[2][NF] = reinterpret_cast<T(*)[2][NF]>(reinterpret_cast<T *>(RX) + NFACE * 2 * NF);
-  T(*VB)[2][NF] = reinterpret_cast<T(*)[2][NF]>(reinterpret_cast<T *>(RX) + 2 * NFACE * 2 * NF);
+  const int t = threadIdx.x, cs = t / NL, q = t % NL;
+  const int q0 = q % NP, q1 = q / NP;
+  const int64_t per = int64_t(gridDim.x) / 8;  // the grid is a multiple of eight blocks
+  const int64_t slot = (int64_t(blockIdx.x % 8) * per + blockIdx.x / 8) * CPB + cs;
+  const bool act = cs < CPB && slot < count;
+  const int64_t sl = act ? slot : 0;
+  const int64_t cell = cells ? int64_t(cells[sl]) : sl;
+  const int ci = int(cell);
+  const int cc[3] = {ci % n, (ci / n) % n, ci / (n * n)};
+  int ra[2][NP];  // ds_bpermute addresses of the rotations (NP != 4)
+  if constexpr(NP != 4)
+#pragma unroll
+    for(int r = 0; r < NP; ++r)
+    {
+      ra[0][r] = 4 * (cs * NL + (q0 + r) % NP + NP * q1);
+      ra[1][r] = 4 * (cs * NL + q0 + NP * ((q1 + r) % NP));
+    }
 
-  const int64_t cell = cells ? int64_t(cells[blockIdx.x]) : int64_t(blockIdx.x);
-  const int t = threadIdx.x;
-  const bool act = t < NDC;
-  const int ts = act ? t : 0;
-  // faces with a neighbour (bit f = 2 d + side) and the index of the cell's first
-  // vertex (vertex indices fit in 32 bits: (n + 1)^3 < 2^31 for n <= 1000)
-  int imask = 0, vbase = 0;
+  for(int i = t; i < NTAB; i += 64) tl[i] = reinterpret_cast<const T *>(&tab)[i];
+  // ---- loads: lines of the cell and of its face neighbours, vertices
+  const T *xc = x + cell * NDC;
+  const int at[3] = {NP * q, q0 + NL * q1, q};      // the lane's line along d in a cell
+  constexpr int st[3] = {1, NP, NL};
+  T ol[3][NP], nl[3][2][NP];
+#pragma unroll
+  for(int d = 0; d < 3; ++d)
   {
-    int r = int(cell);  // cells < n^3 <= 1000^3 < 2^31
-    int vst = 1;
-#pragma unroll
-    for(int d = 0; d < DIM; ++d)
+    const int64_t shift = (d == 0 ? int64_t(1) : d == 1 ? int64_t(n) : int64_t(n) * n) * NDC;
+    const T *pl = xc + at[d] - (cc[d] > 0 ? shift : 0), *pr = xc + at[d] + (cc[d] < n - 1 ? shift : 0);
+    if(d == 0)
     {
-      const int cd = r % n;
-      r /= n;
-      imask |= (cd > 0 ? 1 : 0) << (2 * d);
-      imask |= (cd < n - 1 ? 1 : 0) << (2 * d + 1);
-      vbase += cd * vst;
-      vst *= n + 1;
-    }
-  }
-  const int ix = ts % NP, iy = DIM > 1 ? (ts / NP) % NP : 0, iz = DIM > 2 ? ts / (NP * NP) : 0;
-  auto interior = [&](int f) { return ((imask >> f) & 1) != 0; };
-  auto nb_stride = [&](int d) {
-    int64_t st = 1;
-    for(int e = 0; e < d; ++e) st *= n;
-    return st;
-  };
-
-  // ---------------- P0: loads
-  {
-    const T *src = reinterpret_cast<const T *>(&tab);
-    T *dst = reinterpret_cast<T *>(&tl);
-    constexpr int NTAB = int(sizeof(GeneralTab<NP, T>) / sizeof(T));
-    for(int i = t; i < NTAB; i += NT) dst[i] = src[i];
-  }
-  if(act)
-  {
-    U[t] = x[cell * NDC + t];
-#pragma unroll
-    for(int f = 0; f < NFACE; ++f)
-      if(interior(f))
-      {
-        const int64_t st = nb_stride(f / 2);
-        UN[f][t] = x[(f % 2 == 1 ? cell + st : cell - st) * NDC + t];
-      }
-  }
-  {
-    int vs[3] = {1, n + 1, (n + 1) * (n + 1)};
-    const int vb = vbase;
-    for(int it = t; it < (NCORN + NFACE * NHC) * DIM; it += NT)
-    {
-      const int c = it / DIM, a = it % DIM;
-      int idx = vb;
-      if(c < NCORN)
-      {
-#pragma unroll
-        for(int e = 0; e < DIM; ++e) idx += ((c >> e) & 1) * vs[e];
-      }
-      else
-      {
-        const int f = (c - NCORN) / NHC, cp = (c - NCORN) % NHC;
-        if(!interior(f)) continue;
-        const int d = f / 2, e1 = d == 0 ? 1 : 0;
-        // offsets: 2 or -1 along d, the face corner's bits along e1 < e2
-#pragma unroll
-        for(int e = 0; e < DIM; ++e)
-          idx += (e == d ? (f % 2 == 1 ? 2 : -1) : (e == e1 ? (cp & 1) : (cp >> 1))) * vs[e];
-      }
-      X[c][a] = vert[int64_t(idx) * DIM + a];
-    }
-  }
-  __syncthreads();
-
-  // ---------------- P1: x-interpolation; map coefficients
-  if(act)
-  {
-    T v = 0, g = 0;
-    const int base = ts - ix;
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-    {
-      const T u = U[base + j];
-      v += tl.V[ix * NP + j] * u;
-      g += tl.Dv[ix * NP + j] * u;
-    }
-    A0[t] = v;
-    A1[t] = g;
-  }
-  for(int it = t; it < (NFACE + 1) * DIM; it += NT)
-  {
-    if(it >= NFACE * DIM)
-    {
-      // coordinate a of A_S = sum over subsets R of S of (-1)^{|S \ R|} X_R: one
-      // subtraction stage per direction
-      const int a = it - NFACE * DIM;
-      double c[NCORN];
-#pragma unroll
-      for(int R = 0; R < NCORN; ++R) c[R] = X[R][a];
-#pragma unroll
-      for(int e = 0; e < DIM; ++e)
-#pragma unroll
-        for(int S = 0; S < NCORN; ++S)
-          if((S >> e) & 1) c[S] -= c[S ^ (1 << e)];
-#pragma unroll
-      for(int S = 0; S < NCORN; ++S) C[S][a] = T(c[S]);
-      continue;
-    }
-    // face f, coordinate a: Y = the face's corners, E / En = the edges along the
-    // normal direction d of the cell / of the neighbour at those corners (pointing
-    // to increasing x_d), all formed in FP64
-    const int f = it / DIM, a = it % DIM;
-    const int d = f / 2, side = f % 2, e1 = d == 0 ? 1 : 0, e2 = d == 2 ? 1 : 2;
-    const bool inner = interior(f);
-    double Y[NHC], E[NHC], En[NHC];
-#pragma unroll
-    for(int cp = 0; cp < NHC; ++cp)
-    {
-      const int cy = (side << d) | ((cp & 1) << e1) | (DIM == 3 ? ((cp >> 1) << e2) : 0);
-      Y[cp] = X[cy][a];
-      const double z = X[cy ^ (1 << d)][a];
-      E[cp] = side ? Y[cp] - z : z - Y[cp];
-      const double w = inner ? X[NCORN + f * NHC + cp][a] : Y[cp];
-      En[cp] = side ? w - Y[cp] : Y[cp] - w;
-    }
-    if constexpr(DIM == 3)
-    {
-      FG[f][0][a] = T(Y[1] - Y[0]);
-      FG[f][1][a] = T(Y[2] - Y[0]);
-      FG[f][2][a] = T(Y[3] - Y[2] - Y[1] + Y[0]);
-      FG[f][3][a] = T(E[0]);
-      FG[f][4][a] = T(E[1] - E[0]);
-      FG[f][5][a] = T(E[2] - E[0]);
-      FG[f][6][a] = T(E[3] - E[2] - E[1] + E[0]);
-      FG[f][7][a] = T(En[0]);
-      FG[f][8][a] = T(En[1] - En[0]);
-      FG[f][9][a] = T(En[2] - En[0]);
-      FG[f][10][a] = T(En[3] - En[2] - En[1] + En[0]);
+      load_row<NP>(xc + at[0], ol[0]);
+      load_row<NP>(pl, nl[0][0]);
+      load_row<NP>(pr, nl[0][1]);
     }
     else
-    {
-      FG[f][0][a] = T(Y[1] - Y[0]);
-      FG[f][1][a] = T(E[0]);
-      FG[f][2][a] = T(E[1] - E[0]);
-      FG[f][3][a] = T(En[0]);
-      FG[f][4][a] = T(En[1] - En[0]);
-    }
-  }
-  __syncthreads();
-
-  // ---------------- P2: y-interpolation; traces along the face normals
-  T g0 = 0, g1 = 0, g2 = 0;
-  if(act)
-  {
-    const int base = ts - iy * NP;
-    T b0 = 0, b1 = 0, b2 = 0;
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-    {
-      const T a0 = A0[base + j * NP], a1 = A1[base + j * NP];
-      const T vy = tl.V[iy * NP + j], dy = tl.Dv[iy * NP + j];
-      b0 += vy * a1;
-      b1 += dy * a0;
-      b2 += vy * a0;
-    }
-    if constexpr(DIM == 2)
-    {
-      g0 = b0;
-      g1 = b1;
-    }
-    else
-    {
-      B0[t] = b0;
-      B1[t] = b1;
-      B2[t] = b2;
-    }
-  }
-  {
-    auto normal_trace = [&](int d, int side, int sd, int m) {
-      const int f = 2 * d + side;
-      if(sd == 1 && !interior(f)) return;
-      const int e1 = d == 0 ? 1 : 0, e2 = d == 2 ? 1 : 2;
-      const int i1 = m % NP, i2 = DIM == 3 ? m / NP : 0;
-      const int base = i1 * stride(e1) + (DIM == 3 ? i2 * stride(e2) : 0);
-      const T *src = sd == 0 ? U : UN[f];
-      const int fs = sd == 0 ? side : 1 - side;
-      T a = 0, bs = 0;
-#pragma unroll
-      for(int id = 0; id < NP; ++id)
-      {
-        const T u = src[base + id * stride(d)];
-        a += tl.f[fs][id] * u;
-        bs += tl.fd[fs][id] * u;
-      }
-      PA[f][sd][m] = a;
-      PB[f][sd][m] = bs;
-    };
-    if constexpr(DIM == 3 && 4 * NF <= NT && NT < 8 * NF)
-    {
-      // (3D Q3, Q4) the items (side, sd, m) of one normal direction fill a pass:
-      // one pass per direction, which makes d and the strides constants
-      if(t < 4 * NF)
-      {
-        const int side = t / (2 * NF), sd = (t / NF) % 2, m = t % NF;
-#pragma unroll
-        for(int d = 0; d < DIM; ++d) normal_trace(d, side, sd, m);
-      }
-    }
-    else
-      for(int o = t; o < NFACE * 2 * NF; o += NT)
-      {
-        const int f = o / (2 * NF);
-        normal_trace(f / 2, f % 2, (o / NF) % 2, o % NF);
-      }
-  }
-  __syncthreads();
-
-  // ---------------- P3: z-interpolation, geometry, reference flux; tangential
-  // traces along the first face direction
-  if(act)
-  {
-    if constexpr(DIM == 3)
-    {
-      const int base = ts - iz * NP * NP;
 #pragma unroll
       for(int j = 0; j < NP; ++j)
       {
-        const T vz = tl.V[iz * NP + j], dz = tl.Dv[iz * NP + j];
-        g0 += vz * B0[base + j * NP * NP];
-        g1 += vz * B1[base + j * NP * NP];
-        g2 += dz * B2[base + j * NP * NP];
+        ol[d][j] = xc[at[d] + j * st[d]];
+        nl[d][0][j] = pl[j * st[d]];
+        nl[d][1][j] = pr[j * st[d]];
       }
-    }
-    T xi[3] = {tl.qx[ix], tl.qx[iy], DIM == 3 ? tl.qx[iz] : T(0)};
-    T J[3][3], Ji[3][3];
-    coef_jacobian<DIM>(C, xi, J);
-    const T det = invert<DIM>(J, Ji);
-    const T jxw = fabs(det) * tl.qw[ix] * tl.qw[iy] * (DIM == 3 ? tl.qw[iz] : T(1));
-    const T g[3] = {g0, g1, g2};
-    T ph[3];
-#pragma unroll
-    for(int c = 0; c < DIM; ++c)
-    {
-      T s = 0;
-#pragma unroll
-      for(int bb = 0; bb < DIM; ++bb) s += Ji[bb][c] * g[bb];
-      ph[c] = s;  // physical gradient
-    }
-    T F[3];
-#pragma unroll
-    for(int a = 0; a < DIM; ++a)
-    {
-      T s = 0;
-#pragma unroll
-      for(int c = 0; c < DIM; ++c) s += Ji[a][c] * ph[c];
-      F[a] = s * jxw;
-    }
-    // F_a into the x-stage arrays (last read in P2)
-    A0[t] = F[0];
-    A1[t] = F[1];
-    if(DIM == 3) A2[t] = F[2];
   }
-  for(int o = t; o < NFACE * 2 * NF; o += NT)
   {
-    // (f, side, l1, i2): along e1 from the nodes i1 to the point l1
-    const int f = o / (2 * NF), sd = (o / NF) % 2, r = o % NF;
-    if(sd == 1 && !interior(f)) continue;
-    const int l1 = r % NP, i2 = r / NP;
-    T va = 0, da = 0, vb = 0;
-#pragma unroll
-    for(int i1 = 0; i1 < NP; ++i1)
+    // vertex c < 8: corner c; else the corner of the neighbour across face
+    // f = (c - 8) / 4 opposite face corner (c - 8) % 4 (absent neighbour: any vertex)
+    const int v1 = n + 1, v2 = v1 * v1, vb = cc[0] + v1 * cc[1] + v2 * cc[2];
+    for(int c = q; c < 32; c += NL)
     {
-      const T a = PA[f][sd][i1 + NP * i2], pb = PB[f][sd][i1 + NP * i2];
-      const T v = tl.V[l1 * NP + i1];
-      va += v * a;
-      da += tl.Dv[l1 * NP + i1] * a;
-      vb += v * pb;
-    }
-    VA[f][sd][r] = va;
-    DA[f][sd][r] = da;
-    VB[f][sd][r] = vb;
-  }
-  __syncthreads();
-
-  // ---------------- P4: z-integration; face fluxes at every face point
-  if(act)
-  {
-    if constexpr(DIM == 3)
-    {
-      const int base = ts - iz * NP * NP;
-      T s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-      for(int q = 0; q < NP; ++q)
+      const int f = (c - 8) >> 2, d = f >> 1, side = f & 1;
+      int o0 = c & 1, o1 = (c >> 1) & 1, o2 = c >> 2;
+      if(c >= 8)
       {
-        const T vz = tl.V[q * NP + iz], dz = tl.Dv[q * NP + iz];
-        s0 += vz * A0[base + q * NP * NP];
-        s1 += vz * A1[base + q * NP * NP];
-        s2 += dz * A2[base + q * NP * NP];
+        const int far = side ? 2 : -1, b1 = c & 1, b2 = (c >> 1) & 1;
+        o0 = d == 0 ? far : b1;
+        o1 = d == 1 ? far : (d == 0 ? b1 : b2);
+        o2 = d == 2 ? far : b2;
+        const int cd = d == 0 ? cc[0] : d == 1 ? cc[1] : cc[2];
+        if(side ? cd == n - 1 : cd == 0) o0 = o1 = o2 = 0;
       }
-      B0[t] = s0;
-      B1[t] = s1;
-      B2[t] = s2;
-    }
-  }
-  const T gamma = p == 0 ? T(1) : T(p) * T(p + 1);
-  for(int pt = t; pt < NFACE * NF; pt += NT)
-  {
-    const int f = pt / NF, l = pt % NF;
-    const int side = f % 2;
-    const bool inner = interior(f);
-    const int l1 = l % NP, l2 = DIM == 3 ? l / NP : 0;
-    // traces: value, normal and tangential reference derivatives of both sides
-    T tr[2][4];  // [side][value, d_normal, d_e1, d_e2]
+      const double *pv = vert + int64_t(vb + o0 + v1 * o1 + v2 * o2) * 3;
 #pragma unroll
-    for(int sd = 0; sd < 2; ++sd)
-    {
-      T u = 0, gn = 0, gt1 = 0, gt2 = 0;
-      if(sd == 0 || inner)
-      {
-#pragma unroll
-        for(int i2 = 0; i2 < NP2; ++i2)
-        {
-          const int r = l1 + NP * i2;
-          const T v2 = DIM == 3 ? tl.V[l2 * NP + i2] : T(1);
-          const T d2 = DIM == 3 ? tl.Dv[l2 * NP + i2] : T(0);
-          const T va = VA[f][sd][r];
-          u += v2 * va;
-          gn += v2 * VB[f][sd][r];
-          gt1 += v2 * DA[f][sd][r];
-          gt2 += d2 * va;
-        }
-      }
-      tr[sd][0] = u;
-      tr[sd][1] = gn;
-      tr[sd][2] = gt1;
-      tr[sd][3] = gt2;
-    }
-    const T q1 = tl.qx[l1], q2 = DIM == 3 ? tl.qx[l2] : T(0);
-    // tangents and the normal-direction Jacobian columns of both cells
-    T t1[3], t2[3] = {0, 0, 0}, jd[3], jn[3], w[3];
-#pragma unroll
-    for(int a = 0; a < DIM; ++a)
-    {
-      if constexpr(DIM == 3)
-      {
-        t1[a] = FG[f][0][a] + q2 * FG[f][2][a];
-        t2[a] = FG[f][1][a] + q1 * FG[f][2][a];
-        jd[a] = FG[f][3][a] + q1 * FG[f][4][a] + q2 * (FG[f][5][a] + q1 * FG[f][6][a]);
-        jn[a] = FG[f][7][a] + q1 * FG[f][8][a] + q2 * (FG[f][9][a] + q1 * FG[f][10][a]);
-      }
-      else
-      {
-        t1[a] = FG[f][0][a];
-        jd[a] = FG[f][1][a] + q1 * FG[f][2][a];
-        jn[a] = FG[f][3][a] + q1 * FG[f][4][a];
-      }
-    }
-    if constexpr(DIM == 3)
-    {
-      w[0] = t1[1] * t2[2] - t1[2] * t2[1];
-      w[1] = t1[2] * t2[0] - t1[0] * t2[2];
-      w[2] = t1[0] * t2[1] - t1[1] * t2[0];
-    }
-    else
-    {
-      w[0] = t1[1];
-      w[1] = -t1[0];
-    }
-    T ww = 0, wj = 0;
-#pragma unroll
-    for(int a = 0; a < DIM; ++a)
-    {
-      ww += w[a] * w[a];
-      wj += w[a] * jd[a];
-    }
-    const T nw = root(ww), inw = recip(nw);
-    // outward: n . J_d > 0 on the face x_d = 1 of the cell, < 0 on x_d = 0
-    const T sg = ((wj > T(0)) == (side == 1)) ? inw : -inw;
-    T nv[3];
-#pragma unroll
-    for(int a = 0; a < DIM; ++a) nv[a] = sg * w[a];
-    const T wq = tl.qw[l1] * (DIM == 3 ? tl.qw[l2] : T(1));
-    const T dS = nw * wq;
-    // Gram matrix of the tangents (2D: t1 . t1) and its inverse
-    T g11 = 0, g12 = 0, g22 = 0;
-#pragma unroll
-    for(int a = 0; a < DIM; ++a)
-    {
-      g11 += t1[a] * t1[a];
-      g12 += t1[a] * t2[a];
-      g22 += t2[a] * t2[a];
-    }
-    const T iG = DIM == 3 ? recip(g11 * g22 - g12 * g12) : recip(g11);
-    // c = J^{-1} n in the face frame: [0] normal direction, [1] e1, [2] e2
-    auto coeffs = [&](const T *jc, T *c) {
-      T jnv = 0, r1 = 0, r2 = 0;
-#pragma unroll
-      for(int a = 0; a < DIM; ++a)
-      {
-        jnv += jc[a] * nv[a];
-        r1 += t1[a] * jc[a];
-        r2 += t2[a] * jc[a];
-      }
-      const T cd = recip(jnv);
-      c[0] = cd;
-      if constexpr(DIM == 3)
-      {
-        c[1] = -cd * (g22 * r1 - g12 * r2) * iG;
-        c[2] = -cd * (g11 * r2 - g12 * r1) * iG;
-      }
-      else
-      {
-        c[1] = -cd * r1 * iG;
-        c[2] = T(0);
-      }
-    };
-    T co[3];
-    coeffs(jd, co);
-    const T dno = tr[0][1] * co[0] + tr[0][2] * co[1] + (DIM == 3 ? tr[0][3] * co[2] : T(0));
-    T jv, av, fnd, cnd = T(1);
-    if(inner)
-    {
-      T cn[3];
-      coeffs(jn, cn);
-      cnd = cn[0];
-      const T dnn =
-        tr[1][1] * cn[0] + tr[1][2] * cn[1] + (DIM == 3 ? tr[1][3] * cn[2] : T(0));
-      const T jump = tr[0][0] - tr[1][0];
-      jv = dS * jump;
-      av = -dS * T(0.5) * (dno + dnn);
-      fnd = dS * T(-0.5) * jump;
-    }
-    else
-    {
-      jv = dS * tr[0][0];
-      av = -dS * dno;
-      fnd = -dS * tr[0][0];
-    }
-    JV[f][l] = jv;
-    AV[f][l] = av;
-#pragma unroll
-    for(int bb = 0; bb < DIM; ++bb) FH[f][bb][l] = fnd * co[bb];  // face frame
-    // inverse penalty lengths 1/h = |(J^{-1} n)_d| at the first face quadrature
-    // point of both cells (apps/laplace_integrator.h:651-656, 692-693)
-    if(l == 0)
-    {
-      HI[f][0] = fabs(co[0]);
-      HI[f][1] = inner ? fabs(cnd) : T(1);
+      for(int a = 0; a < 3; ++a) X[cs][c][a] = pv[a];
     }
   }
   __syncthreads();
-
-  // ---------------- P5: y-integration; face projections on the tangential
-  // test functions (into PA / PB, last read in P3)
-  if(act)
+  // ---- traces on the tangential nodes: value and normal derivative of the cell and
+  // of its neighbour (0 where there is none), on both sides of every direction
+  T vo[3][2], go_[3][2], vn[3][2], gn_[3][2];
+#pragma unroll
+  for(int d = 0; d < 3; ++d)
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
+      T dd = 0, dn = 0;
+#pragma unroll
+      for(int j = 0; j < NP; ++j)
+      {
+        dd += tab.fd[side][j] * ol[d][j];
+        dn += tab.fd[1 - side][j] * nl[d][side][j];
+      }
+      vo[d][side] = ol[d][side ? P : 0];
+      go_[d][side] = dd;
+      vn[d][side] = in ? nl[d][side][side ? 0 : P] : T(0);
+      gn_[d][side] = in ? dn : T(0);
+    }
+  // ---- map coefficients, formed in FP64: item (coordinate a) of the cell, then of
+  // the six neighbours' normal columns
+  for(int it = q; it < 21; it += NL)
   {
-    if constexpr(DIM == 3)
+    const int a = it % 3, f = it / 3 - 1;
+    if(f < 0)
     {
-      const int base = ts - iy * NP;
-      T s0 = 0, s12 = 0;
+      double c[8];
 #pragma unroll
-      for(int q = 0; q < NP; ++q)
-      {
-        const T vy = tl.V[q * NP + iy], dy = tl.Dv[q * NP + iy];
-        s0 += vy * B0[base + q * NP];
-        s12 += dy * B1[base + q * NP] + vy * B2[base + q * NP];
-      }
-      A2[t] = s0;    // A2 was last read in P4
-      U[t] = s12;    // U was last read in P2
+      for(int R = 0; R < 8; ++R) c[R] = X[cs][R][a];
+#pragma unroll
+      for(int e = 0; e < 3; ++e)
+#pragma unroll
+        for(int S = 0; S < 8; ++S)
+          if((S >> e) & 1) c[S] -= c[S ^ (1 << e)];
+#pragma unroll
+      for(int S = 0; S < 8; ++S) A_[cs][S][a] = T(c[S]);
+      continue;
     }
-    else
+    const int d = f >> 1, side = f & 1;
+    const int m1 = d == 0 ? 2 : 1, m2 = d == 2 ? 2 : 4;  // corner bits along e1, e2
+    const bool in = side ? cc[0] * (d == 0) + cc[1] * (d == 1) + cc[2] * (d == 2) < n - 1
+                         : cc[0] * (d == 0) + cc[1] * (d == 1) + cc[2] * (d == 2) > 0;
+    double e[4];
+#pragma unroll
+    for(int cp = 0; cp < 4; ++cp)
     {
-      const int base = ts - iy * NP;
-      T s0 = 0, s1 = 0;
-#pragma unroll
-      for(int q = 0; q < NP; ++q)
-      {
-        s0 += tl.V[q * NP + iy] * A0[base + q * NP];
-        s1 += tl.Dv[q * NP + iy] * A1[base + q * NP];
-      }
-      A2[t] = s0;
-      U[t] = s1;
+      const int cy = (side << d) | ((cp & 1) ? m1 : 0) | ((cp >> 1) ? m2 : 0);
+      // absent neighbour: the cell's own edge (finite; its products are multiplied by 0)
+      const double far = in ? X[cs][8 + 4 * f + cp][a] : X[cs][cy ^ (1 << d)][a];
+      const double ed = far - X[cs][cy][a];
+      e[cp] = (side == 1) == in ? ed : -ed;
     }
-  }
-  if constexpr(DIM == 3)
-  {
-    // projections sum-factorised over the two face coordinates, first over l1
-    // (into the trace storage, last read in P4): at (i1, l2)
-    //   SA = sum_l1 phi_i1(l1) (sigma JV + AV) + phi'_i1(l1) FH_e1
-    //   SB = sum_l1 phi_i1(l1) FH_e2,  SC = sum_l1 phi_i1(l1) FH_n
-    T(*SA)[NF] = reinterpret_cast<T(*)[NF]>(RX);
-    T(*SB)[NF] = SA + NFACE;
-    T(*SC)[NF] = SA + 2 * NFACE;
-    for(int it = t; it < NFACE * NF; it += NT)
-    {
-      const int f = it / NF, m = it % NF;
-      const int i1 = m % NP, l2 = m / NP;
-      const T sigma = interior(f) ? T(ip) * gamma * T(0.5) * (HI[f][0] + HI[f][1])
-                                  : T(ip) * T(2) * gamma * HI[f][0];
-      T sa = 0, sb = 0, sc = 0;
-#pragma unroll
-      for(int l1 = 0; l1 < NP; ++l1)
-      {
-        const int l = l1 + NP * l2;
-        const T v = tl.V[l1 * NP + i1], dv = tl.Dv[l1 * NP + i1];
-        sa += v * (sigma * JV[f][l] + AV[f][l]) + dv * FH[f][1][l];
-        sb += v * FH[f][2][l];
-        sc += v * FH[f][0][l];
-      }
-      SA[f][m] = sa;
-      SB[f][m] = sb;
-      SC[f][m] = sc;
-    }
-    __syncthreads();
-    // then over l2: the projections on phi_i1 phi_i2 (value) and on the normal
-    // derivative's coefficient
-    for(int it = t; it < NFACE * NF; it += NT)
-    {
-      const int f = it / NF, m = it % NF;
-      const int i1 = m % NP, i2 = m / NP;
-      T pv = 0, pd = 0;
-#pragma unroll
-      for(int l2 = 0; l2 < NP; ++l2)
-      {
-        const int r = i1 + NP * l2;
-        const T v = tl.V[l2 * NP + i2], dv = tl.Dv[l2 * NP + i2];
-        pv += v * SA[f][r] + dv * SB[f][r];
-        pd += v * SC[f][r];
-      }
-      PA[f][0][m] = pv;
-      PB[f][0][m] = pd;
-    }
-  }
-  else
-  {
-    for(int it = t; it < NFACE * NF; it += NT)
-    {
-      const int f = it / NF, i1 = it % NF;
-      const T sigma = interior(f) ? T(ip) * gamma * T(0.5) * (HI[f][0] + HI[f][1])
-                                  : T(ip) * T(2) * gamma * HI[f][0];
-      T pv = 0, pd = 0;
-#pragma unroll
-      for(int l = 0; l < NF; ++l)
-      {
-        const T v = tl.V[l * NP + i1];
-        pv += v * (sigma * JV[f][l] + AV[f][l]) + tl.Dv[l * NP + i1] * FH[f][1][l];
-        pd += v * FH[f][0][l];
-      }
-      PA[f][0][i1] = pv;
-      PB[f][0][i1] = pd;
-    }
+    N_[cs][f][0][a] = T(e[0]);
+    N_[cs][f][1][a] = T(e[1] - e[0]);
+    N_[cs][f][2][a] = T(e[2] - e[0]);
+    N_[cs][f][3][a] = T(e[3] - e[2] - e[1] + e[0]);
   }
   __syncthreads();
+  // For NP >= 4 the lanes' rows of the tables and the map coefficients are read from
+  // LDS again for every face (a compiler fence keeps them from staying in registers,
+  // where they spill: 64^3 Q3 FP64 556 us kept, 412 us re-read); shorter lines keep
+  // them (60^3 Q2 FP64 244 us kept, 300 us re-read)
+  auto rows = [&](int m, int q_, T *o) {
+#pragma unroll
+    for(int r = 0; r < NP; ++r) o[r] = tl[2 * NL + 4 * NP + m * NL + q_ * NP + r];
+  };
+  T A[8][3], Va[NP], Da[NP], VaT[NP], DaT[NP], Vb[NP], Db[NP], VbT[NP], DbT[NP];
+  auto fetch = [&]() {
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for(int S = 1; S < 8; ++S)
+#pragma unroll
+      for(int a = 0; a < 3; ++a) A[S][a] = A_[cs][S][a];
+    rows(0, q0, Va), rows(1, q0, Da), rows(2, q0, VaT), rows(3, q0, DaT);
+    rows(0, q1, Vb), rows(1, q1, Db), rows(2, q1, VbT), rows(3, q1, DbT);
+  };
+  fetch();
+  const T p0 = tl[2 * NL + q0], p1 = tl[2 * NL + q1];                  // points along the lane indices
+  const T wq = tl[2 * NL + NP + q0] * tl[2 * NL + NP + q1];
 
-  // ---------------- P6: x-integration and the face terms of this test function
-  if(act)
+  T acc[3][NP];
+#pragma unroll
+  for(int d = 0; d < 3; ++d)
+#pragma unroll
+    for(int j = 0; j < NP; ++j) acc[d][j] = 0;
+
+  // ---------------- cell term
   {
-    const int base = ts - ix;
-    T acc = 0;
+    T F0[NP], F1[NP], F2[NP];
+    T g0[NP], g1[NP], g2[NP];
 #pragma unroll
-    for(int q = 0; q < NP; ++q)
-      acc += tl.Dv[q * NP + ix] * A2[base + q] + tl.V[q * NP + ix] * U[base + q];
-    const int ti[3] = {ix, iy, iz};
-#pragma unroll
-    for(int f = 0; f < NFACE; ++f)
+    for(int i = 0; i < NP; ++i)
     {
-      const int d = f / 2, side = f % 2;
-      const int e1 = d == 0 ? 1 : 0, e2 = d == 2 ? 1 : 2;
-      const int m = ti[e1] + (DIM == 3 ? NP * ti[e2] : 0);
-      acc += tl.f[side][ti[d]] * PA[f][0][m] + tl.fd[side][ti[d]] * PB[f][0][m];
+      T v = 0, g = 0, rv[NP], rg[NP], r2[NP];
+#pragma unroll
+      for(int j = 0; j < NP; ++j)
+      {
+        v += tab.V[i * NP + j] * ol[0][j];
+        g += tab.Dv[i * NP + j] * ol[0][j];
+      }
+      lane_gather<NP, 0>(v, ra[0], rv);
+      lane_gather<NP, 0>(g, ra[0], rg);
+      lane_gather<NP, 1>(dotn<NP>(Va, rg), ra[1], r2);
+      g0[i] = dotn<NP>(Vb, r2);
+      lane_gather<NP, 1>(dotn<NP>(Da, rv), ra[1], r2);
+      g1[i] = dotn<NP>(Vb, r2);
+      lane_gather<NP, 1>(dotn<NP>(Va, rv), ra[1], r2);
+      g2[i] = dotn<NP>(Db, r2);
     }
-    if(RESIDUAL)
-      y[cell * NDC + t] = b[cell * NDC + t] - acc;
-    else
-      y[cell * NDC + t] = acc;
+    // Jacobian columns: J_0 constant along the line, J_1 and J_2 linear in x
+    T c0[3], c1[3], s1[3], c2[3], s2[3];
+#pragma unroll
+    for(int a = 0; a < 3; ++a)
+    {
+      s1[a] = A[3][a] + p1 * A[7][a];
+      s2[a] = A[5][a] + p0 * A[7][a];
+      c0[a] = A[1][a] + p1 * A[5][a] + p0 * s1[a];
+      c1[a] = A[2][a] + p1 * A[6][a];
+      c2[a] = A[4][a] + p0 * A[6][a];
+    }
+#pragma unroll
+    for(int i = 0; i < NP; ++i)
+    {
+      const T xi = tab.qx[i];
+      T J1[3], J2[3], R0[3], R1[3], R2[3];
+#pragma unroll
+      for(int a = 0; a < 3; ++a)
+      {
+        J1[a] = c1[a] + xi * s1[a];
+        J2[a] = c2[a] + xi * s2[a];
+      }
+      // rows of the adjugate: J_1 x J_2, J_2 x J_0, J_0 x J_1
+#pragma unroll
+      for(int a = 0; a < 3; ++a)
+      {
+        const int k = (a + 1) % 3, l = (a + 2) % 3;
+        R0[a] = J1[k] * J2[l] - J1[l] * J2[k];
+        R1[a] = J2[k] * c0[l] - J2[l] * c0[k];
+        R2[a] = c0[k] * J1[l] - c0[l] * J1[k];
+      }
+      const T det = c0[0] * R0[0] + c0[1] * R0[1] + c0[2] * R0[2];
+      const T w = wq * tab.qw[i] * fast_recip(fabs(det));
+      T h[3];
+#pragma unroll
+      for(int a = 0; a < 3; ++a) h[a] = w * (R0[a] * g0[i] + R1[a] * g1[i] + R2[a] * g2[i]);
+      F0[i] = R0[0] * h[0] + R0[1] * h[1] + R0[2] * h[2];
+      F1[i] = R1[0] * h[0] + R1[1] * h[1] + R1[2] * h[2];
+      F2[i] = R2[0] * h[0] + R2[1] * h[1] + R2[2] * h[2];
+    }
+#pragma unroll
+    for(int i = 0; i < NP; ++i)
+    {
+      T r0[NP], r1[NP], r2[NP];
+      lane_gather<NP, 1>(F0[i], ra[1], r0);
+      lane_gather<NP, 1>(F1[i], ra[1], r1);
+      lane_gather<NP, 1>(F2[i], ra[1], r2);
+      const T z0 = dotn<NP>(VbT, r0), z1 = dotn<NP>(VbT, r1), z2 = dotn<NP>(DbT, r2);
+      lane_gather<NP, 0>(z0, ra[0], r0);
+      lane_gather<NP, 0>(z1, ra[0], r1);
+      lane_gather<NP, 0>(z2, ra[0], r2);
+      const T a0 = dotn<NP>(VaT, r0), a1 = dotn<NP>(DaT, r1) + dotn<NP>(VaT, r2);
+#pragma unroll
+      for(int j = 0; j < NP; ++j) acc[0][j] += tab.Dv[i * NP + j] * a0 + tab.V[i * NP + j] * a1;
+    }
   }
+
+  // ---------------- faces
+  const int lane0 = min(cs, CPB - 1) * NL;  // the lane of the cell's first face point
+#pragma unroll
+  for(int d = 0; d < 3; ++d)
+  {
+    const int bd = 1 << d, b1 = d == 0 ? 2 : 1, b2 = d == 2 ? 2 : 4, b12 = b1 | b2;
+    T jd[3];
+#pragma unroll
+    for(int a = 0; a < 3; ++a)
+      jd[a] = A[bd][a] + p0 * A[bd | b1][a] + p1 * (A[bd | b2][a] + p0 * A[7][a]);
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const int f = 2 * d + side;
+      const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
+      if constexpr(NP >= 4) fetch();
+      // at the face points: jump, normal and tangential reference derivatives
+      T r0[NP], r1[NP], jump, go[3], gn[3];
+      {
+        T m[NP];
+        lane_gather<NP, 0>(vo[d][side], ra[0], r0);
+        lane_gather<NP, 0>(vn[d][side], ra[0], r1);
+        const T Vo = dotn<NP>(Va, r0), Vn = dotn<NP>(Va, r1);
+        const T Do = dotn<NP>(Da, r0), Dn = dotn<NP>(Da, r1);
+        lane_gather<NP, 0>(go_[d][side], ra[0], r0);
+        lane_gather<NP, 0>(gn_[d][side], ra[0], r1);
+        const T No = dotn<NP>(Va, r0), Nn = dotn<NP>(Va, r1);
+        lane_gather<NP, 1>(Vo, ra[1], r0);
+        lane_gather<NP, 1>(Vn, ra[1], r1);
+        go[2] = dotn<NP>(Db, r0);
+        gn[2] = dotn<NP>(Db, r1);
+#pragma unroll
+        for(int r = 0; r < NP; ++r) m[r] = r0[r] - r1[r];
+        jump = dotn<NP>(Vb, m);
+        lane_gather<NP, 1>(Do, ra[1], r0);
+        lane_gather<NP, 1>(Dn, ra[1], r1);
+        go[1] = dotn<NP>(Vb, r0);
+        gn[1] = dotn<NP>(Vb, r1);
+        lane_gather<NP, 1>(No, ra[1], r0);
+        lane_gather<NP, 1>(Nn, ra[1], r1);
+        go[0] = dotn<NP>(Vb, r0);
+        gn[0] = dotn<NP>(Vb, r1);
+      }
+      // geometry
+      T t1[3], t2[3], jn[3], w[3];
+#pragma unroll
+      for(int a = 0; a < 3; ++a)
+      {
+        const T s = side ? A[b12][a] + A[7][a] : A[b12][a];
+        t1[a] = (side ? A[b1][a] + A[bd | b1][a] : A[b1][a]) + p1 * s;
+        t2[a] = (side ? A[b2][a] + A[bd | b2][a] : A[b2][a]) + p0 * s;
+        jn[a] = N_[cs][f][0][a] + p0 * N_[cs][f][1][a] + p1 * (N_[cs][f][2][a] + p0 * N_[cs][f][3][a]);
+      }
+#pragma unroll
+      for(int a = 0; a < 3; ++a)
+      {
+        const int k = (a + 1) % 3, l = (a + 2) % 3;
+        w[a] = t1[k] * t2[l] - t1[l] * t2[k];
+      }
+      T ww = 0, wo = 0, wn = 0, g11 = 0, g12 = 0, g22 = 0, o1 = 0, o2 = 0, n1 = 0, n2 = 0;
+#pragma unroll
+      for(int a = 0; a < 3; ++a)
+      {
+        ww += w[a] * w[a];
+        wo += w[a] * jd[a];
+        wn += w[a] * jn[a];
+        g11 += t1[a] * t1[a];
+        g12 += t1[a] * t2[a];
+        g22 += t2[a] * t2[a];
+        o1 += t1[a] * jd[a];
+        o2 += t2[a] * jd[a];
+        n1 += t1[a] * jn[a];
+        n2 += t2[a] * jn[a];
+      }
+      // outward: the normal derivative grows along J_d on side 1, against it on side 0
+      const T sg = (wo > T(0)) == (side == 1) ? T(1) : T(-1);
+      const T io = sg * fast_recip(wo), in_ = sg * fast_recip(wn);
+      const T nw = root(ww);
+      const T ko[3] = {io * ww, io * (g12 * o2 - g22 * o1), io * (g12 * o1 - g11 * o2)};
+      const T kn[3] = {in_ * ww, in_ * (g12 * n2 - g22 * n1), in_ * (g12 * n1 - g11 * n2)};
+      // penalty: inverse lengths |(J^{-1} n)_d| at the first face point of both cells
+      // (apps/laplace_integrator.h:651-656, 692-693)
+      T sigma = nw * (in ? T(0.5) * (fabs(io) + fabs(in_)) : T(2) * fabs(io));
+      sigma = ipg * lane_read(sigma, lane0);
+      const T hf = (in ? T(0.5) : T(1)) * wq;
+      const T pa = sigma * (nw * wq) * jump - hf * (ko[0] * go[0] + ko[1] * go[1] + ko[2] * go[2] +
+                                                    kn[0] * gn[0] + kn[1] * gn[1] + kn[2] * gn[2]);
+      const T hj = -hf * jump;
+      // projections on the tangential test functions
+      T ra_[NP], rb[NP], rc[NP];
+      lane_gather<NP, 1>(pa, ra[1], ra_);
+      lane_gather<NP, 1>(hj * ko[2], ra[1], rb);
+      const T sa = dotn<NP>(VbT, ra_) + dotn<NP>(DbT, rb);
+      lane_gather<NP, 1>(hj * ko[1], ra[1], rb);
+      lane_gather<NP, 1>(hj * ko[0], ra[1], rc);
+      const T sb = dotn<NP>(VbT, rb), sc = dotn<NP>(VbT, rc);
+      lane_gather<NP, 0>(sa, ra[0], ra_);
+      lane_gather<NP, 0>(sb, ra[0], rb);
+      lane_gather<NP, 0>(sc, ra[0], rc);
+      const T pv = dotn<NP>(VaT, ra_) + dotn<NP>(DaT, rb), pd = dotn<NP>(VaT, rc);
+#pragma unroll
+      for(int j = 0; j < NP; ++j) acc[d][j] += tab.fd[side][j] * pd;
+      acc[d][side ? P : 0] += pv;
+    }
+  }
+#pragma unroll
+  for(int j = 0; j < NP; ++j)
+  {
+    L1[cs][at[1] + j * st[1]] = acc[1][j];
+    L2[cs][at[2] + j * st[2]] = acc[2][j];
+  }
+  __syncthreads();
+  if(!act) return;
+  T out[NP];
+#pragma unroll
+  for(int j = 0; j < NP; ++j) out[j] = acc[0][j] + L1[cs][NP * q + j] + L2[cs][NP * q + j];
+  if(RESIDUAL)
+  {
+    T bv[NP];
+    load_row<NP>(b + cell * NDC + NP * q, bv);
+#pragma unroll
+    for(int j = 0; j < NP; ++j) out[j] = bv[j] - out[j];
+  }
+  store_row<NP>(y + cell * NDC + NP * q, out);
+}
+
+// the 2D form: a cell is NP lanes, 64 / NP cells per block
+template<int NP, typename VT, bool RESIDUAL>
+__global__ void __launch_bounds__(64, 2)
+k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
+                const double *__restrict__ vert, const GeneralTab<NP, VT> tab, const int n,
+                const VT ipg, const uint32_t *__restrict__ cells, const int64_t count)
+{
+  using T = VT;
+  constexpr int NDC = NP * NP, CPB = moved_cells_per_block<2, NP>(), P = NP - 1;
+  constexpr int CSL = (64 + NP - 1) / NP;  // cell slots, idle lanes included
+  __shared__ double X[CSL][12][2];         // corners; far corners of the face neighbours
+  __shared__ T A_[CSL][4][2];              // map coefficients
+  __shared__ T N_[CSL][4][2][2];           // normal columns of the neighbours' maps on the faces
+  __shared__ __align__(16) T L1[CSL][NDC];  // y-face contributions
+
+  const int t = threadIdx.x, cs = t / NP, q = t % NP;
+  const int64_t per = int64_t(gridDim.x) / 8;  // the grid is a multiple of eight blocks
+  const int64_t slot = (int64_t(blockIdx.x % 8) * per + blockIdx.x / 8) * CPB + cs;
+  const bool act = cs < CPB && slot < count;
+  const int64_t sl = act ? slot : 0;
+  const int64_t cell = cells ? int64_t(cells[sl]) : sl;
+  const int cc[2] = {int(cell) % n, int(cell) / n};
+  int ra[NP];  // ds_bpermute addresses of the rotations (NP != 4)
+#pragma unroll
+  for(int r = 0; r < NP; ++r) ra[r] = 4 * (cs * NP + (q + r) % NP);
+
+  {
+    // vertex c < 4: corner c; else the corner of the neighbour across face
+    // f = (c - 4) / 2 opposite face corner (c - 4) % 2 (absent neighbour: any vertex)
+    const int vb = cc[0] + (n + 1) * cc[1];
+    for(int c = q; c < 12; c += NP)
+    {
+      const int f = (c - 4) >> 1, d = f >> 1, side = f & 1;
+      int o0 = c & 1, o1 = c >> 1;
+      if(c >= 4)
+      {
+        const int far = side ? 2 : -1;
+        o0 = d == 0 ? far : (c & 1);
+        o1 = d == 1 ? far : (c & 1);
+        const int cd = d == 0 ? cc[0] : cc[1];
+        if(side ? cd == n - 1 : cd == 0) o0 = o1 = 0;
+      }
+      const double *pv = vert + int64_t(vb + o0 + (n + 1) * o1) * 2;
+      X[cs][c][0] = pv[0];
+      X[cs][c][1] = pv[1];
+    }
+  }
+  const T *xc = x + cell * NDC;
+  T u[NP], vo[2][2], go_[2][2], vn[2][2], gn_[2][2];
+#pragma unroll
+  for(int d = 0; d < 2; ++d)
+  {
+    const int at = d == 0 ? NP * q : q, st = d == 0 ? 1 : NP;
+    T ol[NP];
+#pragma unroll
+    for(int j = 0; j < NP; ++j) ol[j] = xc[at + j * st];
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
+      const int64_t shift = (d == 0 ? int64_t(1) : int64_t(n)) * NDC;
+      const T *pn = xc + at + (in ? (side ? shift : -shift) : 0);
+      T dd = 0, dn = 0, nl[NP];
+#pragma unroll
+      for(int j = 0; j < NP; ++j)
+      {
+        nl[j] = pn[j * st];
+        dd += tab.fd[side][j] * ol[j];
+        dn += tab.fd[1 - side][j] * nl[j];
+      }
+      vo[d][side] = ol[side ? P : 0];
+      go_[d][side] = dd;
+      vn[d][side] = in ? nl[side ? 0 : P] : T(0);
+      gn_[d][side] = in ? dn : T(0);
+    }
+    if(d == 0)
+#pragma unroll
+      for(int j = 0; j < NP; ++j) u[j] = ol[j];
+  }
+  // the lanes' rows of the tables (kernel arguments, read by lane)
+  const T *tk = reinterpret_cast<const T *>(&tab);
+  T Va[NP], Da[NP], VaT[NP], DaT[NP];
+#pragma unroll
+  for(int r = 0; r < NP; ++r)
+  {
+    const int at = 2 * NDC + 4 * NP + q * NP + r;
+    Va[r] = tk[at];
+    Da[r] = tk[at + NDC];
+    VaT[r] = tk[at + 2 * NDC];
+    DaT[r] = tk[at + 3 * NDC];
+  }
+  const T p0 = tk[2 * NDC + q], wq = tk[2 * NDC + NP + q];
+  __syncthreads();
+  // map coefficients, formed in FP64: item (coordinate a) of the cell, then of the
+  // four neighbours' normal columns
+  for(int it = q; it < 10; it += NP)
+  {
+    const int a = it & 1, f = (it >> 1) - 1;
+    if(f < 0)
+    {
+      const double c0 = X[cs][0][a], c1 = X[cs][1][a], c2 = X[cs][2][a], c3 = X[cs][3][a];
+      A_[cs][1][a] = T(c1 - c0);
+      A_[cs][2][a] = T(c2 - c0);
+      A_[cs][3][a] = T(c3 - c2 - (c1 - c0));
+      continue;
+    }
+    const int d = f >> 1, side = f & 1, m1 = d == 0 ? 2 : 1;
+    const int cd = d == 0 ? cc[0] : cc[1];
+    const bool in = side ? cd < n - 1 : cd > 0;
+    double e[2];
+#pragma unroll
+    for(int cp = 0; cp < 2; ++cp)
+    {
+      const int cy = (side << d) | (cp ? m1 : 0);
+      // absent neighbour: the cell's own edge (finite; its products are multiplied by 0)
+      const double far = in ? X[cs][4 + 2 * f + cp][a] : X[cs][cy ^ (1 << d)][a];
+      const double ed = far - X[cs][cy][a];
+      e[cp] = (side == 1) == in ? ed : -ed;
+    }
+    N_[cs][f][0][a] = T(e[0]);
+    N_[cs][f][1][a] = T(e[1] - e[0]);
+  }
+  __syncthreads();
+  T A[4][2];
+#pragma unroll
+  for(int S = 1; S < 4; ++S)
+#pragma unroll
+    for(int a = 0; a < 2; ++a) A[S][a] = A_[cs][S][a];
+
+  T acc[2][NP];
+#pragma unroll
+  for(int j = 0; j < NP; ++j) acc[0][j] = acc[1][j] = 0;
+  // ---------------- cell term
+  {
+    const T c0[2] = {A[1][0] + p0 * A[3][0], A[1][1] + p0 * A[3][1]};
+#pragma unroll
+    for(int i = 0; i < NP; ++i)
+    {
+      T v = 0, g = 0, r0[NP], r1[NP];
+#pragma unroll
+      for(int j = 0; j < NP; ++j)
+      {
+        v += tab.V[i * NP + j] * u[j];
+        g += tab.Dv[i * NP + j] * u[j];
+      }
+      lane_gather<NP, 0>(g, ra, r0);
+      lane_gather<NP, 0>(v, ra, r1);
+      const T g0 = dotn<NP>(Va, r0), g1 = dotn<NP>(Da, r1);
+      const T c1[2] = {A[2][0] + tab.qx[i] * A[3][0], A[2][1] + tab.qx[i] * A[3][1]};
+      const T det = c0[0] * c1[1] - c0[1] * c1[0];
+      const T w = wq * tab.qw[i] * fast_recip(fabs(det));
+      const T h0 = w * (c1[1] * g0 - c0[1] * g1), h1 = w * (c0[0] * g1 - c1[0] * g0);
+      lane_gather<NP, 0>(c1[1] * h0 - c1[0] * h1, ra, r0);
+      lane_gather<NP, 0>(c0[0] * h1 - c0[1] * h0, ra, r1);
+      const T a0 = dotn<NP>(VaT, r0), a1 = dotn<NP>(DaT, r1);
+#pragma unroll
+      for(int j = 0; j < NP; ++j) acc[0][j] += tab.Dv[i * NP + j] * a0 + tab.V[i * NP + j] * a1;
+    }
+  }
+  // ---------------- faces
+  const int lane0 = min(cs, CPB - 1) * NP;  // the lane of the cell's first face point
+#pragma unroll
+  for(int d = 0; d < 2; ++d)
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const int f = 2 * d + side, bd = 1 << d, b1 = 2 >> d;
+      const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
+      T r0[NP], r1[NP], m[NP], go[2], gn[2];
+      lane_gather<NP, 0>(vo[d][side], ra, r0);
+      lane_gather<NP, 0>(vn[d][side], ra, r1);
+#pragma unroll
+      for(int r = 0; r < NP; ++r) m[r] = r0[r] - r1[r];
+      const T jump = dotn<NP>(Va, m);
+      go[1] = dotn<NP>(Da, r0);
+      gn[1] = dotn<NP>(Da, r1);
+      lane_gather<NP, 0>(go_[d][side], ra, r0);
+      lane_gather<NP, 0>(gn_[d][side], ra, r1);
+      go[0] = dotn<NP>(Va, r0);
+      gn[0] = dotn<NP>(Va, r1);
+      T t1[2], jd[2], jn[2];
+#pragma unroll
+      for(int a = 0; a < 2; ++a)
+      {
+        t1[a] = side ? A[b1][a] + A[3][a] : A[b1][a];
+        jd[a] = A[bd][a] + p0 * A[3][a];
+        jn[a] = N_[cs][f][0][a] + p0 * N_[cs][f][1][a];
+      }
+      const T ww = t1[0] * t1[0] + t1[1] * t1[1];
+      const T wo = t1[1] * jd[0] - t1[0] * jd[1], wn = t1[1] * jn[0] - t1[0] * jn[1];
+      // outward: the normal derivative grows along J_d on side 1, against it on side 0
+      const T sg = (wo > T(0)) == (side == 1) ? T(1) : T(-1);
+      const T io = sg * fast_recip(wo), in_ = sg * fast_recip(wn);
+      const T nw = root(ww);
+      const T ko[2] = {io * ww, -io * (t1[0] * jd[0] + t1[1] * jd[1])};
+      const T kn[2] = {in_ * ww, -in_ * (t1[0] * jn[0] + t1[1] * jn[1])};
+      // penalty: inverse lengths |(J^{-1} n)_d| at the first face point of both cells
+      // (apps/laplace_integrator.h:651-656, 692-693)
+      T sigma = nw * (in ? T(0.5) * (fabs(io) + fabs(in_)) : T(2) * fabs(io));
+      sigma = ipg * lane_read(sigma, lane0);
+      const T hf = (in ? T(0.5) : T(1)) * wq;
+      const T pa = sigma * (nw * wq) * jump -
+                   hf * (ko[0] * go[0] + ko[1] * go[1] + kn[0] * gn[0] + kn[1] * gn[1]);
+      const T hj = -hf * jump;
+      lane_gather<NP, 0>(pa, ra, r0);
+      lane_gather<NP, 0>(hj * ko[1], ra, r1);
+      const T pv = dotn<NP>(VaT, r0) + dotn<NP>(DaT, r1);
+      lane_gather<NP, 0>(hj * ko[0], ra, r0);
+      const T pd = dotn<NP>(VaT, r0);
+#pragma unroll
+      for(int j = 0; j < NP; ++j) acc[d][j] += tab.fd[side][j] * pd;
+      acc[d][side ? P : 0] += pv;
+    }
+#pragma unroll
+  for(int j = 0; j < NP; ++j) L1[cs][q + j * NP] = acc[1][j];
+  __syncthreads();
+  if(!act) return;
+  T out[NP];
+#pragma unroll
+  for(int j = 0; j < NP; ++j) out[j] = acc[0][j] + L1[cs][NP * q + j];
+  if(RESIDUAL)
+  {
+    T bv[NP];
+    load_row<NP>(b + cell * NDC + NP * q, bv);
+#pragma unroll
+    for(int j = 0; j < NP; ++j) out[j] = bv[j] - out[j];
+  }
+  store_row<NP>(y + cell * NDC + NP * q, out);
 }
 
 }  // namespace tpss
