@@ -453,3 +453,39 @@ def test_gmg_iterative_coarse_solve():
     xr, itr, histr = ref.cg(b, rel_tol=1e-8)
     assert info.iterations == itr
     assert rel_err(host(x), xr) < 1e-7
+
+
+# vmult starts from zero whatever dst holds: even and odd cell counts, sequences that
+# do and do not begin with the two colors of a chessboard, damped and undamped
+@pytest.mark.parametrize("dim,p,n,kw", [
+    (2, 3, 8, {}), (2, 3, 7, {}), (2, 2, 6, dict(relaxation=0.7)), (2, 3, 8, dict(reverse=True)),
+    (3, 3, 4, {}), (3, 3, 5, {}), (3, 3, 4, dict(symmetrized=True)), (3, 3, 2, dict(relaxation=0.8)),
+    (3, 2, 4, dict(relaxation=0.6)), (3, 4, 4, {}), (3, 3, 18, dict(relaxation=0.9)),
+    (2, 2, 6, dict(damping=0.8)), (2, 3, 6, dict(n_steps=2)), (3, 2, 4, dict(damping=0.8, n_steps=2))])
+@pytest.mark.parametrize("distorted", [False, True])
+def test_vmult_ignores_the_contents_of_dst(dim, p, n, kw, distorted):
+    if distorted and n > 8:
+        pytest.skip("the fine-level passes run on Cartesian levels")
+    V = o.distorted_vertices(dim, n, 0.1, seed=3) if distorted else None
+    lv, sm, ref = make(dim, p, n, 1, ip=2.0, vertices=V, **kw)
+    src = o.splitmix_uniform(4, ref.N)
+    for _ in range(2):
+        d = dev(np.full(ref.N, np.nan))
+        sm.vmult(d, dev(src))
+        assert rel_err(host(d), ref.smoother_vmult(src)) < 1e-12
+        sm.finite_status()
+    d = dev(np.full(ref.N, np.nan))
+    sm.precond_vmult(d, dev(src))
+    assert rel_err(host(d), ref.precond_vmult(src)) < 1e-12
+
+
+@pytest.mark.parametrize("n", [6, 7])
+def test_vmult_ignores_the_contents_of_dst_with_patch_damping(n):
+    lv, sm, ref = make(3, 3, n, 1)
+    omega = 0.8 + 0.4 * np.abs(o.splitmix_uniform(9, ref.P))
+    sm.set_patch_damping(omega)
+    ref.set_patch_damping(omega)
+    src = o.splitmix_uniform(4, ref.N)
+    d = dev(np.full(ref.N, np.nan))
+    sm.vmult(d, dev(src))
+    assert rel_err(host(d), ref.smoother_vmult(src)) < 1e-6  # omega is kept in FP32

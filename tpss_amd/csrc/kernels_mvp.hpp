@@ -21,6 +21,10 @@
 
 namespace tpss
 {
+// what a color pass may take as zero without reading it (x_zero): the cells outside
+// its patches, the patches' own cells
+constexpr int kOuterZero = 1, kOwnZero = 2;
+
 typedef short tpss_bf16x4 __attribute__((__vector_size__(4 * sizeof(short))));
 typedef float tpss_floatx4 __attribute__((__vector_size__(4 * sizeof(float))));
 
@@ -126,7 +130,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
                   const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
                   const uint32_t *__restrict__ eo_tab, const float *__restrict__ omega,
                   const CT relaxation, const int patch_begin,
-                  const int patch_end, const int n, const int x_is_zero,
+                  const int patch_end, const int n, const int x_zero,
                   int *__restrict__ nonfinite)
 {
   using PS = PatchShape<DIM, K>;
@@ -248,7 +252,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
 #pragma unroll
     for(int i = 0; i < K; ++i) g[i] = CT(0);
 
-  if(!x_is_zero)
+  if(!(x_zero & kOuterZero))
   {
     // z_0: x-neighbours of the two x-cells of this line
     CT z0[K], t1[K], t2[K];
@@ -535,7 +539,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   }
   // the factor tables in LDS are complete (without the coupling stage no
   // barrier has passed since they were written)
-  else if(x_is_zero)
+  else if(x_zero & kOuterZero)
     __syncthreads();
   if constexpr(FD == 1)
   {
@@ -585,7 +589,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
                                      ls[plc][DIM > 2 ? 2 : 1], w, t, owner);
   }
   if(!valid) return;
-  if(!x_is_zero && w != CT(1))
+  if(!(x_zero & kOwnZero) && w != CT(1))
   {
     CT old[K];
     load_row<NP>(x + c_lo * NDC + lyz, old);

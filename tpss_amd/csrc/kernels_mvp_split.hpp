@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
+#include "kernels_mvp.hpp"
 
 namespace tpss
 {
@@ -69,7 +70,7 @@ k_patch_mvp_split(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
                   const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
                   const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
                   const float *__restrict__ omega, const CT relaxation, const int patch_begin,
-                  const int n, const int x_is_zero, int *__restrict__ nonfinite)
+                  const int n, const int x_zero, int *__restrict__ nonfinite)
 {
   constexpr int K = 8, NP = 4, NDC = 64;
   constexpr int SY = 8, SZ = 72;     // solve buffer (x, y, z) -> x + SY y + SZ z
@@ -109,7 +110,7 @@ k_patch_mvp_split(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   load_pair(b + cell * NDC + lyz + lx0, g);
 
   CT z0[2] = {CT(0), CT(0)}, t1[2] = {CT(0), CT(0)}, t2[2] = {CT(0), CT(0)};
-  if(!x_is_zero)
+  if(!(x_zero & kOuterZero))
   {
     // z_0: the x-neighbour of this thread's x-cell (left of cell 0, right of cell 1)
     const bool hx = cx == 0 ? (v[0] - 1 > 0) : (v[0] + 1 < n);
@@ -185,7 +186,7 @@ k_patch_mvp_split(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   if(t < 3 * K) (&ls[0][0])[t] = lv;
   const CT w = omega ? CT(omega[j]) : relaxation;
 
-  if(!x_is_zero)
+  if(!(x_zero & kOuterZero))
   {
     // cross-line mass contractions:  g -= M_y M_x z_2 + M_z (M_x z_1 + M_y z_0)
     CT *Z = A1;
@@ -231,7 +232,7 @@ k_patch_mvp_split(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   CT *B = A2;
   CT rr[K];
   CT o[2];
-  if(x_is_zero) __syncthreads();  // publishes Ss / ls (else the coupling's barriers do)
+  if(x_zero & kOuterZero) __syncthreads();  // publishes Ss / ls (else the coupling's barriers do)
   // forward x: the x-line (ty, tz), gathered from the quad
   quad_gather(g, rr);
 #pragma unroll
@@ -313,7 +314,7 @@ k_patch_mvp_split(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
     o[k] = s;
   }
   VT *px = x + cell * NDC + lyz + lx0;
-  if(!x_is_zero && w != CT(1))
+  if(!(x_zero & kOwnZero) && w != CT(1))
   {
     CT old[2];
     load_pair(px, old);

@@ -131,7 +131,7 @@ struct PassCheck
   ~PassCheck() { sm->pass_flag = nullptr; }
 };
 void smoother_step_any(tpss_smoother *sm, void *dst, const void *src, hipStream_t s,
-                       bool x_is_zero = false);
+                       bool from_zero = false);
 template<typename VT>
 void precond_vmult_bf16(tpss_smoother *sm, VT *dst, const VT *src, hipStream_t s, bool accumulate,
                         double alpha, const std::vector<int> &seq);
