@@ -460,7 +460,7 @@ def test_gmg_iterative_coarse_solve():
 @pytest.mark.parametrize("dim,p,n,kw", [
     (2, 3, 8, {}), (2, 3, 7, {}), (2, 2, 6, dict(relaxation=0.7)), (2, 3, 8, dict(reverse=True)),
     (3, 3, 4, {}), (3, 3, 5, {}), (3, 3, 4, dict(symmetrized=True)), (3, 3, 2, dict(relaxation=0.8)),
-    (3, 2, 4, dict(relaxation=0.6)), (3, 4, 4, {}), (3, 3, 18, dict(relaxation=0.9)),
+    (3, 2, 4, dict(relaxation=0.6)), (3, 4, 4, {}), (3, 3, 22, dict(relaxation=0.9)),
     (2, 2, 6, dict(damping=0.8)), (2, 3, 6, dict(n_steps=2)), (3, 2, 4, dict(damping=0.8, n_steps=2))])
 @pytest.mark.parametrize("distorted", [False, True])
 def test_vmult_ignores_the_contents_of_dst(dim, p, n, kw, distorted):
@@ -479,7 +479,8 @@ def test_vmult_ignores_the_contents_of_dst(dim, p, n, kw, distorted):
     assert rel_err(host(d), ref.precond_vmult(src)) < 1e-12
 
 
-@pytest.mark.parametrize("n", [6, 7])
+# 22^3: more than 512 patches per color, the fine-level color pass
+@pytest.mark.parametrize("n", [6, 7, 22])
 def test_vmult_ignores_the_contents_of_dst_with_patch_damping(n):
     lv, sm, ref = make(3, 3, n, 1)
     omega = 0.8 + 0.4 * np.abs(o.splitmix_uniform(9, ref.P))

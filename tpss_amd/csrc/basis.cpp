@@ -159,6 +159,9 @@ Operator1D make_operator_1d(int p, double h, double ip)
   std::memset(&op, 0, sizeof(op));
   const double sig_i = ip * 0.5 * nitsche_penalty(p, h, h);
   const double sig_b = ip * nitsche_penalty(p, h, h);
+  op.sigma = sig_i;
+  for(int f = 0; f < 2; ++f)
+    for(int i = 0; i < np; ++i) op.g[f][i] = b.fgrad[i * 2 + f] / h;
   double K[MAXNP * MAXNP], Fmm[MAXNP * MAXNP], Fpp[MAXNP * MAXNP], Bl[MAXNP * MAXNP],
     Br[MAXNP * MAXNP];
   for(int i = 0; i < np; ++i)

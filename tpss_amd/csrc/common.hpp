@@ -144,6 +144,8 @@ struct Operator1D
   double D[4][MAXNP * MAXNP];   // K + left-face + right-face; index = has_left | has_right<<1
   double Fpm[MAXNP * MAXNP];    // coupling to the left neighbour
   double Fmp[MAXNP * MAXNP];    // coupling to the right neighbour
+  double g[2][MAXNP];           // phi_i'(0) / h, phi_i'(1) / h
+  double sigma;                 // penalty of an interior face
 };
 Operator1D make_operator_1d(int p, double h, double ip);
 

@@ -148,6 +148,50 @@ __device__ __forceinline__ CT lane_read(CT v, int lane)
   }
 }
 
+// value of lane (q + r) mod NP along the first (AX = 0) or second (AX = 1) lane
+// index of a cell whose NP^2 (2D: NP) nodes are consecutive lanes; addr: byte address of that lane for ds_bpermute (NP != 4)
+template<int NP, int AX, int R, typename T>
+__device__ __forceinline__ T lane_rot(T v, const int *addr)
+{
+  if constexpr(R == 0)
+    return v;
+  else if constexpr(NP == 4)
+  {
+    // quad_perm (i + R) mod 4; row_ror by 16 - 4 R
+    constexpr int CTRL = AX == 0 ? ((R & 3) | (((1 + R) & 3) << 2) | (((2 + R) & 3) << 4) | (((3 + R) & 3) << 6))
+                                 : 0x120 + 16 - 4 * R;
+    if constexpr(sizeof(T) == 4)
+      return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+    else
+      return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true),
+                              __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true));
+  }
+  else if constexpr(sizeof(T) == 4)
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr[R], __float_as_int(v)));
+  else
+    return __hiloint2double(__builtin_amdgcn_ds_bpermute(addr[R], __double2hiint(v)),
+                            __builtin_amdgcn_ds_bpermute(addr[R], __double2loint(v)));
+}
+
+template<int NP, int AX, typename T>
+__device__ __forceinline__ void lane_gather(T v, const int *addr, T *o)
+{
+  o[0] = v;
+  o[1] = lane_rot<NP, AX, 1>(v, addr);
+  if constexpr(NP > 2) o[2] = lane_rot<NP, AX, 2>(v, addr);
+  if constexpr(NP > 3) o[3] = lane_rot<NP, AX, 3>(v, addr);
+  if constexpr(NP > 4) o[4] = lane_rot<NP, AX, 4>(v, addr);
+}
+
+template<int NP, typename T>
+__device__ __forceinline__ T dotn(const T *a, const T *b)
+{
+  T s = 0;
+#pragma unroll
+  for(int r = 0; r < NP; ++r) s += a[r] * b[r];
+  return s;
+}
+
 template<int DIM, int NP, typename VT, typename CT, int CPB, bool RESIDUAL>
 __global__ void __launch_bounds__(256)
 k_sipg_cartesian(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
@@ -881,8 +925,8 @@ __device__ __forceinline__ CT eig_scale(CT s, CT w, CT lam)
 // face), so each product takes two (K/2 x K/2) blocks of S on the folded line
 // r_a +- r_{K-1-a}: half the multiply-adds.  (A compile-time choice: a
 // run-time one keeps the line arrays out of registers.)
-template<int K, bool EVEN_ODD, typename CT>
-__device__ __forceinline__ void s_forward(const CT *S, const CT *r, CT *o)
+template<int K, bool EVEN_ODD, typename SP, typename CT>
+__device__ __forceinline__ void s_forward(const SP S, const CT *r, CT *o)
 {
   constexpr int P = K / 2;
   if constexpr(EVEN_ODD)
@@ -921,8 +965,8 @@ __device__ __forceinline__ void s_forward(const CT *S, const CT *r, CT *o)
   }
 }
 
-template<int K, bool EVEN_ODD, typename CT>
-__device__ __forceinline__ void s_backward(const CT *S, const CT *o, CT *r)
+template<int K, bool EVEN_ODD, typename SP, typename CT>
+__device__ __forceinline__ void s_backward(const SP S, const CT *o, CT *r)
 {
   constexpr int P = K / 2;
   if constexpr(EVEN_ODD)
@@ -954,6 +998,20 @@ __device__ __forceinline__ void s_backward(const CT *S, const CT *o, CT *r)
   }
 }
 
+// A wave-uniform matrix in read-only global memory as an operand of scalar loads at
+// the point of use.  The pointer is opaque to the compiler: without that it loads the
+// matrices of all stages at once, which exceeds the scalar registers (in the FP64
+// solve 440 of 1300 VALU instructions saved and restored them).
+template<typename CT>
+using scalar_ptr = const __attribute__((address_space(4))) CT *;
+template<typename CT>
+__device__ __forceinline__ scalar_ptr<CT> scalar_rows(const CT *p)
+{
+  scalar_ptr<CT> q = (scalar_ptr<CT>)p;
+  asm volatile("" : "+s"(q));
+  return q;
+}
+
 // Fast-diagonalization inverse of one patch held as x-lines: thread t owns the
 // x-line (y, z) = (t % K, t / K); on entry r is that line of the patch
 // right-hand side, on exit o is the same line of
@@ -961,15 +1019,22 @@ __device__ __forceinline__ void s_backward(const CT *S, const CT *o, CT *r)
 // The line direction rotates x -> y -> z -> y -> x through the patch's LDS
 // buffer B (entry (x, y, z) at x + SY y + SZ z: padded strides keep the
 // transposes free of LDS bank conflicts); EO: even-odd products in every
-// direction.  Contains __syncthreads (every thread of the block must call it).
-template<int DIM, int K, typename CT, int SY = K, int SZ = K * K, bool EO = false>
+// direction; SCALAR: the matrices are wave-uniform in global memory (scalar_rows).
+// Contains __syncthreads (every thread of the block must call it).
+template<int DIM, int K, typename CT, int SY = K, int SZ = K * K, bool EO = false, bool SCALAR = false>
 __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, const CT *S1,
                                          const CT *S2, const CT *l0, const CT *l1, const CT *l2,
                                          const CT w, const int t, const bool owner)
 {
   const int ty = DIM > 1 ? t % K : 0;
   const int tz = DIM > 2 ? t / K : 0;
-  s_forward<K, EO>(S0, r, o);
+  auto rows = [](const CT *S) {
+    if constexpr(SCALAR)
+      return scalar_rows(S);
+    else
+      return S;
+  };
+  s_forward<K, EO>(rows(S0), r, o);
   if(DIM == 2)
   {
 #pragma unroll
@@ -979,10 +1044,10 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
     const int x0 = t;
 #pragma unroll
     for(int jj = 0; jj < K; ++jj) r[jj] = B[x0 + SY * jj];
-    s_forward<K, EO>(S1, r, o);
+    s_forward<K, EO>(rows(S1), r, o);
 #pragma unroll
     for(int jj = 0; jj < K; ++jj) o[jj] = eig_scale(o[jj], w, l0[x0] + l1[jj]);
-    s_backward<K, EO>(S1, o, r);
+    s_backward<K, EO>(rows(S1), o, r);
     __syncthreads();
 #pragma unroll
     for(int b = 0; b < K; ++b)
@@ -1001,7 +1066,7 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
       const int x0 = t % K, z0 = t / K;
 #pragma unroll
       for(int jj = 0; jj < K; ++jj) r[jj] = B[x0 + SY * jj + SZ * z0];
-      s_forward<K, EO>(S1, r, o);
+      s_forward<K, EO>(rows(S1), r, o);
 #pragma unroll
       for(int jj = 0; jj < K; ++jj)
         if(owner) B[x0 + SY * jj + SZ * z0] = o[jj];
@@ -1012,10 +1077,11 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
 #pragma unroll
       for(int l = 0; l < K; ++l) r[l] = B[x0 + SY * y0 + SZ * l];
       const CT lxy = l0[x0] + l1[y0];
-      s_forward<K, EO>(S2, r, o);
+      const auto R2 = rows(S2);
+      s_forward<K, EO>(R2, r, o);
 #pragma unroll
       for(int l = 0; l < K; ++l) o[l] = eig_scale(o[l], w, lxy + l2[l]);
-      s_backward<K, EO>(S2, o, r);
+      s_backward<K, EO>(R2, o, r);
 #pragma unroll
       for(int c = 0; c < K; ++c)
         if(owner) B[x0 + SY * y0 + SZ * c] = r[c];
@@ -1025,7 +1091,7 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
       const int x0 = t % K, z0 = t / K;
 #pragma unroll
       for(int jj = 0; jj < K; ++jj) r[jj] = B[x0 + SY * jj + SZ * z0];
-      s_backward<K, EO>(S1, r, o);
+      s_backward<K, EO>(rows(S1), r, o);
 #pragma unroll
       for(int b = 0; b < K; ++b)
         if(owner) B[x0 + SY * b + SZ * z0] = o[b];
@@ -1034,7 +1100,7 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
 #pragma unroll
     for(int i = 0; i < K; ++i) r[i] = B[i + SY * ty + SZ * tz];
   }
-  s_backward<K, EO>(S0, r, o);
+  s_backward<K, EO>(rows(S0), r, o);
 }
 
 template<int DIM, int K, typename VT, typename CT, int MODE>

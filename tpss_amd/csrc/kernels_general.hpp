@@ -69,50 +69,6 @@ constexpr int moved_cells_per_block()
   return 64 / cpow(NP, DIM - 1);
 }
 
-// value of lane (q + r) mod NP along the first (AX = 0) or second (AX = 1) lane
-// index of the cell; addr: byte address of that lane for ds_bpermute (NP != 4)
-template<int NP, int AX, int R, typename T>
-__device__ __forceinline__ T lane_rot(T v, const int *addr)
-{
-  if constexpr(R == 0)
-    return v;
-  else if constexpr(NP == 4)
-  {
-    // quad_perm (i + R) mod 4; row_ror by 16 - 4 R
-    constexpr int CTRL = AX == 0 ? ((R & 3) | (((1 + R) & 3) << 2) | (((2 + R) & 3) << 4) | (((3 + R) & 3) << 6))
-                                 : 0x120 + 16 - 4 * R;
-    if constexpr(sizeof(T) == 4)
-      return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
-    else
-      return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true),
-                              __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true));
-  }
-  else if constexpr(sizeof(T) == 4)
-    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr[R], __float_as_int(v)));
-  else
-    return __hiloint2double(__builtin_amdgcn_ds_bpermute(addr[R], __double2hiint(v)),
-                            __builtin_amdgcn_ds_bpermute(addr[R], __double2loint(v)));
-}
-
-template<int NP, int AX, typename T>
-__device__ __forceinline__ void lane_gather(T v, const int *addr, T *o)
-{
-  o[0] = v;
-  o[1] = lane_rot<NP, AX, 1>(v, addr);
-  if constexpr(NP > 2) o[2] = lane_rot<NP, AX, 2>(v, addr);
-  if constexpr(NP > 3) o[3] = lane_rot<NP, AX, 3>(v, addr);
-  if constexpr(NP > 4) o[4] = lane_rot<NP, AX, 4>(v, addr);
-}
-
-template<int NP, typename T>
-__device__ __forceinline__ T dotn(const T *a, const T *b)
-{
-  T s = 0;
-#pragma unroll
-  for(int r = 0; r < NP; ++r) s += a[r] * b[r];
-  return s;
-}
-
 // 1/a: the hardware reciprocal, in FP64 refined by two Newton steps (within an ulp
 // or two of the correctly rounded quotient)
 __device__ __forceinline__ float fast_recip(float a) { return __builtin_amdgcn_rcpf(a); }

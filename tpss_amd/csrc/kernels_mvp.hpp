@@ -99,55 +99,30 @@ __device__ __forceinline__ void fd_mfma_pair(float (*B2)[512], const float (*S)[
 
 // FD = 0: vector FMA contractions in CT; FD = 1: BF16 MFMA contractions with
 // FP32 accumulation (3D, K = 8, CT = float)
-// Waves per SIMD the register allocation must allow.  Up to K = 8: FP32 patch
-// solves 5 (<= 96 VGPRs) so that more patches keep their loads in flight while
-// others compute; longer lines (K = 10) hold more values per thread: 3.  FP64
-// solves unconstrained (3D K = 8: 186 VGPRs, 2 waves; forcing 3 spills and
-// measured 20 % slower).
-
+// Waves per SIMD the register allocation must allow: FP32 patch solves 5 (<= 96
+// VGPRs) up to K = 8; longer lines (K = 10) hold more values per thread: 3; FP64
+// solves unconstrained.
 template<int K, typename CT, int FD>
 constexpr int mvp_min_waves()
 {
   return FD == 1 || !std::is_same<CT, float>::value ? 1 : K <= 8 ? 5 : 3;
 }
 
-// Launch shape of the fused pass: one patch per block where a patch fills a
-// wave (3D, K = 8, vector solves), so that the block is a single wave, its
-// barriers cost nothing and no patch waits for another; otherwise the shape of
-// the other patch kernels (the BF16-MFMA solve pairs two patches per block).
-template<int DIM, int K, int FD>
-struct MvpShape
-{
-  using PS = PatchShape<DIM, K>;
-  static constexpr int PPB = (FD == 0 && PS::L == 64) ? 1 : PS::PPB;
-  static constexpr int THREADS = ((PPB * PS::L + 63) / 64) * 64;
-};
-
 template<int DIM, int K, typename VT, typename CT, int FD = 0>
-__global__ void __launch_bounds__((MvpShape<DIM, K, FD>::THREADS), (mvp_min_waves<K, CT, FD>()))
+__global__ void __launch_bounds__((PatchShape<DIM, K>::THREADS), (mvp_min_waves<K, CT, FD>()))
 k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, K / 2> tab,
                   const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
                   const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
-                  const uint32_t *__restrict__ eo_tab, const float *__restrict__ omega,
-                  const CT relaxation, const int patch_begin,
+                  const float *__restrict__ omega, const CT relaxation, const int patch_begin,
                   const int patch_end, const int n, const int x_zero,
                   int *__restrict__ nonfinite)
 {
   using PS = PatchShape<DIM, K>;
-  using MS = MvpShape<DIM, K, FD>;
-  constexpr int NP = PS::NP, L = PS::L, NPD = PS::NPD, NDC = PS::NDC, PPB = MS::PPB;
-  // LDS strides (y, z) of the patch buffers, padded for 3D K = 8 so that the
-  // line transposes of the solve (FSY, FSZ) and the cross-line reads of the
-  // coupling stage (CSY, CSZ) are free of bank conflicts.  The padded solve
-  // buffer reuses the coupling buffer A2, whose last read precedes a barrier
-  // that every thread passes before the solve writes.
-  constexpr bool PAD = FD == 0 && DIM == 3 && K == 8;
-  constexpr int FSY = K, FSZ = PAD ? 72 : K * K;
-  constexpr int CSY = PAD ? 12 : K, CSZ = PAD ? 96 : K * K;
-  static_assert(!PAD || K * FSZ <= K * CSZ, "solve buffer must fit in the coupling buffer");
-  __shared__ CT buf[PPB][PAD ? 1 : NPD];
-  __shared__ CT A1[PPB][DIM > 2 ? K * CSZ : NPD];
-  __shared__ CT A2[PPB][DIM > 2 ? K * CSZ : 1];
+  constexpr int NP = PS::NP, L = PS::L, NPD = PS::NPD, NDC = PS::NDC, PPB = PS::PPB;
+  constexpr int SY = K, SZ = K * K;  // strides (y, z) of the patch buffers
+  __shared__ CT buf[PPB][NPD];
+  __shared__ CT A1[PPB][NPD];
+  __shared__ CT A2[PPB][DIM > 2 ? NPD : 1];
   __shared__ CT Ss[PPB][DIM][K * K];
   __shared__ CT ls[PPB][DIM][K];
 
@@ -158,68 +133,23 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   const int plc = pl < PPB ? pl : 0;
   const bool owner = pl < PPB;
 
-  // FP32 solves with one patch per wave (3D, K = 8): the eigenvector matrices
-  // of the wave's patch are read with wave-uniform addresses straight into
-  // scalar registers (operands of the contraction FMAs) instead of being
-  // staged through LDS, which takes most LDS reads off the pass.  (FP64
-  // matrices would need twice the scalar registers and spill.)
-  constexpr bool WAVE_PATCH = FD == 0 && L == 64 && MS::THREADS == PPB * 64;
-  constexpr bool S_SCALAR = WAVE_PATCH && std::is_same<CT, float>::value;
-  // One patch per wave, 3D, K = 8 (the fine levels): every global load of the
-  // pass is issued in two batches -- the patch's vertex and factor rows, then
-  // its factor tables, b and the outer neighbour rows -- before the first wait,
-  // so that a wave waits for two memory round trips, not for one per table and
-  // neighbour.  Each lane loads one row of the y- and z-neighbour planes and
-  // takes the other three rows of a plane from the lanes that loaded them: the
-  // lanes sharing a y-plane form a quad (DPP), those sharing a z-plane sit 8
-  // lanes apart (their rows pass through LDS: 4 writes and 16 reads of 16 bytes
-  // per lane instead of 64 ds_bpermute).  The patch tables are staged
-  // unconditionally (the full matrices are unused by the even-odd products).
-  constexpr bool BATCH = WAVE_PATCH && DIM == 3 && K == 8 && !std::is_same<CT, float>::value;
+  for(int idx = threadIdx.x; idx < PPB * DIM * K * K; idx += blockDim.x)
+  {
+    const int q = idx / (DIM * K * K), r = idx % (DIM * K * K);
+    const int d = r / (K * K), e = r % (K * K);
+    const int jj = j0 + q;
+    Ss[q][d][e] = jj < patch_end ? S_tab[size_t(fac[size_t(jj) * DIM + d]) * K * K + e] : CT(0);
+  }
+  for(int idx = threadIdx.x; idx < PPB * DIM * K; idx += blockDim.x)
+  {
+    const int q = idx / (DIM * K), r = idx % (DIM * K);
+    const int d = r / K, e = r % K;
+    const int jj = j0 + q;
+    ls[q][d][e] = jj < patch_end ? lam_tab[size_t(fac[size_t(jj) * DIM + d]) * K + e] : CT(1);
+  }
   int v[3] = {1, 1, 1};
-  uint32_t fw[3] = {0, 0, 0};  // factor rows of the wave's patch (BATCH)
-  CT w;
-  if constexpr(BATCH)
-  {
-    // a starting wave issues its loads ahead of the other wave's arithmetic on
-    // the SIMD (raised priority until the last load of the batch is issued)
-    __builtin_amdgcn_s_setprio(3);
-    const int jw = min(j0, patch_end - 1);  // wave-uniform
-    const uint32_t pv = vtx[jw];
-#pragma unroll
-    for(int d = 0; d < 3; ++d) fw[d] = fac[size_t(jw) * 3 + d];
-    unpack_vertex(pv, v);
-  }
-  else
-  {
-    // one wave per patch with the matrices not in scalar registers (FP64): the
-    // even-odd products take the half matrices straight from scalar loads, so
-    // only patches without mirror symmetry stage the full matrices in LDS
-    bool stage_S = true;
-    if constexpr(WAVE_PATCH && !S_SCALAR)
-    {
-      const int jw = min(j0, patch_end - 1);
-      stage_S = !(eo_tab && (eo_tab[fac[size_t(jw) * DIM]] & eo_tab[fac[size_t(jw) * DIM + 1]] &
-                             eo_tab[fac[size_t(jw) * DIM + 2]]) != 0u);
-    }
-    if constexpr(!S_SCALAR)
-      for(int idx = threadIdx.x; stage_S && idx < PPB * DIM * K * K; idx += blockDim.x)
-      {
-        const int q = idx / (DIM * K * K), r = idx % (DIM * K * K);
-        const int d = r / (K * K), e = r % (K * K);
-        const int jj = j0 + q;
-        Ss[q][d][e] = jj < patch_end ? S_tab[size_t(fac[size_t(jj) * DIM + d]) * K * K + e] : CT(0);
-      }
-    for(int idx = threadIdx.x; idx < PPB * DIM * K; idx += blockDim.x)
-    {
-      const int q = idx / (DIM * K), r = idx % (DIM * K);
-      const int d = r / K, e = r % K;
-      const int jj = j0 + q;
-      ls[q][d][e] = jj < patch_end ? lam_tab[size_t(fac[size_t(jj) * DIM + d]) * K + e] : CT(1);
-    }
-    if(valid) unpack_vertex(vtx[j], v);
-    w = valid ? (omega ? CT(omega[j]) : relaxation) : CT(0);
-  }
+  if(valid) unpack_vertex(vtx[j], v);
+  const CT w = valid ? (omega ? CT(omega[j]) : relaxation) : CT(0);
 
   const int ty = DIM > 1 ? t % K : 0;
   const int tz = DIM > 2 ? t / K : 0;
@@ -231,19 +161,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   const int64_t c_lo = patch_cell<DIM, NP>(v, n, 0, ty, tz);
   const int lyz = patch_local<DIM, NP>(0, ty, tz);
   CT g[K], r[K], o[K];
-  // BATCH: this lane's entries of the patch tables, staged in LDS after the
-  // coupling stage (their loads go out with those of b and the neighbours)
-  CT sv[3], lv = CT(1);
-  if constexpr(BATCH)
-  {
-    if constexpr(!S_SCALAR)
-#pragma unroll
-      for(int d = 0; d < 3; ++d) sv[d] = S_tab[size_t(fw[d]) * K * K + t];
-    if(t < 3 * K) lv = lam_tab[size_t(fw[t / K]) * K + t % K];
-    load_row<NP>(b + c_lo * NDC + lyz, g);
-    load_row<NP>(b + (c_lo + 1) * NDC + lyz, g + NP);
-  }
-  else if(valid)
+  if(valid)
   {
     load_row<NP>(b + c_lo * NDC + lyz, g);
     load_row<NP>(b + (c_lo + 1) * NDC + lyz, g + NP);
@@ -263,57 +181,48 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
       t1[i] = 0;
       t2[i] = 0;
     }
-    if constexpr(BATCH)
+    if(valid && v[0] - 1 > 0)
     {
-      // the outer neighbour rows of this lane: the x-neighbours of its line and
-      // one row of each of the two y- and z-neighbour planes; absent neighbours
-      // read the patch's own cells (in bounds) and are discarded below
-      const bool hl = v[0] - 1 > 0, hr = v[0] + 1 < n;
-      const bool hy = by == 0 ? (v[1] - 1 > 0) : (v[1] + 1 < n);
-      const bool hz = bz == 0 ? (v[2] - 1 > 0) : (v[2] + 1 < n);
-      CT xl[NP], xr[NP], ry[2][NP], rz[2][NP];
-      load_row<NP>(x + (hl ? c_lo - 1 : c_lo) * NDC + lyz, xl);
-      load_row<NP>(x + (hr ? c_lo + 2 : c_lo + 1) * NDC + lyz, xr);
-      const int64_t sy = hy ? (by == 0 ? -int64_t(n) : int64_t(n)) : 0;
-      const int64_t sz = hz ? (bz == 0 ? -nn : nn) : 0;
-#pragma unroll
-      for(int cx = 0; cx < 2; ++cx)
-      {
-        // y-plane lz, row ly; z-plane ly, row lz
-        load_row<NP>(x + (c_lo + cx + sy) * NDC + NP * NP * lz + NP * ly, ry[cx]);
-        load_row<NP>(x + (c_lo + cx + sz) * NDC + NP * ly + NP * NP * lz, rz[cx]);
-      }
-      __builtin_amdgcn_s_setprio(0);
-      // z_0 = F x_out along x, z_1 / z_2 = the y- / z-neighbour planes contracted
-      // along the face normal, from the rows loaded above.  The contractions run
-      // for absent neighbours too and are discarded by selection: a branch would
-      // let the compiler move the loads into it, behind the waits of the others.
-      const int lane0 = int(threadIdx.x) & ~(3 << 3);
+      CT xl[NP];
+      load_row<NP>(x + (c_lo - 1) * NDC + lyz, xl);
 #pragma unroll
       for(int i = 0; i < NP; ++i)
       {
-        CT s = 0, s2 = 0;
+        CT s = 0;
 #pragma unroll
-        for(int jj = 0; jj < NP; ++jj)
-        {
-          s += tab.Fpm[i * NP + jj] * xl[jj];
-          s2 += tab.Fmp[i * NP + jj] * xr[jj];
-        }
-        z0[i] = hl ? s : CT(0);
-        z0[NP + i] = hr ? s2 : CT(0);
+        for(int jj = 0; jj < NP; ++jj) s += tab.Fpm[i * NP + jj] * xl[jj];
+        z0[i] = s;
       }
+    }
+    if(valid && v[0] + 1 < n)
+    {
+      CT xr[NP];
+      load_row<NP>(x + (c_lo + 2) * NDC + lyz, xr);
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
       {
-        // the quad's four lanes (ly = 0..3) hold the four rows of the plane
-        const CT *F = by == 0 ? tab.Fpm : tab.Fmp;
+        CT s = 0;
+#pragma unroll
+        for(int jj = 0; jj < NP; ++jj) s += tab.Fmp[i * NP + jj] * xr[jj];
+        z0[NP + i] = s;
+      }
+    }
+    // z_1 (y-neighbour outside the patch) then t1 = M_x z_1 per x-cell
+    {
+      const bool has = by == 0 ? (v[1] - 1 > 0) : (v[1] + 1 < n);
+      const CT *F = by == 0 ? tab.Fpm : tab.Fmp;
+      if(valid && has)
+      {
+        const int64_t shift = by == 0 ? -int64_t(n) : int64_t(n);
         CT z1[K];
 #pragma unroll
         for(int cx = 0; cx < 2; ++cx)
         {
+          // the x-y plane lz of the neighbour cell: NP rows, contiguous
           CT xn[NP * NP];
+          const VT *pn = x + (c_lo + cx + shift) * NDC + NP * NP * lz;
 #pragma unroll
-          for(int jj = 0; jj < NP; ++jj)
-#pragma unroll
-            for(int lx = 0; lx < NP; ++lx) xn[lx + NP * jj] = quad_bcast_rt(ry[cx][lx], jj);
+          for(int jj = 0; jj < NP; ++jj) load_row<NP>(pn + NP * jj, xn + NP * jj);
 #pragma unroll
           for(int lx = 0; lx < NP; ++lx)
           {
@@ -331,28 +240,26 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
             CT s = 0;
 #pragma unroll
             for(int jj = 0; jj < NP; ++jj) s += tab.M[i * NP + jj] * z1[cx * NP + jj];
-            t1[cx * NP + i] = hy ? s : CT(0);
+            t1[cx * NP + i] = s;
           }
       }
+    }
+    if(DIM > 2)
+    {
+      const bool has = bz == 0 ? (v[2] - 1 > 0) : (v[2] + 1 < n);
+      const CT *F = bz == 0 ? tab.Fpm : tab.Fmp;
+      if(valid && has)
       {
-        // the lanes of line (ty, NP bz + kk), kk = 0..3, hold the rows kk: exchanged
-        // through LDS (A2 is free until the coupling stage writes T2 there)
-        const CT *F = bz == 0 ? tab.Fpm : tab.Fmp;
+        const int64_t shift = bz == 0 ? -nn : nn;
         CT z2[K];
-        CT *RZ = A2[0];
-#pragma unroll
-        for(int cx = 0; cx < 2; ++cx)
-#pragma unroll
-          for(int lx = 0; lx < NP; ++lx) RZ[(t * 2 + cx) * NP + lx] = rz[cx][lx];
-        __syncthreads();
 #pragma unroll
         for(int cx = 0; cx < 2; ++cx)
         {
+          // the x-z plane ly of the neighbour cell: NP rows at stride NP^2
           CT xn[NP * NP];
+          const VT *pn = x + (c_lo + cx + shift) * NDC + NP * ly;
 #pragma unroll
-          for(int kk = 0; kk < NP; ++kk)
-#pragma unroll
-            for(int lx = 0; lx < NP; ++lx) xn[lx + NP * kk] = RZ[((lane0 | (kk << 3)) * 2 + cx) * NP + lx];
+          for(int kk = 0; kk < NP; ++kk) load_row<NP>(pn + NP * NP * kk, xn + NP * kk);
 #pragma unroll
           for(int lx = 0; lx < NP; ++lx)
           {
@@ -370,114 +277,10 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
             CT s = 0;
 #pragma unroll
             for(int jj = 0; jj < NP; ++jj) s += tab.M[i * NP + jj] * z2[cx * NP + jj];
-            t2[cx * NP + i] = hz ? s : CT(0);
+            t2[cx * NP + i] = s;
           }
       }
     }
-    else
-    {
-      if(valid && v[0] - 1 > 0)
-      {
-        CT xl[NP];
-        load_row<NP>(x + (c_lo - 1) * NDC + lyz, xl);
-#pragma unroll
-        for(int i = 0; i < NP; ++i)
-        {
-          CT s = 0;
-#pragma unroll
-          for(int jj = 0; jj < NP; ++jj) s += tab.Fpm[i * NP + jj] * xl[jj];
-          z0[i] = s;
-        }
-      }
-      if(valid && v[0] + 1 < n)
-      {
-        CT xr[NP];
-        load_row<NP>(x + (c_lo + 2) * NDC + lyz, xr);
-#pragma unroll
-        for(int i = 0; i < NP; ++i)
-        {
-          CT s = 0;
-#pragma unroll
-          for(int jj = 0; jj < NP; ++jj) s += tab.Fmp[i * NP + jj] * xr[jj];
-          z0[NP + i] = s;
-        }
-      }
-      // z_1 (y-neighbour outside the patch) then t1 = M_x z_1 per x-cell
-      {
-        const bool has = by == 0 ? (v[1] - 1 > 0) : (v[1] + 1 < n);
-        const CT *F = by == 0 ? tab.Fpm : tab.Fmp;
-        if(valid && has)
-        {
-          const int64_t shift = by == 0 ? -int64_t(n) : int64_t(n);
-          CT z1[K];
-#pragma unroll
-          for(int cx = 0; cx < 2; ++cx)
-          {
-            // the x-y plane lz of the neighbour cell: NP rows, contiguous
-            CT xn[NP * NP];
-            const VT *pn = x + (c_lo + cx + shift) * NDC + NP * NP * lz;
-#pragma unroll
-            for(int jj = 0; jj < NP; ++jj) load_row<NP>(pn + NP * jj, xn + NP * jj);
-#pragma unroll
-            for(int lx = 0; lx < NP; ++lx)
-            {
-              CT s = 0;
-#pragma unroll
-              for(int jj = 0; jj < NP; ++jj) s += F[ly * NP + jj] * xn[lx + NP * jj];
-              z1[cx * NP + lx] = s;
-            }
-          }
-#pragma unroll
-          for(int cx = 0; cx < 2; ++cx)
-#pragma unroll
-            for(int i = 0; i < NP; ++i)
-            {
-              CT s = 0;
-#pragma unroll
-              for(int jj = 0; jj < NP; ++jj) s += tab.M[i * NP + jj] * z1[cx * NP + jj];
-              t1[cx * NP + i] = s;
-            }
-        }
-      }
-      if(DIM > 2)
-      {
-        const bool has = bz == 0 ? (v[2] - 1 > 0) : (v[2] + 1 < n);
-        const CT *F = bz == 0 ? tab.Fpm : tab.Fmp;
-        if(valid && has)
-        {
-          const int64_t shift = bz == 0 ? -nn : nn;
-          CT z2[K];
-#pragma unroll
-          for(int cx = 0; cx < 2; ++cx)
-          {
-            // the x-z plane ly of the neighbour cell: NP rows at stride NP^2
-            CT xn[NP * NP];
-            const VT *pn = x + (c_lo + cx + shift) * NDC + NP * ly;
-#pragma unroll
-            for(int kk = 0; kk < NP; ++kk) load_row<NP>(pn + NP * NP * kk, xn + NP * kk);
-#pragma unroll
-            for(int lx = 0; lx < NP; ++lx)
-            {
-              CT s = 0;
-#pragma unroll
-              for(int kk = 0; kk < NP; ++kk) s += F[lz * NP + kk] * xn[lx + NP * kk];
-              z2[cx * NP + lx] = s;
-            }
-          }
-#pragma unroll
-          for(int cx = 0; cx < 2; ++cx)
-#pragma unroll
-            for(int i = 0; i < NP; ++i)
-            {
-              CT s = 0;
-#pragma unroll
-              for(int jj = 0; jj < NP; ++jj) s += tab.M[i * NP + jj] * z2[cx * NP + jj];
-              t2[cx * NP + i] = s;
-            }
-        }
-      }
-    }
-    if constexpr(BATCH) __syncthreads();  // the z-plane rows in A2 are read
     // cross-line mass contractions through LDS
     CT *Z = A1[plc];
     CT *T2 = A2[plc];
@@ -485,8 +288,8 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
     for(int i = 0; i < K; ++i)
       if(owner)
       {
-        Z[i + CSY * ty + CSZ * tz] = z0[i];
-        if(DIM > 2) T2[i + CSY * ty + CSZ * tz] = t2[i];
+        Z[i + SY * ty + SZ * tz] = z0[i];
+        if(DIM > 2) T2[i + SY * ty + SZ * tz] = t2[i];
       }
     __syncthreads();
     CT a[K], bb[K];
@@ -498,8 +301,8 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
 #pragma unroll
       for(int jj = 0; jj < NP; ++jj)
       {
-        s += tab.M[ly * NP + jj] * Z[i + CSY * (y0 + jj) + CSZ * tz];
-        if(DIM > 2) s2 += tab.M[ly * NP + jj] * T2[i + CSY * (y0 + jj) + CSZ * tz];
+        s += tab.M[ly * NP + jj] * Z[i + SY * (y0 + jj) + SZ * tz];
+        if(DIM > 2) s2 += tab.M[ly * NP + jj] * T2[i + SY * (y0 + jj) + SZ * tz];
       }
       a[i] = s;
       bb[i] = s2;
@@ -514,7 +317,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
       __syncthreads();
 #pragma unroll
       for(int i = 0; i < K; ++i)
-        if(owner) Z[i + CSY * ty + CSZ * tz] = a[i];
+        if(owner) Z[i + SY * ty + SZ * tz] = a[i];
       __syncthreads();
       const int z00 = bz * NP;
 #pragma unroll
@@ -522,25 +325,15 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
       {
         CT s = bb[i];
 #pragma unroll
-        for(int kk = 0; kk < NP; ++kk) s += tab.M[lz * NP + kk] * Z[i + CSY * ty + CSZ * (z00 + kk)];
+        for(int kk = 0; kk < NP; ++kk) s += tab.M[lz * NP + kk] * Z[i + SY * ty + SZ * (z00 + kk)];
         g[i] -= s;
       }
     }
   }
 
-  if constexpr(BATCH)
-  {
-    if constexpr(!S_SCALAR)
-#pragma unroll
-      for(int d = 0; d < 3; ++d) Ss[0][d][t] = sv[d];
-    if(t < 3 * K) (&ls[0][0][0])[t] = lv;
-    w = valid ? (omega ? CT(omega[min(j0, patch_end - 1)]) : relaxation) : CT(0);
-    __syncthreads();
-  }
-  // the factor tables in LDS are complete (without the coupling stage no
-  // barrier has passed since they were written)
-  else if(x_zero & kOuterZero)
-    __syncthreads();
+  // the factor tables in LDS are complete (without the coupling stage no barrier has
+  // passed since they were written)
+  if(x_zero & kOuterZero) __syncthreads();
   if constexpr(FD == 1)
   {
     static_assert(DIM == 3 && K == 8 && PPB == 2, "MFMA patch solve: 3D, K = 8, two patches per block");
@@ -561,32 +354,8 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   {
 #pragma unroll
     for(int i = 0; i < K; ++i) r[i] = g[i];
-    if constexpr(WAVE_PATCH)
-    {
-      // wave index as a wave-uniform value; the last patch of the pass stands
-      // in for a missing one (its results are discarded)
-      const int pw = __builtin_amdgcn_readfirstlane(int(threadIdx.x)) / 64;
-      const int jw = min(j0 + pw, patch_end - 1);
-      const uint32_t f0 = fac[size_t(jw) * DIM + 0], f1 = fac[size_t(jw) * DIM + 1],
-                     f2 = fac[size_t(jw) * DIM + 2];
-      const CT *G0 = S_tab + size_t(f0) * K * K, *G1 = S_tab + size_t(f1) * K * K,
-               *G2 = S_tab + size_t(f2) * K * K;
-      // even-odd products where all three 1D problems are mirror-symmetric
-      // (interior patches of a uniform mesh); a wave-uniform branch.  They read
-      // only the first K/2 rows of each matrix, which fit the scalar registers
-      // in FP64 too.
-      if(eo_tab && (eo_tab[f0] & eo_tab[f1] & eo_tab[f2]) != 0u)
-        fd_lines<DIM, K, CT, FSY, FSZ, true>(r, o, PAD ? A2[plc] : buf[plc], G0, G1, G2,
-                                             ls[plc][0], ls[plc][1], ls[plc][2], w, t, owner);
-      else
-        fd_lines<DIM, K, CT, FSY, FSZ, false>(
-          r, o, PAD ? A2[plc] : buf[plc], S_SCALAR ? G0 : Ss[plc][0], S_SCALAR ? G1 : Ss[plc][1],
-          S_SCALAR ? G2 : Ss[plc][2], ls[plc][0], ls[plc][1], ls[plc][2], w, t, owner);
-    }
-    else
-      fd_lines<DIM, K, CT, FSY, FSZ>(r, o, PAD ? A2[plc] : buf[plc], Ss[plc][0], Ss[plc][1],
-                                     Ss[plc][DIM > 2 ? 2 : 1], ls[plc][0], ls[plc][1],
-                                     ls[plc][DIM > 2 ? 2 : 1], w, t, owner);
+    fd_lines<DIM, K, CT>(r, o, buf[plc], Ss[plc][0], Ss[plc][1], Ss[plc][DIM > 2 ? 2 : 1],
+                         ls[plc][0], ls[plc][1], ls[plc][DIM > 2 ? 2 : 1], w, t, owner);
   }
   if(!valid) return;
   if(!(x_zero & kOwnZero) && w != CT(1))
@@ -607,6 +376,211 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   }
   store_row<NP>(x + c_lo * NDC + lyz, o);
   store_row<NP>(x + (c_lo + 1) * NDC + lyz, o + NP);
+}
+
+// ----------------------------------------------------------------------------
+// 3D Q3 color pass (K = 8) with vector solves: one patch per single-wave block.
+//
+// The coupling uses the rank of the face terms: with a neighbour line's trace
+// (v, v') on the face (its node value there, Gauss-Lobatto nodes, and one 4-term
+// product), s = +1 on the left face of a line, -1 on the right one,
+//   (B_j x_out)_i = (e_i P - s/2 g_i v) M M,  P = -sigma v + s/2 v',
+// e_i = 1 at the node on the face, g_i = phi_i' there.  Lane (l1, l2, c1, c2) =
+// bits (0-1, 2-3, 4, 5) holds the x-line (y, z) = (4 c1 + l1, 4 c2 + l2) of the
+// patch and, of each y- (z-) face, the tangential point (x, z) ((x, y)) of the same
+// indices with the neighbour's line along the normal: a cell is a DPP row and its
+// mass products run across its lanes without LDS.  The y- and z-face points then
+// pass through LDS once to the lanes of the x-lines, which take their M_x product in
+// registers.
+//
+// Bound by HBM: per color of the 64^3 level 42 us FP64 / 22 us FP32 (195 / 97.5 MB
+// compulsory, 222 / 106 MB moved), 57 / 29 us with plane-wise face products
+// (F z along the normal on every node, the masses across lines through LDS) and all
+// eigenvector matrices loaded at once (their scalar registers spilled).
+// ----------------------------------------------------------------------------
+template<typename CT>
+struct MvpTab
+{
+  CT M[16];
+  CT R[16];      // rows of M rotated to start at the diagonal: R[q*4 + r] = M(q, (q + r) mod 4)
+  CT g[2][4];    // phi_i'(0) / h, phi_i'(1) / h
+  CT sigma;
+};
+
+template<typename VT, typename CT>
+__global__ void __launch_bounds__(64, (std::is_same<CT, float>::value ? 6 : 2))
+k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<CT> tab,
+               const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
+               const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
+               const uint32_t *__restrict__ eo_tab, const float *__restrict__ omega,
+               const CT relaxation, const int patch_begin, const int n, const int x_zero,
+               int *__restrict__ nonfinite)
+{
+  constexpr int K = 8, NP = 4, NDC = 64, P = 3;
+  constexpr int SY = 8, SZ = 72;  // solve buffer (x, y, z) -> x + SY y + SZ z (bank conflicts)
+  // FP32 solves read the eigenvector matrices with wave-uniform addresses straight
+  // into scalar registers; FP64 ones only for the even-odd products (half matrices),
+  // the full ones are staged
+  constexpr bool S_SCALAR = std::is_same<CT, float>::value;
+  __shared__ __align__(16) CT B[K * SZ];  // solve; before it the face points [dir][side][v, P][64]
+  __shared__ CT Ss[3][S_SCALAR ? 1 : K * K];
+  __shared__ CT ls[3][K];
+  const int j = patch_begin + int(blockIdx.x);
+  const int t = threadIdx.x;
+  const int l1 = t & 3, l2 = (t >> 2) & 3, c1 = (t >> 4) & 1, c2 = t >> 5;
+  const int ty = 4 * c1 + l1, tz = 4 * c2 + l2;
+
+  // a starting wave issues its loads ahead of the other waves' arithmetic on the SIMD
+  // (raised priority until the last load of the batch is issued)
+  __builtin_amdgcn_s_setprio(3);
+  const uint32_t f0 = fac[size_t(j) * 3], f1 = fac[size_t(j) * 3 + 1], f2 = fac[size_t(j) * 3 + 2];
+  int v[3];
+  unpack_vertex(vtx[j], v);
+  const int64_t nn = int64_t(n) * n;
+  const int64_t cell0 = (v[0] - 1) + int64_t(n) * (v[1] - 1) + nn * (v[2] - 1);
+  const int64_t c_lo = cell0 + int64_t(n) * c1 + nn * c2;
+  const int lyz = NP * (t & 15);
+  CT sv[3], lv = CT(1);
+  if constexpr(!S_SCALAR)
+  {
+    sv[0] = S_tab[size_t(f0) * K * K + t];
+    sv[1] = S_tab[size_t(f1) * K * K + t];
+    sv[2] = S_tab[size_t(f2) * K * K + t];
+  }
+  if(t < 3 * K) lv = lam_tab[size_t(t < K ? f0 : t < 2 * K ? f1 : f2) * K + t % K];
+  CT g[K], r[K], o[K];
+  load_row<NP>(b + c_lo * NDC + lyz, g);
+  load_row<NP>(b + (c_lo + 1) * NDC + lyz, g + NP);
+
+  if(!(x_zero & kOuterZero))
+  {
+    // neighbour lines [direction][side]; absent neighbours read the patch's own cells (in
+    // bounds) and are discarded by selection (a branch would hold its loads back)
+    CT nl[3][2][NP];
+    const CT *tt = reinterpret_cast<const CT *>(&tab);
+    CT Ma[NP], Mb[NP];
+    load_row<NP>(x + (v[0] > 1 ? c_lo - 1 : c_lo) * NDC + lyz, nl[0][0]);
+    load_row<NP>(x + (v[0] + 1 < n ? c_lo + 2 : c_lo) * NDC + lyz, nl[0][1]);
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool hy = side ? v[1] + 1 < n : v[1] > 1, hz = side ? v[2] + 1 < n : v[2] > 1;
+      const VT *py = x + (cell0 + c1 + nn * c2 + (hy ? (side ? 2 * n : -n) : 0)) * NDC + l1 + 16 * l2;
+      const VT *pz = x + (cell0 + c1 + int64_t(n) * c2 + (hz ? (side ? 2 * nn : -nn) : 0)) * NDC + (t & 15);
+#pragma unroll
+      for(int jj = 0; jj < NP; ++jj)
+      {
+        nl[1][side][jj] = py[NP * jj];
+        nl[2][side][jj] = pz[NP * NP * jj];
+      }
+    }
+#pragma unroll
+    for(int q = 0; q < NP; ++q)
+    {
+      Ma[q] = tt[16 + l1 * NP + q];
+      Mb[q] = tt[16 + l2 * NP + q];
+    }
+    const CT gy = tt[32 + NP * c1 + l1], gz = tt[32 + NP * c2 + l2];  // g of this lane's y- and z-node
+    __builtin_amdgcn_s_setprio(0);
+    CT fv[3][2], fp[3][2];
+#pragma unroll
+    for(int d = 0; d < 3; ++d)
+#pragma unroll
+      for(int side = 0; side < 2; ++side)
+      {
+        const bool has = side ? v[d] + 1 < n : v[d] > 1;
+        CT dv = 0, q[NP];
+#pragma unroll
+        for(int jj = 0; jj < NP; ++jj) dv += tab.g[1 - side][jj] * nl[d][side][jj];
+        const CT vv = has ? nl[d][side][side ? 0 : P] : CT(0);
+        dv = has ? dv : CT(0);
+        const CT pp = (side ? CT(-0.5) : CT(0.5)) * dv - tab.sigma * vv;
+        // mass products across the lanes of the cell: both directions of an x-face, the
+        // second of a y- or z-face (z or y; x follows in the lanes of the lines)
+        lane_gather<NP, 1>(vv, nullptr, q);
+        fv[d][side] = dotn<NP>(Mb, q);
+        lane_gather<NP, 1>(pp, nullptr, q);
+        fp[d][side] = dotn<NP>(Mb, q);
+        if(d == 0)
+        {
+          lane_gather<NP, 0>(fv[d][side], nullptr, q);
+          fv[d][side] = dotn<NP>(Ma, q);
+          lane_gather<NP, 0>(fp[d][side], nullptr, q);
+          fp[d][side] = dotn<NP>(Ma, q);
+        }
+        else
+        {
+          CT *F = B + ((d - 1) * 2 + side) * 128 + K * tz + ty;
+          F[0] = fv[d][side];
+          F[64] = fp[d][side];
+        }
+      }
+    __syncthreads();
+    const CT ey = l1 == (c1 ? P : 0) ? CT(1) : CT(0), ez = l2 == (c2 ? P : 0) ? CT(1) : CT(0);
+    const CT ay = (c1 ? CT(0.5) : CT(-0.5)) * gy, az = (c2 ? CT(0.5) : CT(-0.5)) * gz;
+    const CT *Fy = B + c1 * 128 + K * tz, *Fz = B + 256 + c2 * 128 + K * ty;
+#pragma unroll
+    for(int cx = 0; cx < 2; ++cx)
+    {
+      CT q[NP];
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+        q[i] = ay * Fy[NP * cx + i] + ey * Fy[64 + NP * cx + i] + az * Fz[NP * cx + i] +
+               ez * Fz[64 + NP * cx + i];
+      const CT a = cx ? CT(0.5) * fv[0][1] : CT(-0.5) * fv[0][0];
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+      {
+        CT s = a * tab.g[cx][i];
+#pragma unroll
+        for(int jj = 0; jj < NP; ++jj) s += tab.M[i * NP + jj] * q[jj];
+        g[NP * cx + i] -= s;
+      }
+      g[cx ? K - 1 : 0] -= fp[0][cx];
+    }
+    __syncthreads();  // the face points are read: B is free for the solve
+  }
+  else
+    __builtin_amdgcn_s_setprio(0);
+
+  if constexpr(!S_SCALAR)
+#pragma unroll
+    for(int d = 0; d < 3; ++d) Ss[d][t] = sv[d];
+  if(t < 3 * K) (&ls[0][0])[t] = lv;
+  const CT w = omega ? CT(omega[j]) : relaxation;
+  __syncthreads();
+#pragma unroll
+  for(int i = 0; i < K; ++i) r[i] = g[i];
+  const CT *G0 = S_tab + size_t(f0) * K * K, *G1 = S_tab + size_t(f1) * K * K,
+           *G2 = S_tab + size_t(f2) * K * K;
+  // even-odd products where all three 1D problems are mirror-symmetric (interior
+  // patches of a uniform mesh); a wave-uniform branch
+  if((eo_tab[f0] & eo_tab[f1] & eo_tab[f2]) != 0u)
+    fd_lines<3, K, CT, SY, SZ, true, true>(r, o, B, G0, G1, G2, ls[0], ls[1], ls[2], w, ty + K * tz,
+                                           true);
+  else
+    fd_lines<3, K, CT, SY, SZ, false, S_SCALAR>(r, o, B, S_SCALAR ? G0 : Ss[0],
+                                                S_SCALAR ? G1 : Ss[1], S_SCALAR ? G2 : Ss[2], ls[0],
+                                                ls[1], ls[2], w, ty + K * tz, true);
+  VT *px = x + c_lo * NDC + lyz;
+  if(!(x_zero & kOwnZero) && w != CT(1))
+  {
+    CT old[K];
+    load_row<NP>(px, old);
+    load_row<NP>(px + NDC, old + NP);
+#pragma unroll
+    for(int a = 0; a < K; ++a) o[a] += (CT(1) - w) * old[a];
+  }
+  if(nonfinite)
+  {
+    // the non-finite check of the caller's output, on the values stored here
+    bool bad = false;
+#pragma unroll
+    for(int a = 0; a < K; ++a) bad = bad || !__builtin_isfinite(o[a]);
+    if(bad) *nonfinite = 1;
+  }
+  store_row<NP>(px, o);
+  store_row<NP>(px + NDC, o + NP);
 }
 
 // BF16-MFMA patch solves of the block-diagonal elasticity smoother (3D Q2, k = 6),

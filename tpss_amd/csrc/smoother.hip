@@ -206,15 +206,13 @@ void fit_local_solvers(const tpss_level *lv, LocalSolvers *ls, int sweeps, const
 // is cut into kTx x (8 / kTx) column tiles, one per XCD; a tile's patches go
 // z-slab by z-slab (lexicographic inside a slab), and the tiles' lists are
 // interleaved patch by patch (one patch per block), so that block i runs on XCD
-// i mod 8 and the three readers of a cell run on one XCD a slab apart.  Tiles
-// measured per 64^3 Q3 step: FP64 passes 0.914 ms with 1 x 8 (full-width y
-// bands), 0.920 with 2 x 4, 0.927 with 4 x 2, 0.969 with 8 x 1; FP32 passes
-// 0.453 ms with 4 x 2 or 2 x 4, 0.459 with 1 x 8.
+// i mod 8 and the three readers of a cell run on one XCD a slab apart.  kTx = 2
+// measured best or within 1 % of it (FP64 / FP32 sweeps with kTx = 1, 2, 4, 8: 64^3
+// 678, 678, 684, 717 / 364, 362, 365, 368 us; 48^3 FP64 375, 361, 359, 374 us).
 // Returns the positions [begin, end) in launch order.
-std::vector<int> xcd_launch_order(const LocalSolvers &ls, int begin, int end, int kTx)
+std::vector<int> xcd_launch_order(const LocalSolvers &ls, int begin, int end)
 {
-  constexpr int kXcd = 8;
-  const int kTy = kXcd / kTx;
+  constexpr int kXcd = 8, kTx = 2, kTy = kXcd / kTx;
   int lo[3] = {1 << 30, 1 << 30, 1 << 30}, hi[3] = {-1, -1, -1};
   auto block = [&](int j, int d) {
     const int x = ls.vtx_unpacked[size_t(j) * 3 + d] - 1;
@@ -403,8 +401,8 @@ std::shared_ptr<LocalSolvers> build_local_solvers(const tpss_level *lv,
     std::vector<uint32_t> vtx_l(static_cast<size_t>(P)), fac_l(static_cast<size_t>(P) * 3);
     for(int c = 0; c < ls->n_colors; ++c)
     {
-      const std::vector<int> order = xcd_launch_order(
-        *ls, ls->color_ptr[c], ls->color_ptr[c + 1], desc.local_precision == TPSS_F64 ? 1 : 4);
+      const std::vector<int> order =
+        xcd_launch_order(*ls, ls->color_ptr[c], ls->color_ptr[c + 1]);
       for(size_t q = 0; q < order.size(); ++q)
       {
         const size_t at = size_t(ls->color_ptr[c]) + q, j = size_t(order[q]);
@@ -561,7 +559,6 @@ void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, i
   const CT relax = CT(sm->desc.relaxation);
   dispatch_dim_np(ls.dim, ls.np, [&](auto D, auto NPc) {
     constexpr int DIM = decltype(D)::value, NP = decltype(NPc)::value, K = 2 * NP;
-    using PS = PatchShape<DIM, K>;
     OpTab<CT, NP> tab;
     const Operator1D &op = sm->level->op1d;
     for(int e = 0; e < NP * NP; ++e)
@@ -571,13 +568,13 @@ void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, i
       tab.Fmp[e] = CT(op.Fmp[e]);
       for(int c = 0; c < 4; ++c) tab.D[c][e] = CT(op.D[c][e]);
     }
-    using MS = MvpShape<DIM, K, FD>;
-    const unsigned grid = unsigned((end - begin + MS::PPB - 1) / MS::PPB);
+    using PS = PatchShape<DIM, K>;
+    const unsigned grid = unsigned((end - begin + PS::PPB - 1) / PS::PPB);
     if constexpr(FD == 1)
     {
       if constexpr(DIM == 3 && K == 8 && std::is_same<CT, float>::value)
-        hipLaunchKernelGGL((k_patch_mvp_fused<DIM, K, VT, CT, 1>), dim3(grid), dim3(MS::THREADS), 0,
-                           s, b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, nullptr, om, relax,
+        hipLaunchKernelGGL((k_patch_mvp_fused<DIM, K, VT, CT, 1>), dim3(grid), dim3(PS::THREADS), 0,
+                           s, b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax,
                            begin, end, ls.n, x_zero, sm->pass_flag);
       else
         throw Error(TPSS_E_UNSUPPORTED, "BF16-MFMA patch solves are built for 3D Q3 (k = 8)");
@@ -594,12 +591,29 @@ void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, i
           TPSS_HIP(hipGetLastError());
           return;
         }
-      // the XCD launch order where no per-patch damping is indexed by position
-      const bool xcd = om == nullptr && ls.d_vtx_launch.ptr != nullptr && MS::PPB == 1;
-      hipLaunchKernelGGL((k_patch_mvp_fused<DIM, K, VT, CT>), dim3(grid), dim3(MS::THREADS), 0, s,
-                         b, x, tab, xcd ? ls.d_vtx_launch.ptr : ls.d_vtx.ptr,
-                         xcd ? ls.d_fac_launch.ptr : ls.d_fac.ptr, S, lam, ls.d_eo.ptr, om, relax,
-                         begin, end, ls.n, x_zero, sm->pass_flag);
+      if constexpr(DIM == 3 && K == 8)
+      {
+        MvpTab<CT> mt;
+        for(int q = 0; q < 4; ++q)
+          for(int r = 0; r < 4; ++r)
+          {
+            mt.M[q * 4 + r] = CT(op.M[q * 4 + r]);
+            mt.R[q * 4 + r] = CT(op.M[q * 4 + (q + r) % 4]);
+          }
+        for(int f = 0; f < 2; ++f)
+          for(int i = 0; i < 4; ++i) mt.g[f][i] = CT(op.g[f][i]);
+        mt.sigma = CT(op.sigma);
+        // the XCD launch order where no per-patch damping is indexed by position
+        const bool xcd = om == nullptr && ls.d_vtx_launch.ptr != nullptr;
+        hipLaunchKernelGGL((k_patch_mvp_q3<VT, CT>), dim3(unsigned(end - begin)), dim3(64), 0, s, b,
+                           x, mt, xcd ? ls.d_vtx_launch.ptr : ls.d_vtx.ptr,
+                           xcd ? ls.d_fac_launch.ptr : ls.d_fac.ptr, S, lam, ls.d_eo.ptr, om, relax,
+                           begin, ls.n, x_zero, sm->pass_flag);
+      }
+      else
+        hipLaunchKernelGGL((k_patch_mvp_fused<DIM, K, VT, CT>), dim3(grid), dim3(PS::THREADS), 0, s,
+                           b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax,
+                           begin, end, ls.n, x_zero, sm->pass_flag);
     }
     TPSS_HIP(hipGetLastError());
   });
