@@ -124,8 +124,8 @@ def write_traffic(fetch_csv, write_csv, cal_fetch_csv, cal_write_csv, n=64, p=3)
     f, w = means(fetch_csv), means(write_csv)
     out = {"fetch_factor": fetch_factor, "write_factor": write_factor,
            "calibration": f"k_convert<float, double>, N = {n_copy}"}
-    for name, tag in (("f64", "double, double, 0>"), ("f32", "float, float, 0>")):
-        k = next((k for k in f if "k_patch_mvp_fused<3, 8, " + tag in k), None)
+    for name, tag in (("f64", "double, double>"), ("f32", "float, float>")):
+        k = next((k for k in f if "k_patch_mvp_q3<" + tag in k), None)
         if k is None:
             continue
         fk, wk = float(np.mean([v for v, _ in f[k]])), float(np.mean([v for v, _ in w[k]]))

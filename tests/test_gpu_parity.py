@@ -490,3 +490,23 @@ def test_vmult_ignores_the_contents_of_dst_with_patch_damping(n):
     d = dev(np.full(ref.N, np.nan))
     sm.vmult(d, dev(src))
     assert rel_err(host(d), ref.smoother_vmult(src)) < 1e-6  # omega is kept in FP32
+
+
+# every color pass kernel at the edges of its blocks: patches per block 64 / K (2D), 4 (3D
+# Q1) or 1, patches with boundary faces on both sides, colors without patches; from a
+# given x, damped and undamped, FP64, FP32 and FP32 solves of FP64 vectors
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 2), (2, 1, 9), (2, 2, 3), (2, 2, 12), (2, 3, 5), (2, 3, 14),
+                                     (2, 4, 4), (2, 4, 11), (3, 1, 2), (3, 1, 7), (3, 2, 3), (3, 2, 5),
+                                     (3, 3, 2), (3, 3, 3), (3, 4, 2), (3, 4, 5)])
+@pytest.mark.parametrize("vec,loc,relax", [(0, 0, 1.0), (0, 0, 0.8), (1, 1, 1.0), (0, 1, 0.9)])
+def test_color_pass_block_edges(dim, p, n, vec, loc, relax):
+    lv, sm, ref = make(dim, p, n, 1, ip=2.0, relaxation=relax, precision=vec, local_precision=loc)
+    dt = np.float32 if vec else np.float64
+    x0 = o.splitmix_uniform(5, ref.N).astype(dt)
+    b = o.splitmix_uniform(6, ref.N).astype(dt)
+    x = dev(np.concatenate([x0, np.full(8, 7.0, dt)]), vec)  # guard values behind the output
+    sm.step(x, dev(b, vec))
+    got = host(x)
+    assert rel_err(got[:ref.N], ref.step(x0.astype(np.float64), b.astype(np.float64))) < (
+        2e-5 if loc else 1e-12)
+    assert (got[ref.N:] == 7.0).all()

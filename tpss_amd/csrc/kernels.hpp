@@ -925,8 +925,8 @@ __device__ __forceinline__ CT eig_scale(CT s, CT w, CT lam)
 // face), so each product takes two (K/2 x K/2) blocks of S on the folded line
 // r_a +- r_{K-1-a}: half the multiply-adds.  (A compile-time choice: a
 // run-time one keeps the line arrays out of registers.)
-template<int K, bool EVEN_ODD, typename SP, typename CT>
-__device__ __forceinline__ void s_forward(const SP S, const CT *r, CT *o)
+template<int K, bool EVEN_ODD, typename CT>
+__device__ __forceinline__ void s_forward(const CT *S, const CT *r, CT *o)
 {
   constexpr int P = K / 2;
   if constexpr(EVEN_ODD)
@@ -965,8 +965,8 @@ __device__ __forceinline__ void s_forward(const SP S, const CT *r, CT *o)
   }
 }
 
-template<int K, bool EVEN_ODD, typename SP, typename CT>
-__device__ __forceinline__ void s_backward(const SP S, const CT *o, CT *r)
+template<int K, bool EVEN_ODD, typename CT>
+__device__ __forceinline__ void s_backward(const CT *S, const CT *o, CT *r)
 {
   constexpr int P = K / 2;
   if constexpr(EVEN_ODD)
@@ -998,18 +998,69 @@ __device__ __forceinline__ void s_backward(const SP S, const CT *o, CT *r)
   }
 }
 
-// A wave-uniform matrix in read-only global memory as an operand of scalar loads at
-// the point of use.  The pointer is opaque to the compiler: without that it loads the
-// matrices of all stages at once, which exceeds the scalar registers (in the FP64
-// solve 440 of 1300 VALU instructions saved and restored them).
+// The same products with a wave-uniform matrix in read-only global memory, its rows
+// loaded into scalar registers a few at a time.  The pointer of every group is opaque
+// to the compiler: without that it loads the matrices of all stages at once, which
+// exceeds the scalar registers (in the FP64 K = 8 solve 440 of 1300 VALU instructions
+// saved and restored them).
 template<typename CT>
-using scalar_ptr = const __attribute__((address_space(4))) CT *;
-template<typename CT>
-__device__ __forceinline__ scalar_ptr<CT> scalar_rows(const CT *p)
+__device__ __forceinline__ auto scalar_rows(const CT *p)
 {
-  scalar_ptr<CT> q = (scalar_ptr<CT>)p;
+  typedef const __attribute__((address_space(4))) CT *ptr;
+  ptr q = (ptr)p;
   asm volatile("" : "+s"(q));
   return q;
+}
+
+// rows of K values per group: at most 64 scalar registers
+template<int K, typename CT>
+constexpr int scalar_row_group()
+{
+  return 64 / (K * int(sizeof(CT) / 4));
+}
+
+template<int K, bool EVEN_ODD, typename CT>
+__device__ __forceinline__ void s_forward_scalar(const CT *S, const CT *r, CT *o)
+{
+  constexpr int P = K / 2, R = EVEN_ODD ? P : K, G = scalar_row_group<K, CT>();
+#pragma unroll
+  for(int i = 0; i < K; ++i) o[i] = 0;
+#pragma unroll
+  for(int a0 = 0; a0 < R; a0 += G)
+  {
+    const auto rows = scalar_rows(S + a0 * K);
+#pragma unroll
+    for(int a = a0; a < (a0 + G < R ? a0 + G : R); ++a)
+    {
+      const CT rp = EVEN_ODD ? r[a] + r[K - 1 - a] : r[a], rm = EVEN_ODD ? r[a] - r[K - 1 - a] : r[a];
+#pragma unroll
+      for(int i = 0; i < K; ++i) o[i] += rows[(a - a0) * K + i] * (i < P ? rp : rm);
+    }
+  }
+}
+
+template<int K, bool EVEN_ODD, typename CT>
+__device__ __forceinline__ void s_backward_scalar(const CT *S, const CT *o, CT *r)
+{
+  constexpr int P = K / 2, R = EVEN_ODD ? P : K, G = scalar_row_group<K, CT>();
+#pragma unroll
+  for(int a0 = 0; a0 < R; a0 += G)
+  {
+    const auto rows = scalar_rows(S + a0 * K);
+#pragma unroll
+    for(int a = a0; a < (a0 + G < R ? a0 + G : R); ++a)
+    {
+      CT sp = 0, sm = 0;
+#pragma unroll
+      for(int i = 0; i < P; ++i)
+      {
+        sp += rows[(a - a0) * K + i] * o[i];
+        sm += rows[(a - a0) * K + P + i] * o[P + i];
+      }
+      r[a] = sp + sm;
+      if(EVEN_ODD) r[K - 1 - a] = sp - sm;
+    }
+  }
 }
 
 // Fast-diagonalization inverse of one patch held as x-lines: thread t owns the
@@ -1019,7 +1070,7 @@ __device__ __forceinline__ scalar_ptr<CT> scalar_rows(const CT *p)
 // The line direction rotates x -> y -> z -> y -> x through the patch's LDS
 // buffer B (entry (x, y, z) at x + SY y + SZ z: padded strides keep the
 // transposes free of LDS bank conflicts); EO: even-odd products in every
-// direction; SCALAR: the matrices are wave-uniform in global memory (scalar_rows).
+// direction; SCALAR: the matrices are wave-uniform in global memory.
 // Contains __syncthreads (every thread of the block must call it).
 template<int DIM, int K, typename CT, int SY = K, int SZ = K * K, bool EO = false, bool SCALAR = false>
 __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, const CT *S1,
@@ -1028,13 +1079,19 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
 {
   const int ty = DIM > 1 ? t % K : 0;
   const int tz = DIM > 2 ? t / K : 0;
-  auto rows = [](const CT *S) {
+  auto fwd = [](const CT *S, const CT *in, CT *out) {
     if constexpr(SCALAR)
-      return scalar_rows(S);
+      s_forward_scalar<K, EO>(S, in, out);
     else
-      return S;
+      s_forward<K, EO>(S, in, out);
   };
-  s_forward<K, EO>(rows(S0), r, o);
+  auto bwd = [](const CT *S, const CT *in, CT *out) {
+    if constexpr(SCALAR)
+      s_backward_scalar<K, EO>(S, in, out);
+    else
+      s_backward<K, EO>(S, in, out);
+  };
+  fwd(S0, r, o);
   if(DIM == 2)
   {
 #pragma unroll
@@ -1044,10 +1101,10 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
     const int x0 = t;
 #pragma unroll
     for(int jj = 0; jj < K; ++jj) r[jj] = B[x0 + SY * jj];
-    s_forward<K, EO>(rows(S1), r, o);
+    fwd(S1, r, o);
 #pragma unroll
     for(int jj = 0; jj < K; ++jj) o[jj] = eig_scale(o[jj], w, l0[x0] + l1[jj]);
-    s_backward<K, EO>(rows(S1), o, r);
+    bwd(S1, o, r);
     __syncthreads();
 #pragma unroll
     for(int b = 0; b < K; ++b)
@@ -1066,7 +1123,7 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
       const int x0 = t % K, z0 = t / K;
 #pragma unroll
       for(int jj = 0; jj < K; ++jj) r[jj] = B[x0 + SY * jj + SZ * z0];
-      s_forward<K, EO>(rows(S1), r, o);
+      fwd(S1, r, o);
 #pragma unroll
       for(int jj = 0; jj < K; ++jj)
         if(owner) B[x0 + SY * jj + SZ * z0] = o[jj];
@@ -1077,11 +1134,10 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
 #pragma unroll
       for(int l = 0; l < K; ++l) r[l] = B[x0 + SY * y0 + SZ * l];
       const CT lxy = l0[x0] + l1[y0];
-      const auto R2 = rows(S2);
-      s_forward<K, EO>(R2, r, o);
+      fwd(S2, r, o);
 #pragma unroll
       for(int l = 0; l < K; ++l) o[l] = eig_scale(o[l], w, lxy + l2[l]);
-      s_backward<K, EO>(R2, o, r);
+      bwd(S2, o, r);
 #pragma unroll
       for(int c = 0; c < K; ++c)
         if(owner) B[x0 + SY * y0 + SZ * c] = r[c];
@@ -1091,7 +1147,7 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
       const int x0 = t % K, z0 = t / K;
 #pragma unroll
       for(int jj = 0; jj < K; ++jj) r[jj] = B[x0 + SY * jj + SZ * z0];
-      s_backward<K, EO>(rows(S1), r, o);
+      bwd(S1, r, o);
 #pragma unroll
       for(int b = 0; b < K; ++b)
         if(owner) B[x0 + SY * b + SZ * z0] = o[b];
@@ -1100,7 +1156,7 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
 #pragma unroll
     for(int i = 0; i < K; ++i) r[i] = B[i + SY * ty + SZ * tz];
   }
-  s_backward<K, EO>(rows(S0), r, o);
+  bwd(S0, r, o);
 }
 
 template<int DIM, int K, typename VT, typename CT, int MODE>

@@ -97,32 +97,24 @@ __device__ __forceinline__ void fd_mfma_pair(float (*B2)[512], const float (*S)[
   }
 }
 
-// FD = 0: vector FMA contractions in CT; FD = 1: BF16 MFMA contractions with
-// FP32 accumulation (3D, K = 8, CT = float)
-// Waves per SIMD the register allocation must allow: FP32 patch solves 5 (<= 96
-// VGPRs) up to K = 8; longer lines (K = 10) hold more values per thread: 3; FP64
-// solves unconstrained.
-template<int K, typename CT, int FD>
-constexpr int mvp_min_waves()
+// Color pass with BF16-MFMA patch solves (3D, K = 8; FP32 arithmetic elsewhere), two
+// patches per block.
+template<typename VT>
+__global__ void __launch_bounds__(128)
+k_patch_mvp_bf16(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<float, 4> tab,
+                 const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
+                 const float *__restrict__ S_tab, const float *__restrict__ lam_tab,
+                 const float *__restrict__ omega, const float relaxation, const int patch_begin,
+                 const int patch_end, const int n, const int x_zero)
 {
-  return FD == 1 || !std::is_same<CT, float>::value ? 1 : K <= 8 ? 5 : 3;
-}
-
-template<int DIM, int K, typename VT, typename CT, int FD = 0>
-__global__ void __launch_bounds__((PatchShape<DIM, K>::THREADS), (mvp_min_waves<K, CT, FD>()))
-k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, K / 2> tab,
-                  const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
-                  const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
-                  const float *__restrict__ omega, const CT relaxation, const int patch_begin,
-                  const int patch_end, const int n, const int x_zero,
-                  int *__restrict__ nonfinite)
-{
+  using CT = float;
+  constexpr int DIM = 3, K = 8;
   using PS = PatchShape<DIM, K>;
   constexpr int NP = PS::NP, L = PS::L, NPD = PS::NPD, NDC = PS::NDC, PPB = PS::PPB;
   constexpr int SY = K, SZ = K * K;  // strides (y, z) of the patch buffers
   __shared__ CT buf[PPB][NPD];
   __shared__ CT A1[PPB][NPD];
-  __shared__ CT A2[PPB][DIM > 2 ? NPD : 1];
+  __shared__ CT A2[PPB][NPD];
   __shared__ CT Ss[PPB][DIM][K * K];
   __shared__ CT ls[PPB][DIM][K];
 
@@ -151,8 +143,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   if(valid) unpack_vertex(vtx[j], v);
   const CT w = valid ? (omega ? CT(omega[j]) : relaxation) : CT(0);
 
-  const int ty = DIM > 1 ? t % K : 0;
-  const int tz = DIM > 2 ? t / K : 0;
+  const int ty = t % K, tz = t / K;
   const int ly = ty >= NP ? ty - NP : ty, lz = tz >= NP ? tz - NP : tz;
   const int by = ty >= NP ? 1 : 0, bz = tz >= NP ? 1 : 0;
   const int64_t nn = int64_t(n) * n;
@@ -160,7 +151,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
   // the x-line (ty, tz) of the patch: row lyz of the cells c_lo and c_lo + 1
   const int64_t c_lo = patch_cell<DIM, NP>(v, n, 0, ty, tz);
   const int lyz = patch_local<DIM, NP>(0, ty, tz);
-  CT g[K], r[K], o[K];
+  CT g[K];
   if(valid)
   {
     load_row<NP>(b + c_lo * NDC + lyz, g);
@@ -244,7 +235,6 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
           }
       }
     }
-    if(DIM > 2)
     {
       const bool has = bz == 0 ? (v[2] - 1 > 0) : (v[2] + 1 < n);
       const CT *F = bz == 0 ? tab.Fpm : tab.Fmp;
@@ -289,7 +279,7 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
       if(owner)
       {
         Z[i + SY * ty + SZ * tz] = z0[i];
-        if(DIM > 2) T2[i + SY * ty + SZ * tz] = t2[i];
+        T2[i + SY * ty + SZ * tz] = t2[i];
       }
     __syncthreads();
     CT a[K], bb[K];
@@ -302,61 +292,39 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
       for(int jj = 0; jj < NP; ++jj)
       {
         s += tab.M[ly * NP + jj] * Z[i + SY * (y0 + jj) + SZ * tz];
-        if(DIM > 2) s2 += tab.M[ly * NP + jj] * T2[i + SY * (y0 + jj) + SZ * tz];
+        s2 += tab.M[ly * NP + jj] * T2[i + SY * (y0 + jj) + SZ * tz];
       }
       a[i] = s;
       bb[i] = s2;
     }
-    if(DIM == 2)
+    __syncthreads();
+#pragma unroll
+    for(int i = 0; i < K; ++i)
+      if(owner) Z[i + SY * ty + SZ * tz] = a[i];
+    __syncthreads();
+    const int z00 = bz * NP;
+#pragma unroll
+    for(int i = 0; i < K; ++i)
     {
+      CT s = bb[i];
 #pragma unroll
-      for(int i = 0; i < K; ++i) g[i] -= a[i];
-    }
-    else
-    {
-      __syncthreads();
-#pragma unroll
-      for(int i = 0; i < K; ++i)
-        if(owner) Z[i + SY * ty + SZ * tz] = a[i];
-      __syncthreads();
-      const int z00 = bz * NP;
-#pragma unroll
-      for(int i = 0; i < K; ++i)
-      {
-        CT s = bb[i];
-#pragma unroll
-        for(int kk = 0; kk < NP; ++kk) s += tab.M[lz * NP + kk] * Z[i + SY * ty + SZ * (z00 + kk)];
-        g[i] -= s;
-      }
+      for(int kk = 0; kk < NP; ++kk) s += tab.M[lz * NP + kk] * Z[i + SY * ty + SZ * (z00 + kk)];
+      g[i] -= s;
     }
   }
 
-  // the factor tables in LDS are complete (without the coupling stage no barrier has
-  // passed since they were written)
-  if(x_zero & kOuterZero) __syncthreads();
-  if constexpr(FD == 1)
-  {
-    static_assert(DIM == 3 && K == 8 && PPB == 2, "MFMA patch solve: 3D, K = 8, two patches per block");
-    __shared__ float w2[2];
-    if(t == 0 && owner) w2[pl] = float(w);
-    __syncthreads();  // the coupling stage above may still read A1/A2; buf is free
+  __shared__ float w2[2];
+  if(t == 0 && owner) w2[pl] = w;
 #pragma unroll
-    for(int i = 0; i < K; ++i)
-      if(owner) buf[plc][i + K * ty + K * K * tz] = float(g[i]);
-    __syncthreads();
-    fd_mfma_pair(reinterpret_cast<float(*)[512]>(&buf[0][0]),
-                 reinterpret_cast<const float(*)[3][64]>(&Ss[0][0][0]),
-                 reinterpret_cast<const float(*)[3][8]>(&ls[0][0][0]), w2);
+  for(int i = 0; i < K; ++i)
+    if(owner) buf[plc][i + K * ty + K * K * tz] = g[i];
+  __syncthreads();
+  fd_mfma_pair(reinterpret_cast<float(*)[512]>(&buf[0][0]),
+               reinterpret_cast<const float(*)[3][64]>(&Ss[0][0][0]),
+               reinterpret_cast<const float(*)[3][8]>(&ls[0][0][0]), w2);
+  CT o[K];
 #pragma unroll
-    for(int i = 0; i < K; ++i) o[i] = buf[plc][i + K * ty + K * K * tz];
-  }
-  else
-  {
-#pragma unroll
-    for(int i = 0; i < K; ++i) r[i] = g[i];
-    fd_lines<DIM, K, CT>(r, o, buf[plc], Ss[plc][0], Ss[plc][1], Ss[plc][DIM > 2 ? 2 : 1],
-                         ls[plc][0], ls[plc][1], ls[plc][DIM > 2 ? 2 : 1], w, t, owner);
-  }
+  for(int i = 0; i < K; ++i) o[i] = buf[plc][i + K * ty + K * K * tz];
   if(!valid) return;
   if(!(x_zero & kOwnZero) && w != CT(1))
   {
@@ -365,14 +333,6 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
     load_row<NP>(x + (c_lo + 1) * NDC + lyz, old + NP);
 #pragma unroll
     for(int a = 0; a < K; ++a) o[a] += (CT(1) - w) * old[a];
-  }
-  if(nonfinite)
-  {
-    // the non-finite check of the caller's output, on the values stored here
-    bool bad = false;
-#pragma unroll
-    for(int a = 0; a < K; ++a) bad = bad || !__builtin_isfinite(o[a]);
-    if(bad) *nonfinite = 1;
   }
   store_row<NP>(x + c_lo * NDC + lyz, o);
   store_row<NP>(x + (c_lo + 1) * NDC + lyz, o + NP);
@@ -398,18 +358,18 @@ k_patch_mvp_fused(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<CT, 
 // (F z along the normal on every node, the masses across lines through LDS) and all
 // eigenvector matrices loaded at once (their scalar registers spilled).
 // ----------------------------------------------------------------------------
-template<typename CT>
+template<int NP, typename CT>
 struct MvpTab
 {
-  CT M[16];
-  CT R[16];      // rows of M rotated to start at the diagonal: R[q*4 + r] = M(q, (q + r) mod 4)
-  CT g[2][4];    // phi_i'(0) / h, phi_i'(1) / h
+  CT M[NP * NP];
+  CT R[NP * NP];  // rows of M rotated to start at the diagonal: R[q*NP + r] = M(q, (q + r) mod NP)
+  CT g[2][NP];    // phi_i'(0) / h, phi_i'(1) / h
   CT sigma;
 };
 
 template<typename VT, typename CT>
 __global__ void __launch_bounds__(64, (std::is_same<CT, float>::value ? 6 : 2))
-k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<CT> tab,
+k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<4, CT> tab,
                const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
                const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
                const uint32_t *__restrict__ eo_tab, const float *__restrict__ omega,
@@ -418,12 +378,7 @@ k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<CT> ta
 {
   constexpr int K = 8, NP = 4, NDC = 64, P = 3;
   constexpr int SY = 8, SZ = 72;  // solve buffer (x, y, z) -> x + SY y + SZ z (bank conflicts)
-  // FP32 solves read the eigenvector matrices with wave-uniform addresses straight
-  // into scalar registers; FP64 ones only for the even-odd products (half matrices),
-  // the full ones are staged
-  constexpr bool S_SCALAR = std::is_same<CT, float>::value;
   __shared__ __align__(16) CT B[K * SZ];  // solve; before it the face points [dir][side][v, P][64]
-  __shared__ CT Ss[3][S_SCALAR ? 1 : K * K];
   __shared__ CT ls[3][K];
   const int j = patch_begin + int(blockIdx.x);
   const int t = threadIdx.x;
@@ -440,13 +395,7 @@ k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<CT> ta
   const int64_t cell0 = (v[0] - 1) + int64_t(n) * (v[1] - 1) + nn * (v[2] - 1);
   const int64_t c_lo = cell0 + int64_t(n) * c1 + nn * c2;
   const int lyz = NP * (t & 15);
-  CT sv[3], lv = CT(1);
-  if constexpr(!S_SCALAR)
-  {
-    sv[0] = S_tab[size_t(f0) * K * K + t];
-    sv[1] = S_tab[size_t(f1) * K * K + t];
-    sv[2] = S_tab[size_t(f2) * K * K + t];
-  }
+  CT lv = CT(1);
   if(t < 3 * K) lv = lam_tab[size_t(t < K ? f0 : t < 2 * K ? f1 : f2) * K + t % K];
   CT g[K], r[K], o[K];
   load_row<NP>(b + c_lo * NDC + lyz, g);
@@ -543,9 +492,6 @@ k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<CT> ta
   else
     __builtin_amdgcn_s_setprio(0);
 
-  if constexpr(!S_SCALAR)
-#pragma unroll
-    for(int d = 0; d < 3; ++d) Ss[d][t] = sv[d];
   if(t < 3 * K) (&ls[0][0])[t] = lv;
   const CT w = omega ? CT(omega[j]) : relaxation;
   __syncthreads();
@@ -559,9 +505,8 @@ k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<CT> ta
     fd_lines<3, K, CT, SY, SZ, true, true>(r, o, B, G0, G1, G2, ls[0], ls[1], ls[2], w, ty + K * tz,
                                            true);
   else
-    fd_lines<3, K, CT, SY, SZ, false, S_SCALAR>(r, o, B, S_SCALAR ? G0 : Ss[0],
-                                                S_SCALAR ? G1 : Ss[1], S_SCALAR ? G2 : Ss[2], ls[0],
-                                                ls[1], ls[2], w, ty + K * tz, true);
+    fd_lines<3, K, CT, SY, SZ, false, true>(r, o, B, G0, G1, G2, ls[0], ls[1], ls[2], w, ty + K * tz,
+                                            true);
   VT *px = x + c_lo * NDC + lyz;
   if(!(x_zero & kOwnZero) && w != CT(1))
   {
@@ -574,6 +519,344 @@ k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<CT> ta
   if(nonfinite)
   {
     // the non-finite check of the caller's output, on the values stored here
+    bool bad = false;
+#pragma unroll
+    for(int a = 0; a < K; ++a) bad = bad || !__builtin_isfinite(o[a]);
+    if(bad) *nonfinite = 1;
+  }
+  store_row<NP>(px, o);
+  store_row<NP>(px + NDC, o + NP);
+}
+
+// ----------------------------------------------------------------------------
+// The same 3D color pass for the other degrees (K = 4, 6, 10).  Lane (a, b) = (t % K,
+// t / K) of a patch holds the x-line (y, z) = (a, b) and the tangential point of each
+// face with these indices; the mass products across lanes go through LDS (two
+// exchanges: along b for all face points, then along a for the x-faces and as rows
+// for the y- and z-faces).  Every global load of the pass is issued before the first
+// wait.  K = 6, 10: one patch per block, the eigenvector matrices as scalar operands;
+// K = 4: four patches per wave, matrices staged in LDS.
+// Sweeps: 48^3 Q4 FP64 759 us (2246 with staging loops, plane-wise face products and a
+// branch per neighbour), 27^3 Q4 FP64 268 (534), 64^3 Q2 FP32 290 (404), 33^3 Q2 FP64 142
+// (181), 100^3 Q1 FP32 408 (472).
+// ----------------------------------------------------------------------------
+template<int K>
+struct MvpLinesShape
+{
+  static constexpr int L = K * K;
+  static constexpr int PPB = L <= 16 ? 64 / L : 1;
+  static constexpr int THREADS = ((PPB * L + 63) / 64) * 64;
+};
+
+template<int K, typename VT, typename CT>
+__global__ void __launch_bounds__((MvpLinesShape<K>::THREADS))
+k_patch_mvp_lines(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<K / 2, CT> tab,
+                  const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
+                  const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
+                  const uint32_t *__restrict__ eo_tab, const float *__restrict__ omega,
+                  const CT relaxation, const int patch_begin, const int patch_end, const int n,
+                  const int x_zero, int *__restrict__ nonfinite)
+{
+  using MS = MvpLinesShape<K>;
+  constexpr int NP = K / 2, P = NP - 1, NL = NP * NP, NDC = NL * NP, L = MS::L, PPB = MS::PPB;
+  constexpr bool SCALAR = PPB == 1;
+  constexpr int NS = 3 * K * K;  // eigenvector entries of a patch
+  static_assert(12 * L >= K * L, "the solve buffer fits in the first face buffer");
+  __shared__ CT F1[PPB][12][L];  // face points [direction][side][v, P]; then the solve
+  __shared__ CT F2[PPB][12][L];  // ... contracted along b
+  __shared__ CT Ss[PPB][SCALAR ? 1 : NS];
+  __shared__ CT ls[PPB][3][K];
+  const int pl = PPB == 1 ? 0 : int(threadIdx.x) / L;
+  const int t0 = int(threadIdx.x) - pl * L;
+  const bool owner = t0 < L;
+  const int t = owner ? t0 : L - 1;  // lanes beyond the patch repeat its last line
+  const int jj = patch_begin + int(blockIdx.x) * PPB + pl;
+  const bool valid = owner && jj < patch_end;
+  const int j = jj < patch_end ? jj : patch_end - 1;
+  const int ta = t % K, tb = t / K, c1 = ta / NP, c2 = tb / NP, l1 = ta - NP * c1, l2 = tb - NP * c2;
+
+  const uint32_t f0 = fac[size_t(j) * 3], f1 = fac[size_t(j) * 3 + 1], f2 = fac[size_t(j) * 3 + 2];
+  int v[3];
+  unpack_vertex(vtx[j], v);
+  const int64_t nn = int64_t(n) * n;
+  const int64_t cell0 = (v[0] - 1) + int64_t(n) * (v[1] - 1) + nn * (v[2] - 1);
+  const int64_t c_lo = cell0 + int64_t(n) * c1 + nn * c2;
+  const int lyz = NP * l1 + NL * l2;
+  CT lv = CT(1), sv[SCALAR ? 1 : (NS + L - 1) / L];
+  if(t0 < 3 * K) lv = lam_tab[size_t(t < K ? f0 : t < 2 * K ? f1 : f2) * K + t % K];
+  if constexpr(!SCALAR)
+#pragma unroll
+    for(int k = 0; k < NS / L; ++k)
+    {
+      static_assert(SCALAR || L == K * K, "a lane stages one entry of each matrix");
+      sv[k] = S_tab[size_t(k == 0 ? f0 : k == 1 ? f1 : f2) * K * K + t];
+    }
+  CT g[K], r[K], o[K];
+  load_row<NP>(b + c_lo * NDC + lyz, g);
+  load_row<NP>(b + (c_lo + 1) * NDC + lyz, g + NP);
+  const CT w = omega ? CT(omega[j]) : relaxation;
+
+  if(!(x_zero & kOuterZero))
+  {
+    CT nl[3][2][NP];
+    const CT *tt = reinterpret_cast<const CT *>(&tab);
+    load_row<NP>(x + (v[0] > 1 ? c_lo - 1 : c_lo) * NDC + lyz, nl[0][0]);
+    load_row<NP>(x + (v[0] + 1 < n ? c_lo + 2 : c_lo) * NDC + lyz, nl[0][1]);
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool hy = side ? v[1] + 1 < n : v[1] > 1, hz = side ? v[2] + 1 < n : v[2] > 1;
+      const VT *py = x + (cell0 + c1 + nn * c2 + (hy ? (side ? 2 * n : -n) : 0)) * NDC + l1 + NL * l2;
+      const VT *pz =
+        x + (cell0 + c1 + int64_t(n) * c2 + (hz ? (side ? 2 * nn : -nn) : 0)) * NDC + l1 + NP * l2;
+#pragma unroll
+      for(int k = 0; k < NP; ++k)
+      {
+        nl[1][side][k] = py[NP * k];
+        nl[2][side][k] = pz[NL * k];
+      }
+    }
+    CT Ma[NP], Mb[NP];
+#pragma unroll
+    for(int q = 0; q < NP; ++q)
+    {
+      Ma[q] = tt[l1 * NP + q];
+      Mb[q] = tt[l2 * NP + q];
+    }
+    const CT gy = tt[2 * NL + NP * c1 + l1], gz = tt[2 * NL + NP * c2 + l2];
+#pragma unroll
+    for(int d = 0; d < 3; ++d)
+#pragma unroll
+      for(int side = 0; side < 2; ++side)
+      {
+        const bool has = side ? v[d] + 1 < n : v[d] > 1;
+        CT dv = 0;
+#pragma unroll
+        for(int k = 0; k < NP; ++k) dv += tab.g[1 - side][k] * nl[d][side][k];
+        const CT vv = has ? nl[d][side][side ? 0 : P] : CT(0);
+        dv = has ? dv : CT(0);
+        if(owner)
+        {
+          F1[pl][d * 4 + side * 2][t] = vv;
+          F1[pl][d * 4 + side * 2 + 1][t] = (side ? CT(-0.5) : CT(0.5)) * dv - tab.sigma * vv;
+        }
+      }
+    __syncthreads();
+#pragma unroll
+    for(int k = 0; k < 12; ++k)
+    {
+      CT s = 0;
+#pragma unroll
+      for(int q = 0; q < NP; ++q) s += Mb[q] * F1[pl][k][ta + K * (NP * c2 + q)];
+      if(owner) F2[pl][k][t] = s;
+    }
+    __syncthreads();
+    const CT ey = l1 == (c1 ? P : 0) ? CT(1) : CT(0), ez = l2 == (c2 ? P : 0) ? CT(1) : CT(0);
+    const CT ay = (c1 ? CT(0.5) : CT(-0.5)) * gy, az = (c2 ? CT(0.5) : CT(-0.5)) * gz;
+    const CT *Fy = &F2[pl][4 + 2 * c1][K * tb], *Fz = &F2[pl][8 + 2 * c2][K * ta];
+#pragma unroll
+    for(int cx = 0; cx < 2; ++cx)
+    {
+      CT q[NP], xv = 0, xp = 0;
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+      {
+        q[i] = ay * Fy[NP * cx + i] + ey * Fy[L + NP * cx + i] + az * Fz[NP * cx + i] +
+               ez * Fz[L + NP * cx + i];
+        xv += Ma[i] * F2[pl][2 * cx][NP * c1 + i + K * tb];
+        xp += Ma[i] * F2[pl][2 * cx + 1][NP * c1 + i + K * tb];
+      }
+      const CT a = (cx ? CT(0.5) : CT(-0.5)) * xv;
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+      {
+        CT s = a * tab.g[cx][i];
+#pragma unroll
+        for(int k = 0; k < NP; ++k) s += tab.M[i * NP + k] * q[k];
+        g[NP * cx + i] -= s;
+      }
+      g[cx ? K - 1 : 0] -= xp;
+    }
+  }
+  if constexpr(!SCALAR)
+#pragma unroll
+    for(int k = 0; k < NS / L; ++k) Ss[pl][k * K * K + t] = sv[k];
+  if(t0 < 3 * K) (&ls[pl][0][0])[t0] = lv;
+  __syncthreads();
+#pragma unroll
+  for(int i = 0; i < K; ++i) r[i] = g[i];
+  CT *B = &F1[pl][0][0];
+  if constexpr(SCALAR)
+  {
+    const CT *G0 = S_tab + size_t(f0) * K * K, *G1 = S_tab + size_t(f1) * K * K,
+             *G2 = S_tab + size_t(f2) * K * K;
+    if((eo_tab[f0] & eo_tab[f1] & eo_tab[f2]) != 0u)
+      fd_lines<3, K, CT, K, K * K, true, true>(r, o, B, G0, G1, G2, ls[0][0], ls[0][1], ls[0][2], w,
+                                               t, owner);
+    else
+      fd_lines<3, K, CT, K, K * K, false, true>(r, o, B, G0, G1, G2, ls[0][0], ls[0][1], ls[0][2], w,
+                                                t, owner);
+  }
+  else
+    fd_lines<3, K, CT>(r, o, B, Ss[pl], Ss[pl] + K * K, Ss[pl] + 2 * K * K, ls[pl][0], ls[pl][1],
+                       ls[pl][2], w, t, owner);
+  if(!valid) return;
+  VT *px = x + c_lo * NDC + lyz;
+  if(!(x_zero & kOwnZero) && w != CT(1))
+  {
+    CT old[K];
+    load_row<NP>(px, old);
+    load_row<NP>(px + NDC, old + NP);
+#pragma unroll
+    for(int a = 0; a < K; ++a) o[a] += (CT(1) - w) * old[a];
+  }
+  if(nonfinite)
+  {
+    bool bad = false;
+#pragma unroll
+    for(int a = 0; a < K; ++a) bad = bad || !__builtin_isfinite(o[a]);
+    if(bad) *nonfinite = 1;
+  }
+  store_row<NP>(px, o);
+  store_row<NP>(px + NDC, o + NP);
+}
+
+// ----------------------------------------------------------------------------
+// The 2D color pass: K lanes per patch, 64 / K patches per single-wave block.  Lane t
+// holds the x-line y = t and the points y = t of the x-faces, x = t of the y-faces; the
+// mass product along the face runs across the lanes of a cell.  Every global load of
+// the pass is issued before the first wait; the eigenvector matrices of each patch
+// are staged in LDS (padded: the patches of a wave read their copies without bank
+// conflicts).
+// Bound by launches below about 100^2 cells (4 us each, 8 per sweep), then by HBM:
+// sweeps of 16^2 Q3 FP64 34 us (68), 300^2 Q3 FP64 78 (132), FP32 53 (93), 600^2 Q1 FP64
+// 82 (123), 250^2 Q4 FP32 73 (108); in brackets staging loops and a branch and a wait
+// per neighbour.
+// ----------------------------------------------------------------------------
+template<int K, typename VT, typename CT>
+__global__ void __launch_bounds__(64)
+k_patch_mvp_2d(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<K / 2, CT> tab,
+               const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
+               const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
+               const float *__restrict__ omega, const CT relaxation, const int patch_begin,
+               const int patch_end, const int n, const int x_zero, int *__restrict__ nonfinite)
+{
+  constexpr int NP = K / 2, P = NP - 1, NDC = NP * NP, PPB = 64 / K, PS = (64 + K - 1) / K;
+  constexpr int SS = 2 * K * K + 16 / int(sizeof(CT));  // stride of a patch's matrices
+  constexpr int SY = K, SB = K * K + 16 / int(sizeof(CT));
+  __shared__ __align__(16) CT Ss[PS * SS];
+  __shared__ __align__(16) CT Bs[PS * SB];
+  __shared__ CT ls[PS][2][K];
+  const int pl = int(threadIdx.x) / K, t = int(threadIdx.x) % K;
+  const int jj = patch_begin + int(blockIdx.x) * PPB + pl;
+  const bool valid = pl < PPB && jj < patch_end;
+  const int j = valid ? jj : patch_end - 1;
+  const int c = t / NP, l = t - NP * c;
+  const uint32_t f0 = fac[size_t(j) * 2], f1 = fac[size_t(j) * 2 + 1];
+  int v[3];
+  unpack_vertex(vtx[j], v);
+  const int64_t cell0 = (v[0] - 1) + int64_t(n) * (v[1] - 1);
+  const int64_t c_lo = cell0 + int64_t(n) * c;
+  CT sv[2][K];
+#pragma unroll
+  for(int k = 0; k < K; ++k)
+  {
+    sv[0][k] = S_tab[size_t(f0) * K * K + k * K + t];
+    sv[1][k] = S_tab[size_t(f1) * K * K + k * K + t];
+  }
+  const CT lv0 = lam_tab[size_t(f0) * K + t], lv1 = lam_tab[size_t(f1) * K + t];
+  const CT w = omega ? CT(omega[j]) : relaxation;
+  CT g[K], r[K], o[K];
+  load_row<NP>(b + c_lo * NDC + NP * l, g);
+  load_row<NP>(b + (c_lo + 1) * NDC + NP * l, g + NP);
+  int ra[NP];  // ds_bpermute addresses of the rotations (NP != 4)
+#pragma unroll
+  for(int q = 0; q < NP; ++q) ra[q] = 4 * (int(threadIdx.x) - l + (l + q) % NP);
+  CT *B = Bs + pl * SB;
+
+  if(!(x_zero & kOuterZero))
+  {
+    CT nl[2][2][NP], Ma[NP];
+    const CT *tt = reinterpret_cast<const CT *>(&tab);
+    load_row<NP>(x + (v[0] > 1 ? c_lo - 1 : c_lo) * NDC + NP * l, nl[0][0]);
+    load_row<NP>(x + (v[0] + 1 < n ? c_lo + 2 : c_lo) * NDC + NP * l, nl[0][1]);
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool hy = side ? v[1] + 1 < n : v[1] > 1;
+      const VT *py = x + (cell0 + c + (hy ? (side ? 2 * n : -n) : 0)) * NDC + l;
+#pragma unroll
+      for(int k = 0; k < NP; ++k) nl[1][side][k] = py[NP * k];
+    }
+#pragma unroll
+    for(int q = 0; q < NP; ++q) Ma[q] = tt[NDC + l * NP + q];
+    const CT gy = tt[2 * NDC + NP * c + l];
+    CT fv[2], fp[2];
+#pragma unroll
+    for(int d = 0; d < 2; ++d)
+#pragma unroll
+      for(int side = 0; side < 2; ++side)
+      {
+        const bool has = side ? v[d] + 1 < n : v[d] > 1;
+        CT dv = 0, q[NP];
+#pragma unroll
+        for(int k = 0; k < NP; ++k) dv += tab.g[1 - side][k] * nl[d][side][k];
+        const CT vv = has ? nl[d][side][side ? 0 : P] : CT(0);
+        dv = has ? dv : CT(0);
+        const CT pp = (side ? CT(-0.5) : CT(0.5)) * dv - tab.sigma * vv;
+        lane_gather<NP, 0>(vv, ra, q);
+        const CT mv = dotn<NP>(Ma, q);
+        lane_gather<NP, 0>(pp, ra, q);
+        const CT mp = dotn<NP>(Ma, q);
+        if(d == 0)
+        {
+          fv[side] = mv;
+          fp[side] = mp;
+        }
+        else
+        {
+          B[side * 2 * K + t] = mv;
+          B[side * 2 * K + K + t] = mp;
+        }
+      }
+    __syncthreads();
+    const CT ey = l == (c ? P : 0) ? CT(1) : CT(0), ay = (c ? CT(0.5) : CT(-0.5)) * gy;
+    const CT *Fy = B + c * 2 * K;
+#pragma unroll
+    for(int cx = 0; cx < 2; ++cx)
+    {
+      const CT a = (cx ? CT(0.5) : CT(-0.5)) * fv[cx];
+#pragma unroll
+      for(int i = 0; i < NP; ++i)
+        g[NP * cx + i] -= a * tab.g[cx][i] + ay * Fy[NP * cx + i] + ey * Fy[K + NP * cx + i];
+      g[cx ? K - 1 : 0] -= fp[cx];
+    }
+  }
+#pragma unroll
+  for(int k = 0; k < K; ++k)
+  {
+    Ss[pl * SS + k * K + t] = sv[0][k];
+    Ss[pl * SS + K * K + k * K + t] = sv[1][k];
+  }
+  ls[pl][0][t] = lv0;
+  ls[pl][1][t] = lv1;
+  __syncthreads();  // the tables are staged, the face points are read
+#pragma unroll
+  for(int i = 0; i < K; ++i) r[i] = g[i];
+  fd_lines<2, K, CT, SY>(r, o, B, Ss + pl * SS, Ss + pl * SS + K * K, Ss + pl * SS, ls[pl][0],
+                         ls[pl][1], ls[pl][1], w, t, true);
+  if(!valid) return;
+  VT *px = x + c_lo * NDC + NP * l;
+  if(!(x_zero & kOwnZero) && w != CT(1))
+  {
+    CT old[K];
+    load_row<NP>(px, old);
+    load_row<NP>(px + NDC, old + NP);
+#pragma unroll
+    for(int a = 0; a < K; ++a) o[a] += (CT(1) - w) * old[a];
+  }
+  if(nonfinite)
+  {
     bool bad = false;
 #pragma unroll
     for(int a = 0; a < K; ++a) bad = bad || !__builtin_isfinite(o[a]);

@@ -5,7 +5,7 @@
 // thousand patches, far fewer than the GPU holds waves, and the pass takes as
 // long as one patch takes from its first load to its last store.  Spreading a
 // patch over four waves cuts the arithmetic each wave runs in sequence to a
-// quarter; the values it computes are those of k_patch_mvp_fused with full
+// quarter; the values it computes are those of k_patch_mvp_q3 with full
 // (K x K) products in every direction (the even-odd blocks are a throughput
 // device; the full products give the same result to rounding).
 //

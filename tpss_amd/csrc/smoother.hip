@@ -568,14 +568,12 @@ void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, i
       tab.Fmp[e] = CT(op.Fmp[e]);
       for(int c = 0; c < 4; ++c) tab.D[c][e] = CT(op.D[c][e]);
     }
-    using PS = PatchShape<DIM, K>;
-    const unsigned grid = unsigned((end - begin + PS::PPB - 1) / PS::PPB);
     if constexpr(FD == 1)
     {
       if constexpr(DIM == 3 && K == 8 && std::is_same<CT, float>::value)
-        hipLaunchKernelGGL((k_patch_mvp_fused<DIM, K, VT, CT, 1>), dim3(grid), dim3(PS::THREADS), 0,
-                           s, b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax,
-                           begin, end, ls.n, x_zero, sm->pass_flag);
+        hipLaunchKernelGGL((k_patch_mvp_bf16<VT>), dim3(blocks_for(end - begin, 2)), dim3(128), 0, s,
+                           b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax, begin, end, ls.n,
+                           x_zero);
       else
         throw Error(TPSS_E_UNSUPPORTED, "BF16-MFMA patch solves are built for 3D Q3 (k = 8)");
     }
@@ -591,29 +589,37 @@ void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, i
           TPSS_HIP(hipGetLastError());
           return;
         }
+      MvpTab<NP, CT> mt;
+      for(int q = 0; q < NP; ++q)
+        for(int r = 0; r < NP; ++r)
+        {
+          mt.M[q * NP + r] = CT(op.M[q * NP + r]);
+          mt.R[q * NP + r] = CT(op.M[q * NP + (q + r) % NP]);
+        }
+      for(int f = 0; f < 2; ++f)
+        for(int i = 0; i < NP; ++i) mt.g[f][i] = CT(op.g[f][i]);
+      mt.sigma = CT(op.sigma);
+      const int np = end - begin;
       if constexpr(DIM == 3 && K == 8)
       {
-        MvpTab<CT> mt;
-        for(int q = 0; q < 4; ++q)
-          for(int r = 0; r < 4; ++r)
-          {
-            mt.M[q * 4 + r] = CT(op.M[q * 4 + r]);
-            mt.R[q * 4 + r] = CT(op.M[q * 4 + (q + r) % 4]);
-          }
-        for(int f = 0; f < 2; ++f)
-          for(int i = 0; i < 4; ++i) mt.g[f][i] = CT(op.g[f][i]);
-        mt.sigma = CT(op.sigma);
         // the XCD launch order where no per-patch damping is indexed by position
         const bool xcd = om == nullptr && ls.d_vtx_launch.ptr != nullptr;
-        hipLaunchKernelGGL((k_patch_mvp_q3<VT, CT>), dim3(unsigned(end - begin)), dim3(64), 0, s, b,
-                           x, mt, xcd ? ls.d_vtx_launch.ptr : ls.d_vtx.ptr,
+        hipLaunchKernelGGL((k_patch_mvp_q3<VT, CT>), dim3(unsigned(np)), dim3(64), 0, s, b, x, mt,
+                           xcd ? ls.d_vtx_launch.ptr : ls.d_vtx.ptr,
                            xcd ? ls.d_fac_launch.ptr : ls.d_fac.ptr, S, lam, ls.d_eo.ptr, om, relax,
                            begin, ls.n, x_zero, sm->pass_flag);
       }
+      else if constexpr(DIM == 3)
+      {
+        using MS = MvpLinesShape<K>;
+        hipLaunchKernelGGL((k_patch_mvp_lines<K, VT, CT>), dim3(blocks_for(np, MS::PPB)),
+                           dim3(MS::THREADS), 0, s, b, x, mt, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam,
+                           ls.d_eo.ptr, om, relax, begin, end, ls.n, x_zero, sm->pass_flag);
+      }
       else
-        hipLaunchKernelGGL((k_patch_mvp_fused<DIM, K, VT, CT>), dim3(grid), dim3(PS::THREADS), 0, s,
-                           b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax,
-                           begin, end, ls.n, x_zero, sm->pass_flag);
+        hipLaunchKernelGGL((k_patch_mvp_2d<K, VT, CT>), dim3(blocks_for(np, 64 / K)), dim3(64), 0, s,
+                           b, x, mt, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax, begin, end, ls.n,
+                           x_zero, sm->pass_flag);
     }
     TPSS_HIP(hipGetLastError());
   });
