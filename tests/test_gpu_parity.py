@@ -510,3 +510,23 @@ def test_color_pass_block_edges(dim, p, n, vec, loc, relax):
     assert rel_err(got[:ref.N], ref.step(x0.astype(np.float64), b.astype(np.float64))) < (
         2e-5 if loc else 1e-12)
     assert (got[ref.N:] == 7.0).all()
+
+
+# patch solves with a scatter at the edges of their blocks: 128 / K^2 patches per block
+# (3D), 64 / K (2D), two blocks of threads for FP64 Q4; additive and residual-update
+# multiplicative, FP64, FP32 and FP32 solves of FP64 vectors
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 2), (2, 2, 9), (2, 3, 7), (2, 4, 8), (3, 1, 2), (3, 1, 6),
+                                     (3, 2, 3), (3, 2, 6), (3, 3, 3), (3, 3, 6), (3, 4, 2), (3, 4, 4)])
+@pytest.mark.parametrize("vec,loc", [(0, 0), (1, 1), (0, 1)])
+def test_patch_solve_block_edges(dim, p, n, vec, loc):
+    V = o.distorted_vertices(dim, n, 0.15, seed=7)
+    dt = np.float32 if vec else np.float64
+    for variant in (0, 1):
+        lv, sm, ref = make(dim, p, n, variant, ip=2.0, relaxation=0.8, vertices=V, precision=vec,
+                           local_precision=loc)
+        b = o.splitmix_uniform(6, ref.N).astype(dt)
+        d = dev(np.full(ref.N + 8, 7.0, dt), vec)  # guard values behind the output
+        sm.precond_vmult(d, dev(b, vec))
+        got = host(d)
+        assert rel_err(got[:ref.N], ref.precond_vmult(b.astype(np.float64))) < (2e-5 if loc else 1e-12)
+        assert (got[ref.N:] == 7.0).all()

@@ -825,13 +825,8 @@ k_sipg_lines_q3(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
 }
 
 // ----------------------------------------------------------------------------
-// Fused vertex-patch local solve (A2/A3/A4/A5/A12):
-//   gather r_j = R_j src  ->  u_j = S diag(omega_j / sum lambda) S^T r_j  ->
-//   MODE 0: dst += R_j^T u_j   (multiplicative color pass; same-color patches
-//                               are DoF-disjoint so the update is race free)
-//   MODE 1: U[cell, slot] = u_j (additive; summed per DoF afterwards, no atomics)
-// Thread = one line of the patch tensor; the line direction rotates through
-// LDS between the per-direction contractions.
+// Vertex patches: thread = one line of the patch tensor; the line direction rotates
+// through LDS between the per-direction contractions.
 // ----------------------------------------------------------------------------
 template<int DIM, int K>
 struct PatchShape
@@ -1159,127 +1154,223 @@ __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, cons
   bwd(S0, r, o);
 }
 
+// The same inverse with two x-lines per lane (3D): lane t of a patch's K^2 / 2 lanes
+// owns the lines (t % K, t / K) and (t % K, t / K + K / 2), so that every entry of an
+// eigenvector matrix read from LDS serves two lines (the one-line form is bound by
+// those reads).  B: entry (x, y, z) at x + K y + SZ z.
+template<int K, int SZ, typename CT>
+__device__ __forceinline__ void fd_line_pairs(CT (*r)[K], CT (*o)[K], CT *B, const CT *S,
+                                              const CT *l, const CT w, const int t)
+{
+  constexpr int H = K / 2;
+  const int ta = t % K, tb = t / K;
+  auto fwd = [&](const CT *M) {
+#pragma unroll
+    for(int i = 0; i < K; ++i)
+    {
+      CT s0 = 0, s1 = 0;
+#pragma unroll
+      for(int a = 0; a < K; ++a)
+      {
+        const CT m = M[a * K + i];
+        s0 += m * r[0][a];
+        s1 += m * r[1][a];
+      }
+      o[0][i] = s0;
+      o[1][i] = s1;
+    }
+  };
+  auto bwd = [&](const CT *M) {
+#pragma unroll
+    for(int a = 0; a < K; ++a)
+    {
+      CT s0 = 0, s1 = 0;
+#pragma unroll
+      for(int i = 0; i < K; ++i)
+      {
+        const CT m = M[a * K + i];
+        s0 += m * o[0][i];
+        s1 += m * o[1][i];
+      }
+      r[0][a] = s0;
+      r[1][a] = s1;
+    }
+  };
+  const CT *S0 = S, *S1 = S + K * K, *S2 = S + 2 * K * K;
+  fwd(S0);
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int i = 0; i < K; ++i) B[i + K * ta + SZ * (tb + h * H)] = o[h][i];
+  __syncthreads();
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int a = 0; a < K; ++a) r[h][a] = B[ta + K * a + SZ * (tb + h * H)];
+  fwd(S1);
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int a = 0; a < K; ++a) B[ta + K * a + SZ * (tb + h * H)] = o[h][a];
+  __syncthreads();
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int a = 0; a < K; ++a) r[h][a] = B[ta + K * (tb + h * H) + SZ * a];
+  fwd(S2);
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+  {
+    const CT lxy = l[ta] + l[K + tb + h * H];
+#pragma unroll
+    for(int a = 0; a < K; ++a) o[h][a] = eig_scale(o[h][a], w, lxy + l[2 * K + a]);
+  }
+  bwd(S2);
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int a = 0; a < K; ++a) B[ta + K * (tb + h * H) + SZ * a] = r[h][a];
+  __syncthreads();
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int a = 0; a < K; ++a) o[h][a] = B[ta + K * a + SZ * (tb + h * H)];
+  bwd(S1);
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int a = 0; a < K; ++a) B[ta + K * a + SZ * (tb + h * H)] = r[h][a];
+  __syncthreads();
+#pragma unroll
+  for(int h = 0; h < 2; ++h)
+#pragma unroll
+    for(int a = 0; a < K; ++a) o[h][a] = B[a + K * ta + SZ * (tb + h * H)];
+  bwd(S0);
+}
+
+// k_patch_fd: lines per lane, lanes per patch and patches per block.  3D: two lines a
+// lane in single-wave blocks, except FP64 Q4, whose 40 line values a lane leave one
+// wave per SIMD (40^3 additive step 598 us with two lines, 541 with one); 2D: one.
+template<int DIM, int K, typename CT>
+struct PatchFdShape
+{
+  static constexpr int NLN = DIM == 3 && !(K == 10 && sizeof(CT) == 8) ? 2 : 1;
+  static constexpr int LP = cpow(K, DIM - 1) / NLN;
+  static constexpr int THREADS = (LP + 63) / 64 * 64;
+  static constexpr int PPB = THREADS / LP;
+};
+
+// Fused vertex-patch local solve (A2/A3/A4/A5/A12): gather r_j = R_j src,
+// u_j = S diag(omega_j / sum lambda) S^T r_j, scatter.
+// MODE 0: dst += correction on the patches [patch_begin, patch_end) (one color: their
+// cells are disjoint), component blockIdx.y; MODE 1: the additive slot buffer.
+// Every load is issued in two batches (factor rows and vertex; tables and lines) before
+// the first wait; the matrices of each patch are staged in LDS.  Blocks of one eighth of
+// the launch run on one XCD, so that patches sharing cells mostly share its L2.
+// 3D is bound by LDS reads of the matrices and the slot buffer's traffic, 2D by latency.
+// Additive steps (patches, slot sum, check), with one line a lane, staging loops and a
+// separate check in brackets: 48^3 Q4 moved FP32 397 us (537), 64^3 Q3 FP32 338 (491),
+// FP64 713 (848), 128^2 Q3 FP64 12.5 (18.0); 64^3 elastic Q2 FP32 sweep 1697 -> 1493.
 template<int DIM, int K, typename VT, typename CT, int MODE>
-__global__ void __launch_bounds__((PatchShape<DIM, K>::THREADS))
+__global__ void __launch_bounds__((PatchFdShape<DIM, K, CT>::THREADS))
 k_patch_fd(const VT *__restrict__ src, VT *__restrict__ dst, CT *__restrict__ ubuf,
            const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
            const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
            const float *__restrict__ omega, const CT relaxation, const int patch_begin,
-           const int patch_end, const int n)
+           const int patch_end, const int n, const int64_t comp_stride, const int64_t fac_stride)
 {
-  using PS = PatchShape<DIM, K>;
-  constexpr int NP = PS::NP, L = PS::L, NPD = PS::NPD, NDC = PS::NDC, PPB = PS::PPB;
-  __shared__ CT buf[PPB][NPD];
-  __shared__ CT Ss[PPB][DIM][K * K];
-  __shared__ CT ls[PPB][DIM][K];
-
-  const int pl = threadIdx.x / L, t = threadIdx.x % L;
-  const int j0 = patch_begin + int(blockIdx.x) * PPB;
-  const int j = j0 + pl;
-  const bool valid = pl < PPB && j < patch_end;
-  const int plc = pl < PPB ? pl : 0;
-  constexpr int NT = PS::THREADS;
-
-  // Every load of the pass in three batches instead of one memory round trip
-  // per table entry and line element: the block's factor rows and this lane's
-  // vertex; the table entries this thread stages and its patch line (two cell
-  // rows of b, in MODE 0 also of dst -- the cells of a color's patches are
-  // disjoint, so no other patch of the launch writes them); then the LDS
-  // stores.  Loads are predicated, not branched, so that the compiler issues
-  // them together.
-  constexpr int NSE = PPB * DIM * K * K, NSI = (NSE + NT - 1) / NT;  // eigenvector entries
-  constexpr int NLE = PPB * DIM * K, NLI = (NLE + NT - 1) / NT;      // eigenvalues
-  uint32_t fs[NSI], fl[NLI];
-#pragma unroll
-  for(int k = 0; k < NSI; ++k)
+  using PS = PatchFdShape<DIM, K, CT>;
+  constexpr int NP = K / 2, NDC = cpow(NP, DIM), NLN = PS::NLN, LP = PS::LP, PPB = PS::PPB;
+  constexpr int SLOTS = (PS::THREADS + LP - 1) / LP;  // idle lanes included
+  constexpr int PAD = 16 / int(sizeof(CT));
+  constexpr int SM = DIM * K * K + PAD;      // strides of the patches' tables and buffers
+  constexpr int SZ = DIM == 3 && K == 8 ? 72 : K * K, SB = (DIM == 3 ? K * SZ : K * K) + PAD;
+  constexpr int NE = DIM * K * K / LP, NLAM = (DIM * K + LP - 1) / LP;
+  static_assert(NE * LP == DIM * K * K && NE % DIM == 0, "a lane stages NE / DIM entries of a matrix");
+  __shared__ __align__(16) CT Ss[SLOTS * SM];
+  __shared__ __align__(16) CT Bs[SLOTS * SB];
+  __shared__ CT ls[SLOTS][DIM * K];
+  const int pl = int(threadIdx.x) / LP, t = int(threadIdx.x) % LP;
+  const int per = int(gridDim.x) / 8;  // the grid is a multiple of eight blocks
+  const int blk = int(blockIdx.x % 8) * per + int(blockIdx.x) / 8;
+  const int64_t jj = patch_begin + int64_t(blk) * PPB + pl;
+  const bool valid = pl < PPB && jj < patch_end;
+  const int j = valid ? int(jj) : patch_begin;
+  if(MODE == 0)
   {
-    const int idx = int(threadIdx.x) + k * NT;
-    const int q = idx / (DIM * K * K), d = (idx % (DIM * K * K)) / (K * K);
-    const bool ok = idx < NSE && j0 + q < patch_end;
-    fs[k] = fac[size_t(ok ? j0 + q : patch_begin) * DIM + (ok ? d : 0)];
+    src += blockIdx.y * comp_stride;
+    dst += blockIdx.y * comp_stride;
+    fac += blockIdx.y * fac_stride;
   }
+  uint32_t f[DIM];
 #pragma unroll
-  for(int k = 0; k < NLI; ++k)
-  {
-    const int idx = int(threadIdx.x) + k * NT;
-    const int q = idx / (DIM * K), d = (idx % (DIM * K)) / K;
-    const bool ok = idx < NLE && j0 + q < patch_end;
-    fl[k] = fac[size_t(ok ? j0 + q : patch_begin) * DIM + (ok ? d : 0)];
-  }
+  for(int d = 0; d < DIM; ++d) f[d] = fac[size_t(j) * DIM + d];
   int v[3] = {1, 1, 1};
-  unpack_vertex(vtx[valid ? j : patch_begin], v);
-  const CT w = valid ? (omega ? CT(omega[j]) : relaxation) : CT(0);
-
-  auto cell_of = [&](int i0, int i1, int i2) { return patch_cell<DIM, NP>(v, n, i0, i1, i2); };
-  auto loc_of = [&](int i0, int i1, int i2) { return patch_local<DIM, NP>(i0, i1, i2); };
-  auto slot_of = [&](int i0, int i1, int i2) { return patch_slot<DIM, NP>(i0, i1, i2); };
-
-  CT sv[NSI], lv[NLI];
+  unpack_vertex(vtx[j], v);
+  const CT w = omega ? CT(omega[j]) : relaxation;
+  CT sv[NE], lv[NLAM];
 #pragma unroll
-  for(int k = 0; k < NSI; ++k)
-  {
-    const int idx = int(threadIdx.x) + k * NT;
-    sv[k] = S_tab[size_t(fs[k]) * K * K + idx % (K * K)];
-  }
+  for(int k = 0; k < NE; ++k)
+    sv[k] = S_tab[size_t(f[k / (NE / DIM)]) * K * K + (k % (NE / DIM)) * LP + t];
 #pragma unroll
-  for(int k = 0; k < NLI; ++k)
+  for(int k = 0; k < NLAM; ++k)
   {
-    const int idx = int(threadIdx.x) + k * NT;
-    lv[k] = lam_tab[size_t(fl[k]) * K + idx % K];
+    const int e = t + k * LP, d = e < K ? 0 : e < 2 * K ? 1 : DIM - 1;
+    lv[k] = e < DIM * K ? lam_tab[size_t(d == 0 ? f[0] : d == 1 ? f[1] : f[DIM - 1]) * K + e % K] : CT(1);
   }
-  // this thread's x-line (ty, tz) of the patch: row lyz of the cells c_lo, c_lo + 1
-  const int ty = DIM > 1 ? t % K : 0;
-  const int tz = DIM > 2 ? t / K : 0;
-  const int64_t c_lo = cell_of(0, ty, tz);
-  const int lyz = loc_of(0, ty, tz);
-  CT r[K], o[K], old[K];
-  load_row<NP>(src + c_lo * NDC + lyz, r);
-  load_row<NP>(src + (c_lo + 1) * NDC + lyz, r + NP);
-  if constexpr(MODE == 0)
-  {
-    load_row<NP>(dst + c_lo * NDC + lyz, old);
-    load_row<NP>(dst + (c_lo + 1) * NDC + lyz, old + NP);
-  }
+  // the lane's lines: rows of the cells c_lo and c_lo + 1
+  CT r[NLN][K], o[NLN][K], old[NLN][K];
+  int64_t c_lo[NLN];
+  int lyz[NLN];
 #pragma unroll
-  for(int k = 0; k < NSI; ++k)
+  for(int h = 0; h < NLN; ++h)
   {
-    const int idx = int(threadIdx.x) + k * NT;
-    const int q = idx / (DIM * K * K), rr = idx % (DIM * K * K);
-    const bool ok = idx < NSE;
-    if(ok) Ss[q][rr / (K * K)][rr % (K * K)] = j0 + q < patch_end ? sv[k] : CT(0);
+    const int ty = t % K, tz = DIM == 3 ? t / K + h * (K / 2) : 0;
+    c_lo[h] = patch_cell<DIM, NP>(v, n, 0, ty, tz);
+    lyz[h] = patch_local<DIM, NP>(0, ty, tz);
+    load_row<NP>(src + c_lo[h] * NDC + lyz[h], r[h]);
+    load_row<NP>(src + (c_lo[h] + 1) * NDC + lyz[h], r[h] + NP);
+    if constexpr(MODE == 0)
+    {
+      load_row<NP>(dst + c_lo[h] * NDC + lyz[h], old[h]);
+      load_row<NP>(dst + (c_lo[h] + 1) * NDC + lyz[h], old[h] + NP);
+    }
   }
+  CT *S = Ss + pl * SM, *B = Bs + pl * SB, *l = ls[pl];
 #pragma unroll
-  for(int k = 0; k < NLI; ++k)
-  {
-    const int idx = int(threadIdx.x) + k * NT;
-    const int q = idx / (DIM * K), rr = idx % (DIM * K);
-    if(idx < NLE) ls[q][rr / K][rr % K] = j0 + q < patch_end ? lv[k] : CT(1);
-  }
-  if(!valid)
+  for(int k = 0; k < NE; ++k) S[k * LP + t] = sv[k];
 #pragma unroll
-    for(int i = 0; i < K; ++i) r[i] = CT(0);
+  for(int k = 0; k < NLAM; ++k)
+    if(t + k * LP < DIM * K) l[t + k * LP] = lv[k];
   __syncthreads();
-
-  const CT *S0 = Ss[plc][0];
-  const CT *S1 = Ss[plc][1];
-  const CT *S2 = Ss[plc][DIM > 2 ? 2 : 1];
-  CT *B = buf[plc];
-
-  fd_lines<DIM, K, CT>(r, o, B, S0, S1, S2, ls[plc][0], ls[plc][1], ls[plc][DIM > 2 ? 2 : 1], w,
-                       t, pl < PPB);
-  if(!valid) return;
-  if constexpr(MODE == 0)
+  if constexpr(NLN == 2)
   {
+    fd_line_pairs<K, SZ>(r, o, B, S, l, w, t);
 #pragma unroll
-    for(int a = 0; a < K; ++a) o[a] += old[a];
-    store_row<NP>(dst + c_lo * NDC + lyz, o);
-    store_row<NP>(dst + (c_lo + 1) * NDC + lyz, o + NP);
+    for(int h = 0; h < NLN; ++h)
+#pragma unroll
+      for(int a = 0; a < K; ++a) o[h][a] = r[h][a];
   }
   else
+    fd_lines<DIM, K, CT>(r[0], o[0], B, S, S + K * K, S + (DIM - 1) * K * K, l, l + K,
+                         l + (DIM - 1) * K, w, t, true);
+  if(!valid) return;
+#pragma unroll
+  for(int h = 0; h < NLN; ++h)
   {
-    const int s0 = slot_of(0, ty, tz);
-    store_row<NP>(ubuf + (c_lo * (1 << DIM) + s0) * NDC + lyz, o);
-    store_row<NP>(ubuf + ((c_lo + 1) * (1 << DIM) + (s0 | 1)) * NDC + lyz, o + NP);
+    if constexpr(MODE == 0)
+    {
+#pragma unroll
+      for(int a = 0; a < K; ++a) o[h][a] += old[h][a];
+      store_row<NP>(dst + c_lo[h] * NDC + lyz[h], o[h]);
+      store_row<NP>(dst + (c_lo[h] + 1) * NDC + lyz[h], o[h] + NP);
+    }
+    else
+    {
+      const int s0 = patch_slot<DIM, NP>(0, t % K, DIM == 3 ? t / K + h * (K / 2) : 0);
+      store_row<NP>(ubuf + (c_lo[h] * (1 << DIM) + s0) * NDC + lyz[h], o[h]);
+      store_row<NP>(ubuf + ((c_lo[h] + 1) * (1 << DIM) + (s0 | 1)) * NDC + lyz[h], o[h] + NP);
+    }
   }
 }
 
@@ -1327,16 +1418,17 @@ __device__ __forceinline__ int ras_owner_slot(const int *c, const int *l, const 
 // the number of those patches (use_ras_weights, schwarz_preconditioner.templates.h:
 // 636-641); RAS = 2: only the contribution of the patch that keeps the DoF
 // (use_ras_boolean_weights, rscatter_add, :646-649).
+// One x-row of a cell per thread; a non-finite result sets *nonfinite (if given).
 template<int DIM, int NP, typename VT, typename CT, bool ACCUMULATE, int RAS = 0>
 __global__ void __launch_bounds__(256)
-k_avp_sum(const CT *__restrict__ ubuf, VT *__restrict__ dst, const int n, const int64_t N,
-          const double alpha)
+k_avp_sum(const CT *__restrict__ ubuf, VT *__restrict__ dst, const int n, const int64_t rows,
+          const double alpha, int *__restrict__ nonfinite)
 {
-  constexpr int NDC = cpow(NP, DIM);
+  constexpr int NDC = cpow(NP, DIM), NR = NDC / NP;
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if(i >= N) return;
-  const int64_t cell = i / NDC;
-  const int l = int(i % NDC);
+  if(i >= rows) return;
+  const int64_t cell = i / NR;
+  const int row = int(i - cell * NR), l = row * NP;
   int c[3] = {0, 0, 0};
   {
     int t = int(cell);  // cells < 2^24
@@ -1346,17 +1438,21 @@ k_avp_sum(const CT *__restrict__ ubuf, VT *__restrict__ dst, const int n, const 
       t /= n;
     }
   }
-  CT s = 0;
+  const CT *u = ubuf + cell * (1 << DIM) * NDC + l;
+  CT s[NP];
   if constexpr(RAS == 2)
   {
-    int lm[3] = {0, 0, 0};
-    for(int d = 0, t = l; d < DIM; ++d, t /= NP) lm[d] = t % NP;
-    const int slot = ras_owner_slot<DIM, NP>(c, lm, n);
-    s = ubuf[(cell * (1 << DIM) + slot) * NDC + l];
+#pragma unroll
+    for(int k = 0; k < NP; ++k)
+    {
+      const int lm[3] = {k, row % NP, row / NP};
+      s[k] = u[ras_owner_slot<DIM, NP>(c, lm, n) * NDC + k];
+    }
   }
   else
   {
     int count = 0;
+    CT q[1 << DIM][NP];
 #pragma unroll
     for(int slot = 0; slot < (1 << DIM); ++slot)
     {
@@ -1367,18 +1463,35 @@ k_avp_sum(const CT *__restrict__ ubuf, VT *__restrict__ dst, const int n, const 
         const int vd = c[d] + 1 - ((slot >> d) & 1);
         ok = ok && vd >= 1 && vd <= n - 1;
       }
+#pragma unroll
+      for(int k = 0; k < NP; ++k) q[slot][k] = CT(0);
       if(ok)
       {
-        s += ubuf[(cell * (1 << DIM) + slot) * NDC + l];
+        load_row<NP>(u + slot * NDC, q[slot]);
         ++count;
       }
     }
-    if constexpr(RAS == 1) s /= CT(count);
+#pragma unroll
+    for(int k = 0; k < NP; ++k)
+    {
+      s[k] = q[0][k];
+#pragma unroll
+      for(int slot = 1; slot < (1 << DIM); ++slot) s[k] += q[slot][k];
+      if constexpr(RAS == 1) s[k] /= CT(count);
+    }
   }
-  if(ACCUMULATE)
-    dst[i] = VT(double(dst[i]) + alpha * double(s));
-  else
-    dst[i] = VT(alpha * double(s));
+  VT out[NP];
+  VT *pd = dst + i * NP;
+  if constexpr(ACCUMULATE) load_row<NP>(pd, out);
+  bool bad = false;
+#pragma unroll
+  for(int k = 0; k < NP; ++k)
+  {
+    out[k] = ACCUMULATE ? VT(double(out[k]) + alpha * double(s[k])) : VT(alpha * double(s[k]));
+    bad = bad || !isfinite(out[k]);
+  }
+  store_row<NP>(pd, out);
+  if(nonfinite && bad) *nonfinite = 1;
 }
 
 // restricted-DoF flags of every patch (DoFInfo::restricted_dof_flags_patchwise,

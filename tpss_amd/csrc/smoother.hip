@@ -503,19 +503,16 @@ std::shared_ptr<LocalSolvers> build_local_solvers(const tpss_level *lv,
 
 // ---------------------------------------------------------------------------- apply
 
-// one launch over the patches [begin, end) of component block comp: gather,
-// fast-diagonalization inverse, damping, scatter (mode 0: scatter-add into dst;
-// mode 1: write the additive slot buffer)
+// one launch over the patches [begin, end): gather, fast-diagonalization inverse,
+// damping, scatter (mode 0: scatter-add into dst, all component blocks; mode 1: write
+// the additive slot buffer of component block comp)
 template<typename VT, typename CT>
 void patch_pass(tpss_smoother *sm, const VT *src, VT *dst, CT *ubuf, int begin, int end, int mode,
                 hipStream_t s, int comp = 0)
 {
   const LocalSolvers &ls = *sm->ls;
   if(end <= begin) return;
-  const int64_t off = comp * sm->level->Ns;
-  src += off;
-  if(dst) dst += off;
-  const uint32_t *fac = ls.d_fac.ptr + size_t(comp) * ls.P * ls.dim;
+  const int64_t Ns = sm->level->Ns, fac_stride = int64_t(ls.P) * ls.dim;
   const CT *S = std::is_same<CT, double>::value ? (const CT *)ls.S64.ptr : (const CT *)ls.S32.ptr;
   const CT *lam =
     std::is_same<CT, double>::value ? (const CT *)ls.lam64.ptr : (const CT *)ls.lam32.ptr;
@@ -523,15 +520,17 @@ void patch_pass(tpss_smoother *sm, const VT *src, VT *dst, CT *ubuf, int begin, 
   const CT relax = CT(sm->desc.relaxation);
   dispatch_dim_np(ls.dim, ls.np, [&](auto D, auto NPc) {
     constexpr int DIM = decltype(D)::value, NP = decltype(NPc)::value, K = 2 * NP;
-    using PS = PatchShape<DIM, K>;
-    const unsigned grid = unsigned((end - begin + PS::PPB - 1) / PS::PPB);
-    const unsigned threads = unsigned(PS::THREADS);
+    // eight equal shares of blocks, one per XCD
+    using FS = PatchFdShape<DIM, K, CT>;
+    const unsigned grid = (blocks_for(end - begin, FS::PPB) + 7) / 8 * 8;
     if(mode == 0)
-      hipLaunchKernelGGL((k_patch_fd<DIM, K, VT, CT, 0>), dim3(grid), dim3(threads), 0, s, src,
-                         dst, ubuf, ls.d_vtx.ptr, fac, S, lam, om, relax, begin, end, ls.n);
+      hipLaunchKernelGGL((k_patch_fd<DIM, K, VT, CT, 0>), dim3(grid, unsigned(ls.ncomp)),
+                         dim3(FS::THREADS), 0, s, src, dst, ubuf, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax, begin,
+                         end, ls.n, Ns, fac_stride);
     else
-      hipLaunchKernelGGL((k_patch_fd<DIM, K, VT, CT, 1>), dim3(grid), dim3(threads), 0, s, src,
-                         dst, ubuf, ls.d_vtx.ptr, fac, S, lam, om, relax, begin, end, ls.n);
+      hipLaunchKernelGGL((k_patch_fd<DIM, K, VT, CT, 1>), dim3(grid), dim3(FS::THREADS), 0, s,
+                         src + comp * Ns, dst, ubuf, ls.d_vtx.ptr, ls.d_fac.ptr + comp * fac_stride,
+                         S, lam, om, relax, begin, end, ls.n, Ns, fac_stride);
     TPSS_HIP(hipGetLastError());
   });
 }
@@ -633,11 +632,12 @@ void avp_sum(tpss_smoother *sm, const CT *ubuf, VT *dst, bool accumulate, double
   dst += comp * lv->Ns;
   dispatch_dim_np(lv->dim, lv->np, [&](auto D, auto NPc) {
     constexpr int DIM = decltype(D)::value, NP = decltype(NPc)::value;
-    const unsigned g = blocks_for(lv->Ns, 256);
+    const int64_t rows = lv->Ns / NP;
+    const unsigned g = blocks_for(rows, 256);
     auto launch = [&](auto ACC, auto RASc) {
       hipLaunchKernelGGL((k_avp_sum<DIM, NP, VT, CT, decltype(ACC)::value != 0,
                                     decltype(RASc)::value>),
-                         dim3(g), dim3(256), 0, s, ubuf, dst, lv->n, lv->Ns, alpha);
+                         dim3(g), dim3(256), 0, s, ubuf, dst, lv->n, rows, alpha, sm->pass_flag);
     };
     const int ras = sm->desc.ras;
     if(accumulate)
@@ -749,6 +749,7 @@ void precond_vmult_t(tpss_smoother *sm, VT *dst, const VT *src, hipStream_t s, b
         avp_sum<VT, CT>(sm, ub, dst, accumulate, accumulate ? alpha : 1.0, s, c);
       }
     }
+    if(sm->pass_flag) sm->pass_checked = true;  // every value of dst has been checked
     return;
   }
   // multiplicative: colors in sequence, localized residual before each color
@@ -792,8 +793,7 @@ void precond_vmult_t(tpss_smoother *sm, VT *dst, const VT *src, hipStream_t s, b
       r = res;
     }
     SectionTimer t(sm, 1, s);
-    for(int comp = 0; comp < ls.ncomp; ++comp)
-      patch_pass<VT, CT>(sm, r, out, nullptr, ls.color_ptr[c], ls.color_ptr[c + 1], 0, s, comp);
+    patch_pass<VT, CT>(sm, r, out, nullptr, ls.color_ptr[c], ls.color_ptr[c + 1], 0, s);
   }
   if(accumulate) axpby(dst, out, lv->vec_prec, lv->N, alpha, 1.0, s);
 }
@@ -990,8 +990,8 @@ void smoother_step_any(tpss_smoother *sm, void *dst, const void *src, hipStream_
       operator_apply_any(lv, sm->rich_r.ptr, dst, src, nullptr, 0, s);
       r = sm->rich_r.ptr;
     }
+    sm->pass_checked = false;  // a correction follows the values checked so far
     precond_vmult_any(sm, dst, r, s, true, sm->desc.damping_factor);
-    sm->pass_checked = false;  // a correction was added to the checked values
   }
 }
 
