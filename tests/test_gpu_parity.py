@@ -530,3 +530,29 @@ def test_patch_solve_block_edges(dim, p, n, vec, loc):
         got = host(d)
         assert rel_err(got[:ref.N], ref.precond_vmult(b.astype(np.float64))) < (2e-5 if loc else 1e-12)
         assert (got[ref.N:] == 7.0).all()
+
+
+# cells per block: 64 / (p+1)^(dim-1); last blocks with one cell, full ones, fewer cells
+# than a block, cells with boundary faces on both sides of a direction; all cells and
+# (tiled colors, whose sweep updates the residual color by color) lists of them
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 2), (2, 1, 9), (2, 2, 5), (2, 3, 8), (2, 4, 7), (3, 1, 2),
+                                     (3, 1, 5), (3, 2, 2), (3, 2, 6), (3, 3, 5), (3, 4, 2), (3, 4, 5)])
+def test_cartesian_operator_block_edges(dim, p, n):
+    t = _tpss()
+    ref = o.Smoother(dim, p, n, ip=2.0)
+    x, b = o.splitmix_uniform(3, ref.N), o.splitmix_uniform(4, ref.N)
+    for prec, dt, bar in ((t.F64, np.float64, 1e-12), (t.F32, np.float32, 1e-6)):
+        lv = t.Level(dim, p, n, ip_factor=2.0, precision=prec)
+        xs, bs = x.astype(dt), b.astype(dt)
+        Ax = ref.operator(xs.astype(np.float64))
+        y = dev(np.full(ref.N + 8, 7.0, dt), prec)  # guard values behind the output
+        lv.vmult(y, dev(xs, prec))
+        assert rel_err(host(y)[:ref.N], Ax) < bar
+        assert (host(y)[ref.N:] == 7.0).all()
+        lv.residual(y, dev(bs, prec), dev(xs, prec))
+        assert rel_err(host(y)[:ref.N], bs - Ax) < bar
+        _, sm, rs = make(dim, p, n, 1, coloring=t.COLOR_TILED, ip=2.0, precision=prec,
+                         local_precision=prec)
+        d = dev(np.zeros(ref.N, dt), prec)
+        sm.precond_vmult(d, dev(bs, prec))
+        assert rel_err(host(d), rs.precond_vmult(bs.astype(np.float64))) < (1e-12 if prec == t.F64 else 2e-5)

@@ -188,6 +188,7 @@ Operator1D make_operator_1d(int p, double h, double ip)
       // Dirichlet faces, ghost value -u (apps/laplace_integrator.h:715-739)
       Bl[ij] = sig_b * vi0 * vj0 + vi0 * gj0 + gi0 * vj0;
       Br[ij] = sig_b * vi1 * vj1 - vi1 * gj1 - gi1 * vj1;
+      op.L[ij] = l + 0.5 * (vi0 * gj0 + gi0 * vj0) - 0.5 * (vi1 * gj1 + gi1 * vj1);
     }
   for(int c = 0; c < 4; ++c)
   {

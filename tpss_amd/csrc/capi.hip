@@ -39,11 +39,19 @@ OpTab<T, NP> make_optab(const Operator1D &op)
   return t;
 }
 
-template<int DIM, int NP>
-constexpr int cells_per_block()
+template<typename T, int NP>
+LineTab<NP, T> make_line_tab(const Operator1D &op)
 {
-  constexpr int ndc = cpow(NP, DIM);
-  return ndc >= 256 ? 1 : 256 / ndc;
+  LineTab<NP, T> t;
+  for(int e = 0; e < NP * NP; ++e)
+  {
+    t.M[e] = T(op.M[e]);
+    t.L[e] = T(op.L[e]);
+  }
+  for(int f = 0; f < 2; ++f)
+    for(int i = 0; i < NP; ++i) t.g[f][i] = T(op.g[f][i]);
+  t.sigma = T(op.sigma);
+  return t;
 }
 
 // the 1D matrices of k_elasticity, formed in FP64
@@ -171,59 +179,32 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
   }
   dispatch_dim_np(lv->dim, lv->np, [&](auto D, auto NPc) {
     constexpr int DIM = decltype(D)::value, NP = decltype(NPc)::value;
-    using CT = VT;
-    const auto tab = make_optab<CT, NP>(lv->op1d);
     if(cells && n_list == 0) return;
-    if(cells)
-    {
-      // only the listed cells (the cells a multiplicative color reads)
-      constexpr int CPB = cells_per_block<DIM, NP>();
-      constexpr int NDC = cpow(NP, DIM);
-      const unsigned grid = blocks_for(n_list, CPB);
-      const unsigned threads = unsigned(((CPB * NDC + 63) / 64) * 64);
-      if(b)
-        hipLaunchKernelGGL((k_sipg_cartesian<DIM, NP, VT, CT, CPB, true>), dim3(grid),
-                           dim3(threads), 0, s, x, y, b, tab, lv->n, lv->ncell, cells, n_list);
-      else
-        hipLaunchKernelGGL((k_sipg_cartesian<DIM, NP, VT, CT, CPB, false>), dim3(grid),
-                           dim3(threads), 0, s, x, y, b, tab, lv->n, lv->ncell, cells, n_list);
-      TPSS_HIP(hipGetLastError());
-      return;
-    }
+    // all cells of a 3D Q3 level: the wave-wide row form; anything else a lane per line
     if constexpr(DIM == 3 && NP == 4)
-    {
-      const unsigned grid = blocks_for(lv->ncell, 16);
-      if(b)
-        hipLaunchKernelGGL((k_sipg_lines_q3<VT, CT, true>), dim3(grid), dim3(256), 0, s, x, y, b,
-                           tab, lv->n, lv->ncell);
-      else
-        hipLaunchKernelGGL((k_sipg_lines_q3<VT, CT, false>), dim3(grid), dim3(256), 0, s, x, y,
-                           b, tab, lv->n, lv->ncell);
-      TPSS_HIP(hipGetLastError());
-      return;
-    }
-    if constexpr(DIM == 3)
-    {
-      constexpr int CPB = lines_cells_per_block<NP>();
-      const unsigned grid = blocks_for(lv->ncell, CPB);
-      if(b)
-        hipLaunchKernelGGL((k_sipg_lines<NP, VT, CT, true>), dim3(grid), dim3(256), 0, s, x, y, b,
-                           tab, lv->n, lv->ncell);
-      else
-        hipLaunchKernelGGL((k_sipg_lines<NP, VT, CT, false>), dim3(grid), dim3(256), 0, s, x, y,
-                           b, tab, lv->n, lv->ncell);
-      TPSS_HIP(hipGetLastError());
-      return;
-    }
-    constexpr int TX = row_tile<DIM, NP>();
-    const int64_t rows = DIM == 3 ? int64_t(lv->n) * lv->n : lv->n;
-    const unsigned grid = unsigned(rows * ((lv->n + TX - 1) / TX));
+      if(!cells)
+      {
+        const auto tab = make_optab<VT, NP>(lv->op1d);
+        const unsigned grid = blocks_for(lv->ncell, 16);
+        if(b)
+          hipLaunchKernelGGL((k_sipg_lines_q3<VT, VT, true>), dim3(grid), dim3(256), 0, s, x, y, b,
+                             tab, lv->n, lv->ncell);
+        else
+          hipLaunchKernelGGL((k_sipg_lines_q3<VT, VT, false>), dim3(grid), dim3(256), 0, s, x, y, b,
+                             tab, lv->n, lv->ncell);
+        TPSS_HIP(hipGetLastError());
+        return;
+      }
+    // eight equal shares of blocks, one per XCD
+    const auto tab = make_line_tab<VT, NP>(lv->op1d);
+    const int64_t count = cells ? n_list : lv->ncell;
+    const unsigned grid = (blocks_for(count, line_cells_per_block<DIM, NP>()) + 7) / 8 * 8;
     if(b)
-      hipLaunchKernelGGL((k_sipg_rows<DIM, NP, VT, CT, true>), dim3(grid), dim3(256), 0, s, x, y, b,
-                         tab, lv->n);
+      hipLaunchKernelGGL((k_sipg_cells<DIM, NP, VT, true>), dim3(grid), dim3(64), 0, s, x, y, b, tab,
+                         lv->n, cells, count);
     else
-      hipLaunchKernelGGL((k_sipg_rows<DIM, NP, VT, CT, false>), dim3(grid), dim3(256), 0, s, x, y,
-                         b, tab, lv->n);
+      hipLaunchKernelGGL((k_sipg_cells<DIM, NP, VT, false>), dim3(grid), dim3(64), 0, s, x, y, b, tab,
+                         lv->n, cells, count);
     TPSS_HIP(hipGetLastError());
   });
 }

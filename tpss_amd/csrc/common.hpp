@@ -146,6 +146,7 @@ struct Operator1D
   double Fmp[MAXNP * MAXNP];    // coupling to the right neighbour
   double g[2][MAXNP];           // phi_i'(0) / h, phi_i'(1) / h
   double sigma;                 // penalty of an interior face
+  double L[MAXNP * MAXNP];      // stiffness and the cell's half of the consistency terms
 };
 Operator1D make_operator_1d(int p, double h, double ip);
 

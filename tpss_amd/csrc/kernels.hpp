@@ -24,7 +24,6 @@ constexpr __host__ __device__ int cpow(int b, int e) { return e == 0 ? 1 : b * c
 // tensor-product cells): per cell and direction d the 1D line operator
 //   z = D_d x_c + F_pm x_{c-e_d} + F_mp x_{c+e_d}   (along d)
 // followed by the cell mass along every other direction, summed over d.
-// One thread per cell DoF, CPB cells per block, lines staged in LDS.
 // ----------------------------------------------------------------------------
 template<typename T, int NP>
 struct OpTab
@@ -192,439 +191,300 @@ __device__ __forceinline__ T dotn(const T *a, const T *b)
   return s;
 }
 
-template<int DIM, int NP, typename VT, typename CT, int CPB, bool RESIDUAL>
-__global__ void __launch_bounds__(256)
-k_sipg_cartesian(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
-                 const OpTab<CT, NP> tab, const int n, const int64_t ncell,
-                 const uint32_t *__restrict__ cells, const int64_t n_list)
+// Rows of N values moved through LDS in 16-byte chunks: chunk k of the row of lane
+// l sits at (k * LANES + l), so that the lanes' accesses are free of bank conflicts.
+template<int N, int LANES, typename T>
+struct LaneRows
 {
-  constexpr int NDC = cpow(NP, DIM);
-  __shared__ CT xs[CPB][NDC];
-  __shared__ CT zs[CPB][NDC];
-  const int cs = threadIdx.x / NDC, li = threadIdx.x % NDC;
-  const int64_t slot = int64_t(blockIdx.x) * CPB + cs;
-  const int64_t count = cells ? n_list : ncell;
-  const bool active = cs < CPB && slot < count;
-  const int64_t cell = active ? (cells ? int64_t(cells[slot]) : slot) : 0;
-  const int csafe = cs < CPB ? cs : 0;
-
-  int lid[DIM], cid[DIM];
+  static constexpr int CW = 16 / int(sizeof(T)), NC = (N + CW - 1) / CW;
+  static constexpr int SIZE = NC * LANES * CW;
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  static __device__ __forceinline__ void put(T *buf, int lane, const T *v)
   {
-    int t = li;
-    int c = int(cell);  // cells < n^3 <= 1000^3 < 2^31
-    for(int d = 0; d < DIM; ++d)
+#pragma unroll
+    for(int k = 0; k < NC; ++k)
     {
-      lid[d] = t % NP;
-      t /= NP;
-      cid[d] = c % n;
-      c /= n;
+      vec w;
+#pragma unroll
+      for(int e = 0; e < CW; ++e) w[e] = k * CW + e < N ? v[k * CW + e] : T(0);
+      reinterpret_cast<vec *>(buf)[k * LANES + lane] = w;
     }
   }
-  if(cs < CPB) xs[cs][li] = active ? CT(x[cell * NDC + li]) : CT(0);
-  __syncthreads();
-
-  CT acc = 0;
-  int64_t cstride = 1;
-  int lstride = 1;
-#pragma unroll
-  for(int d = 0; d < DIM; ++d)
+  static __device__ __forceinline__ void get(const T *buf, int lane, T *v)
   {
-    const bool has_l = cid[d] > 0, has_r = cid[d] < n - 1;
-    const CT *D = tab.D[(has_l ? 1 : 0) | (has_r ? 2 : 0)];
-    const int i = lid[d];
-    const int base = li - i * lstride;
-    CT z = 0;
 #pragma unroll
-    for(int j = 0; j < NP; ++j) z += D[i * NP + j] * xs[csafe][base + j * lstride];
-    if(active && has_l)
+    for(int k = 0; k < NC; ++k)
     {
-      const VT *xl = x + (cell - cstride) * NDC + base;
+      const vec w = reinterpret_cast<const vec *>(buf)[k * LANES + lane];
 #pragma unroll
-      for(int j = 0; j < NP; ++j) z += tab.Fpm[i * NP + j] * CT(xl[j * lstride]);
+      for(int e = 0; e < CW; ++e)
+        if(k * CW + e < N) v[k * CW + e] = w[e];
     }
-    if(active && has_r)
-    {
-      const VT *xr = x + (cell + cstride) * NDC + base;
-#pragma unroll
-      for(int j = 0; j < NP; ++j) z += tab.Fmp[i * NP + j] * CT(xr[j * lstride]);
-    }
-    int estride = 1;
-#pragma unroll
-    for(int e = 0; e < DIM; ++e)
-    {
-      if(e != d)
-      {
-        __syncthreads();
-        if(cs < CPB) zs[cs][li] = z;
-        __syncthreads();
-        const int ie = lid[e];
-        const int be = li - ie * estride;
-        CT w = 0;
-#pragma unroll
-        for(int j = 0; j < NP; ++j) w += tab.M[ie * NP + j] * zs[csafe][be + j * estride];
-        z = w;
-      }
-      estride *= NP;
-    }
-    acc += z;
-    cstride *= n;
-    lstride *= NP;
   }
-  if(active)
-  {
-    if(RESIDUAL)
-      y[cell * NDC + li] = VT(CT(b[cell * NDC + li]) - acc);
-    else
-      y[cell * NDC + li] = VT(acc);
-  }
-}
+};
 
-// Row-tiled variant: a block owns TX consecutive cells of one x-row and stages
-// that row (with its two x-halo cells) and the four neighbouring rows (+-y,
-// +-z) in LDS with contiguous loads.  With all neighbours local the operator is
-// evaluated in sum-factorised form
-//   y = M_z (M_y z_0 + M_x z_1) + M_y M_x z_2    (3D)
-//   y = M_y z_0 + M_x z_1                        (2D)
-// where z_d is the 1D line operator along d (own cell + face neighbours).
+// ----------------------------------------------------------------------------
+// The operator with a lane per x-line, any cells.  The face terms have rank two per
+// line: with a neighbour line's trace (v, v') on the face (node value, Gauss-Lobatto
+// nodes; one NP-term product), s = +1 on the left face, -1 on the right one, and the
+// cell's own value u there,
+//   y += (e_i P - s/2 g_i v) M M,  P = sigma (u - v) + s/2 v'
+// beside the cell's own matrix L (stiffness and its half of the consistency terms); a
+// boundary face takes the odd reflection of the cell as its neighbour.  The x
+// products run in registers; the y products read the cell's lines from LDS, each
+// extended by its x-face traces; two rows per lane pass through LDS for the z
+// products.  The y- and z-face traces are formed by lanes that own a tangential point
+// (the z-face ones contracted along y there).  Blocks of one eighth of the launch run
+// on one XCD, so that neighbours in y and z are mostly found in its L2.
+// Bound by LDS and instruction issue.  In brackets the forms with a thread per node or
+// the neighbour planes' rows in every lane: 33^3 Q2 FP64 residual 9.8 us (12.7), 64^3 Q2
+// FP64 46 (61), 40^3 Q4 FP64 71 (137), 100^3 Q1 FP32 32 (40), 500^2 Q3 FP64 16 (42), 300^2
+// Q4 FP32 9 (25).
+// ----------------------------------------------------------------------------
+template<int NP, typename T>
+struct LineTab
+{
+  T M[NP * NP], L[NP * NP];
+  T g[2][NP];  // phi_i'(0) / h, phi_i'(1) / h
+  T sigma;
+};
+
 template<int DIM, int NP>
-constexpr int row_tile()
+constexpr int line_cells_per_block()
 {
-  return cpow(NP, DIM) >= 256 ? 1 : 256 / cpow(NP, DIM);
+  return 64 / cpow(NP, DIM - 1);
 }
 
-template<int DIM, int NP, typename VT, typename CT, bool RESIDUAL>
-__global__ void __launch_bounds__(256)
-k_sipg_rows(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
-            const OpTab<CT, NP> tab, const int n)
+template<int DIM, int NP, typename VT, bool RESIDUAL>
+__global__ void __launch_bounds__(64)
+k_sipg_cells(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
+             const LineTab<NP, VT> tab, const int n, const uint32_t *__restrict__ cells,
+             const int64_t count)
 {
-  constexpr int NDC = cpow(NP, DIM);
-  constexpr int TX = row_tile<DIM, NP>();
-  constexpr int NROW = 2 * DIM - 1;  // own row + (2 DIM - 2) neighbour rows
-  constexpr int TXH = TX + 2;
-  __shared__ CT xs[NROW][TXH][NDC];
-  __shared__ CT zs[DIM][TX][NDC];
-  __shared__ CT as[2][TX][NDC];
+  using T = VT;
+  constexpr bool D3 = DIM == 3;
+  constexpr int NL = cpow(NP, DIM - 1), NDC = NL * NP, P = NP - 1;
+  constexpr int CPB = line_cells_per_block<DIM, NP>();
+  constexpr int NX = NP + 4;  // extended line: values, then v, P of the left and right x-face
+  using Ext = LaneRows<NX, 64, T>;
+  using Row = LaneRows<NP, 64, T>;
+  constexpr int FL = D3 ? NP : 1, FR = ((64 + NL - 1) / NL) * FL, CW = 16 / int(sizeof(T));
+  using Face = LaneRows<NP, FR, T>;
+  constexpr int S1 = Ext::SIZE + 4 * Face::SIZE, S2 = D3 ? 2 * Row::SIZE : 0;
+  __shared__ __align__(16) T buf[S1 > S2 ? S1 : S2];
+  __shared__ __align__(16) T fz[D3 ? 4 * Face::SIZE : 1];
+  T *fy = buf + Ext::SIZE;
+  auto eidx = [](int l, int e) { return ((e / CW) * 64 + l) * CW + e % CW; };
+  auto fidx = [](int k, int r, int e) { return k * Face::SIZE + ((e / CW) * FR + r) * CW + e % CW; };
 
-  const int chunks = (n + TX - 1) / TX;
-  int64_t rid = blockIdx.x;
-  const int chunk = int(rid % chunks);
-  rid /= chunks;
-  const int c1 = int(rid % n);
-  const int c2 = DIM == 3 ? int(rid / n) : 0;
-  const int c0s = chunk * TX;
-  const int64_t nn = int64_t(n) * n;
-  const int64_t row_base = int64_t(c1) * n + (DIM == 3 ? int64_t(c2) * nn : 0);
-
-  // ---- stage rows in LDS (contiguous cells along x)
-  for(int idx = threadIdx.x; idx < NROW * TXH * NDC; idx += blockDim.x)
-  {
-    const int r = idx / (TXH * NDC);
-    const int rem = idx % (TXH * NDC);
-    const int hc = rem / NDC, l = rem % NDC;
-    const int c0 = c0s - 1 + hc;
-    int64_t base = -1;
-    if(c0 >= 0 && c0 < n)
-    {
-      if(r == 0)
-        base = row_base + c0;
-      else if(r == 1 && c1 > 0)
-        base = row_base - n + c0;
-      else if(r == 2 && c1 < n - 1)
-        base = row_base + n + c0;
-      else if(r == 3 && c2 > 0)
-        base = row_base - nn + c0;
-      else if(r == 4 && c2 < n - 1)
-        base = row_base + nn + c0;
-    }
-    xs[r][hc][l] = base >= 0 ? CT(x[base * NDC + l]) : CT(0);
-  }
-  __syncthreads();
-
-  const int cs = threadIdx.x / NDC, li = threadIdx.x % NDC;
-  const bool in_block = cs < TX;
-  const int csafe = in_block ? cs : 0;
-  const int c0 = c0s + csafe;
-  const bool active = in_block && c0 < n;
-  int lid[3] = {0, 0, 0};
-  {
-    int t = li;
-    for(int d = 0; d < DIM; ++d)
-    {
-      lid[d] = t % NP;
-      t /= NP;
-    }
-  }
-  const int cid[3] = {c0, c1, c2};
-  constexpr int LS[3] = {1, NP, NP * NP};
-
-  // ---- 1D line operators z_d
-#pragma unroll
-  for(int d = 0; d < DIM; ++d)
-  {
-    const bool has_l = cid[d] > 0, has_r = cid[d] < n - 1;
-    const CT *D = tab.D[(has_l ? 1 : 0) | (has_r ? 2 : 0)];
-    const int i = lid[d];
-    const int base = li - i * LS[d];
-    const CT *own = xs[0][csafe + 1];
-    const CT *lft = d == 0 ? xs[0][csafe] : xs[2 * d - 1][csafe + 1];
-    const CT *rgt = d == 0 ? xs[0][csafe + 2] : xs[2 * d][csafe + 1];
-    CT z = 0;
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-    {
-      const int o = base + j * LS[d];
-      z += D[i * NP + j] * own[o];
-      // outside the domain the staged rows hold zeros
-      z += tab.Fpm[i * NP + j] * lft[o] + tab.Fmp[i * NP + j] * rgt[o];
-    }
-    if(in_block) zs[d][cs][li] = z;
-  }
-  __syncthreads();
-
-  CT out = 0;
-  if(DIM == 2)
-  {
-    const CT *z0 = zs[0][csafe], *z1 = zs[DIM > 1 ? 1 : 0][csafe];
-    const int b1 = li - lid[1] * NP, b0 = li - lid[0];
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-      out += tab.M[lid[1] * NP + j] * z0[b1 + j * NP] + tab.M[lid[0] * NP + j] * z1[b0 + j];
-  }
-  else
-  {
-    const CT *z0 = zs[0][csafe], *z1 = zs[1][csafe], *z2 = zs[DIM - 1][csafe];
-    const int b0 = li - lid[0], b1 = li - lid[1] * NP;
-    CT a = 0, bb = 0;
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-    {
-      a += tab.M[lid[1] * NP + j] * z0[b1 + j * NP] + tab.M[lid[0] * NP + j] * z1[b0 + j];
-      bb += tab.M[lid[0] * NP + j] * z2[b0 + j];
-    }
-    if(in_block)
-    {
-      as[0][cs][li] = a;
-      as[1][cs][li] = bb;
-    }
-    __syncthreads();
-    const CT *a0 = as[0][csafe], *a1 = as[1][csafe];
-    const int b2 = li - lid[2] * NP * NP;
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-      out += tab.M[lid[2] * NP + j] * a0[b2 + j * NP * NP] + tab.M[lid[1] * NP + j] * a1[b1 + j * NP];
-  }
-  if(active)
-  {
-    const int64_t g = (row_base + c0) * NDC + li;
-    if(RESIDUAL)
-      y[g] = VT(CT(b[g]) - out);
-    else
-      y[g] = VT(out);
-  }
-}
-
-// Line-tiled variant (3D): one thread per x-line (ly, lz) of a cell, its NP
-// values in registers.  The x-direction line operator and the x mass
-// contractions stay in registers; the y and z line operators read the cell's
-// own planes from LDS and the face neighbours' planes (NP contiguous rows)
-// from global memory, shared through the cache by the NP threads of a plane:
-//   y = M_z (M_y z_0 + M_x z_1) + M_y M_x z_2,  z_d = line operator along d.
-template<int NP>
-constexpr int lines_cells_per_block()
-{
-  return 256 / (NP * NP);
-}
-
-// At least 4 waves per SIMD: FP64 Q3 fits 128 VGPRs without spills (130 unbounded,
-// 3 waves; 4 waves measured 5 % faster at 64^3).
-template<int NP, typename VT, typename CT, bool RESIDUAL>
-__global__ void __launch_bounds__(256, 4)
-k_sipg_lines(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
-             const OpTab<CT, NP> tab, const int n, const int64_t ncell)
-{
-  constexpr int NL = NP * NP, NDC = NL * NP, CPB = lines_cells_per_block<NP>();
-  __shared__ CT xs[CPB][NDC];  // own cells
-  __shared__ CT zs[CPB][NDC];  // z_0, later M_y z_0 + M_x z_1
-  __shared__ CT ws[CPB][NDC];  // M_x z_2
-  const int cs = threadIdx.x / NL, ln = threadIdx.x % NL;
-  const int ly = ln % NP, lz = ln / NP;
-  const bool in = cs < CPB;
-  const int csafe = in ? cs : 0;
-  const int64_t cell = int64_t(blockIdx.x) * CPB + csafe;
-  const bool act = in && cell < ncell;
-  const int64_t nn = int64_t(n) * n;
-  // 32-bit coordinates (cells < n^3 <= 1000^3 < 2^31): 64-bit divisions by a
-  // run-time n are long instruction sequences
+  const int t = threadIdx.x, cs = t / NL, q = t % NL;
+  const int cr = min(cs, CPB - 1);  // lanes beyond the last cell read its lines
+  const int q0 = q % NP, q1 = q / NP;
+  const int64_t per = int64_t(gridDim.x) / 8;  // the grid is a multiple of eight blocks
+  const int64_t slot = (int64_t(blockIdx.x % 8) * per + blockIdx.x / 8) * CPB + cs;
+  const bool act = cs < CPB && slot < count;
+  const int64_t sl = act ? slot : 0;
+  const int64_t cell = cells ? int64_t(cells[sl]) : sl;
   const int ci = int(cell);
-  const int cx = ci % n, cy = (ci / n) % n, cz = ci / (n * n);
-  const int lofs = NP * ly + NL * lz;  // this line within the cell
-  CT xo[NP];
-  if(act)
-    load_row<NP>(x + cell * NDC + lofs, xo);
+  const int cx = ci % n, cy = (ci / n) % n, cz = D3 ? ci / (n * n) : 0;
+  const bool has[3][2] = {{cx > 0, cx < n - 1}, {cy > 0, cy < n - 1}, {cz > 0, cz < n - 1}};
+  const T *xc = x + cell * NDC;
+  T u[NP], nx[2][NP], fl[DIM - 1][2][NP], bv[NP];
+  load_row<NP>(xc + NP * q, u);
+  load_row<NP>(xc + NP * q + (has[0][0] ? -NDC : 0), nx[0]);
+  load_row<NP>(xc + NP * q + (has[0][1] ? NDC : 0), nx[1]);
+#pragma unroll
+  for(int d = 1; d < DIM; ++d)
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool in = has[d][side];
+      const int st = d == 1 ? NP : NP * NP;
+      const int64_t shift = (d == 1 ? int64_t(n) : int64_t(n) * n) * NDC;
+      const int at = d == 1 ? q0 + NP * NP * q1 : q0 + NP * q1;
+      // absent neighbour: the cell's own line, reversed
+      const T *src = xc + (in ? (side ? shift : -shift) : 0) + at + (in ? 0 : P * st);
+      const int sst = in ? st : -st;
+#pragma unroll
+      for(int j = 0; j < NP; ++j) fl[d - 1][side][j] = src[j * sst];
+    }
+  if constexpr(RESIDUAL) load_row<NP>(b + cell * NDC + NP * q, bv);
+  // lane-indexed rows of the tables (kernel arguments)
+  const T *tk = reinterpret_cast<const T *>(&tab);
+  T M0[NP], L0[NP], M1[NP], L1[NP], g0[2], g1[2];
+#pragma unroll
+  for(int j = 0; j < NP; ++j)
+  {
+    M0[j] = tk[q0 * NP + j];
+    L0[j] = tk[NP * NP + q0 * NP + j];
+    if constexpr(D3)
+    {
+      M1[j] = tk[q1 * NP + j];
+      L1[j] = tk[NP * NP + q1 * NP + j];
+    }
+  }
+#pragma unroll
+  for(int side = 0; side < 2; ++side)
+  {
+    g0[side] = tk[2 * NP * NP + side * NP + q0];
+    g1[side] = D3 ? tk[2 * NP * NP + side * NP + q1] : T(0);
+  }
+
+  // trace (v, P) of a neighbour line r on this cell's face `side`; sg: -1 for the
+  // reflection; w: the cell's own value there
+  auto trace = [&](const T *r, int side, T sg, T w, T &v, T &jp) {
+    T d = 0;
+#pragma unroll
+    for(int j = 0; j < NP; ++j) d += tab.g[1 - side][j] * r[j];
+    v = sg * (side ? r[0] : r[P]);
+    jp = (side ? T(-0.5) : T(0.5)) * (sg * d) + tab.sigma * (w - v);
+  };
+  {
+    T e[NX];
+#pragma unroll
+    for(int i = 0; i < NP; ++i) e[i] = u[i];
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      T r[NP];
+#pragma unroll
+      for(int j = 0; j < NP; ++j) r[j] = has[0][side] ? nx[side][j] : -u[P - j];
+      trace(r, side, T(1), u[side ? P : 0], e[NP + 2 * side], e[NP + 2 * side + 1]);
+    }
+    Ext::put(buf, t, e);
+  }
+  __syncthreads();  // the lines are staged
+#pragma unroll
+  for(int side = 0; side < 2; ++side)
+  {
+    T v, jp;
+    const int r = cs * FL + q1, e = side ? P : 0;
+    trace(fl[0][side], side, has[1][side] ? T(1) : T(-1), buf[eidx(cr * NL + e + NP * q1, q0)], v, jp);
+    fy[fidx(2 * side, r, q0)] = v;
+    fy[fidx(2 * side + 1, r, q0)] = jp;
+    if constexpr(D3)
+    {
+      trace(fl[DIM - 2][side], side, has[2][side] ? T(1) : T(-1),
+            buf[eidx(cr * NL + q1 + NP * e, q0)], v, jp);
+      fz[fidx(2 * side, r, q0)] = v;
+      fz[fidx(2 * side + 1, r, q0)] = jp;
+    }
+  }
+  __syncthreads();
+  // z-face traces contracted along y by the lanes (lx, ly) = (q0, q1)
+  T zt[4];
+  if constexpr(D3)
+#pragma unroll
+    for(int k = 0; k < 4; ++k)
+    {
+      T m = 0;
+#pragma unroll
+      for(int j = 0; j < NP; ++j) m += M1[j] * fz[fidx(k, cs * NP + j, q0)];
+      zt[k] = m;
+    }
+  // y stage
+  T My[NX], Ly[NP];
+#pragma unroll
+  for(int i = 0; i < NX; ++i) My[i] = 0;
+#pragma unroll
+  for(int i = 0; i < NP; ++i) Ly[i] = 0;
+#pragma unroll
+  for(int j = 0; j < NP; ++j)
+  {
+    T r[NX];
+    Ext::get(buf, cr * NL + j + NP * q1, r);
+#pragma unroll
+    for(int i = 0; i < NX; ++i) My[i] += M0[j] * r[i];
+#pragma unroll
+    for(int i = 0; i < NP; ++i) Ly[i] += L0[j] * r[i];
+  }
+#pragma unroll
+  for(int side = 0; side < 2; ++side)
+  {
+    T v[NP], jp[NP];
+    Face::get(fy + 2 * side * Face::SIZE, cs * FL + q1, v);
+    Face::get(fy + (2 * side + 1) * Face::SIZE, cs * FL + q1, jp);
+    const T es = q0 == (side ? P : 0) ? T(1) : T(0), cv = (side ? T(0.5) : T(-0.5)) * g0[side];
+#pragma unroll
+    for(int i = 0; i < NP; ++i) Ly[i] += cv * v[i] + es * jp[i];
+  }
+  // x products
+  T zm[NP], zl[NP], out[NP];
+#pragma unroll
+  for(int i = 0; i < NP; ++i)
+  {
+    T s = T(0.5) * (tab.g[1][i] * My[NP + 2] - tab.g[0][i] * My[NP]), s2 = 0;
+#pragma unroll
+    for(int j = 0; j < NP; ++j)
+    {
+      s += tab.L[i * NP + j] * My[j] + tab.M[i * NP + j] * Ly[j];
+      if(D3) s2 += tab.M[i * NP + j] * My[j];
+    }
+    zm[i] = s;
+    zl[i] = s2;
+  }
+  zm[0] += My[NP + 1];
+  zm[P] += My[NP + 3];
+  if constexpr(D3)
+  {
+    __syncthreads();  // the lines, the y-face rows and the z-face traces are read
+#pragma unroll
+    for(int k = 0; k < 4; ++k) fz[fidx(k, cs * NP + q1, q0)] = zt[k];
+    Row::put(buf, t, zm);
+    Row::put(buf + Row::SIZE, t, zl);
+    __syncthreads();
+    T tz[NP];
+#pragma unroll
+    for(int i = 0; i < NP; ++i) tz[i] = 0;
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      T v[NP], jp[NP];
+      Face::get(fz + 2 * side * Face::SIZE, cs * NP + q0, v);
+      Face::get(fz + (2 * side + 1) * Face::SIZE, cs * NP + q0, jp);
+      const T ez = q1 == (side ? P : 0) ? T(1) : T(0), cv = (side ? T(0.5) : T(-0.5)) * g1[side];
+#pragma unroll
+      for(int i = 0; i < NP; ++i) tz[i] += cv * v[i] + ez * jp[i];
+    }
+#pragma unroll
+    for(int i = 0; i < NP; ++i)
+    {
+      T s = 0;
+#pragma unroll
+      for(int j = 0; j < NP; ++j) s += tab.M[i * NP + j] * tz[j];
+      out[i] = s;
+    }
+#pragma unroll
+    for(int k = 0; k < NP; ++k)
+    {
+      Row::get(buf, cr * NL + q0 + NP * k, zm);
+      Row::get(buf + Row::SIZE, cr * NL + q0 + NP * k, zl);
+#pragma unroll
+      for(int i = 0; i < NP; ++i) out[i] += M1[k] * zm[i] + L1[k] * zl[i];
+    }
+  }
   else
 #pragma unroll
-    for(int i = 0; i < NP; ++i) xo[i] = CT(0);
-  if(in)
-#pragma unroll
-    for(int i = 0; i < NP; ++i) xs[cs][lofs + i] = xo[i];
-
-  // z_0: along x, own line and the x-neighbours' lines
-  CT z0[NP];
-  {
-    const bool hl = cx > 0, hr = cx < n - 1;
-    const CT *D = tab.D[(hl ? 1 : 0) | (hr ? 2 : 0)];
-    CT xl[NP], xr[NP];
-#pragma unroll
-    for(int i = 0; i < NP; ++i) xl[i] = xr[i] = CT(0);
-    if(act && hl) load_row<NP>(x + (cell - 1) * NDC + lofs, xl);
-    if(act && hr) load_row<NP>(x + (cell + 1) * NDC + lofs, xr);
-#pragma unroll
-    for(int i = 0; i < NP; ++i)
-    {
-      CT s = 0;
-#pragma unroll
-      for(int j = 0; j < NP; ++j)
-        s += D[i * NP + j] * xo[j] + tab.Fpm[i * NP + j] * xl[j] + tab.Fmp[i * NP + j] * xr[j];
-      z0[i] = s;
-    }
-  }
-  __syncthreads();  // own cells staged
-
-  // z_1 (along y) and z_2 (along z) for every x-node of this line
-  CT z1[NP], z2[NP];
-  {
-    const bool hl = cy > 0, hr = cy < n - 1;
-    const CT *D = tab.D[(hl ? 1 : 0) | (hr ? 2 : 0)];
-#pragma unroll
-    for(int i = 0; i < NP; ++i)
-    {
-      CT s = 0;
-#pragma unroll
-      for(int j = 0; j < NP; ++j) s += D[ly * NP + j] * xs[csafe][i + NP * j + NL * lz];
-      z1[i] = s;
-    }
-#pragma unroll
-    for(int side = 0; side < 2; ++side)
-    {
-      if(!(act && (side == 0 ? hl : hr))) continue;
-      const CT *F = side == 0 ? tab.Fpm : tab.Fmp;
-      const VT *pn = x + (side == 0 ? cell - n : cell + n) * NDC + NL * lz;
-#pragma unroll
-      for(int j = 0; j < NP; ++j)
-      {
-        CT row[NP];
-        load_row<NP>(pn + NP * j, row);
-        const CT f = F[ly * NP + j];
-#pragma unroll
-        for(int i = 0; i < NP; ++i) z1[i] += f * row[i];
-      }
-    }
-  }
-  {
-    const bool hl = cz > 0, hr = cz < n - 1;
-    const CT *D = tab.D[(hl ? 1 : 0) | (hr ? 2 : 0)];
-#pragma unroll
-    for(int i = 0; i < NP; ++i)
-    {
-      CT s = 0;
-#pragma unroll
-      for(int k = 0; k < NP; ++k) s += D[lz * NP + k] * xs[csafe][i + NP * ly + NL * k];
-      z2[i] = s;
-    }
-#pragma unroll
-    for(int side = 0; side < 2; ++side)
-    {
-      if(!(act && (side == 0 ? hl : hr))) continue;
-      const CT *F = side == 0 ? tab.Fpm : tab.Fmp;
-      const VT *pn = x + (side == 0 ? cell - nn : cell + nn) * NDC + NP * ly;
-#pragma unroll
-      for(int k = 0; k < NP; ++k)
-      {
-        CT row[NP];
-        load_row<NP>(pn + NL * k, row);
-        const CT f = F[lz * NP + k];
-#pragma unroll
-        for(int i = 0; i < NP; ++i) z2[i] += f * row[i];
-      }
-    }
-  }
-  // x mass contractions in registers
-  CT m1[NP], w2[NP];
-#pragma unroll
-  for(int i = 0; i < NP; ++i)
-  {
-    CT s1 = 0, s2 = 0;
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-    {
-      s1 += tab.M[i * NP + j] * z1[j];
-      s2 += tab.M[i * NP + j] * z2[j];
-    }
-    m1[i] = s1;
-    w2[i] = s2;
-  }
-  if(in)
-#pragma unroll
-    for(int i = 0; i < NP; ++i)
-    {
-      zs[cs][lofs + i] = z0[i];
-      ws[cs][lofs + i] = w2[i];
-    }
-  __syncthreads();
-  CT a[NP], bb[NP];
-#pragma unroll
-  for(int i = 0; i < NP; ++i)
-  {
-    CT s = m1[i], s2 = 0;
-#pragma unroll
-    for(int j = 0; j < NP; ++j)
-    {
-      const CT m = tab.M[ly * NP + j];
-      s += m * zs[csafe][i + NP * j + NL * lz];
-      s2 += m * ws[csafe][i + NP * j + NL * lz];
-    }
-    a[i] = s;
-    bb[i] = s2;
-  }
-  __syncthreads();
-  if(in)
-#pragma unroll
-    for(int i = 0; i < NP; ++i) zs[cs][lofs + i] = a[i];
-  __syncthreads();
-  CT out[NP];
-#pragma unroll
-  for(int i = 0; i < NP; ++i)
-  {
-    CT s = bb[i];
-#pragma unroll
-    for(int k = 0; k < NP; ++k) s += tab.M[lz * NP + k] * zs[csafe][i + NP * ly + NL * k];
-    out[i] = s;
-  }
+    for(int i = 0; i < NP; ++i) out[i] = zm[i];
   if(!act) return;
-  if(RESIDUAL)
-  {
-    CT bv[NP];
-    load_row<NP>(b + cell * NDC + lofs, bv);
+  if constexpr(RESIDUAL)
 #pragma unroll
     for(int i = 0; i < NP; ++i) out[i] = bv[i] - out[i];
-  }
-  store_row<NP>(y + cell * NDC + lofs, out);
+  store_row<NP>(y + cell * NDC + NP * q, out);
 }
 
-// Q3 form of k_sipg_lines (NP = 4: a cell's 16 lines are 16 lanes of one wave).
-// The generic form loads the NP rows of every y- and z-neighbour plane in each of
-// the plane's NP lanes, behind a branch per side (about 20 row loads per lane,
-// one memory round trip after another).  Here every lane loads seven rows at
-// once -- its line of the cell and the row at the same position in each of the
-// six face neighbours (absent neighbours read the cell itself and are zeroed by
-// selection) -- and takes the other rows of a neighbour plane from the lanes
-// that loaded them: those of a y-plane are the lanes of its quad (DPP
-// broadcast), those of a z-plane sit 4 lanes apart (staged in LDS, laid out
-// as the neighbour cell).  The 1D
-// tables indexed by a lane-varying row (mass, face coupling, boundary-dependent
-// cell matrices) are read from LDS.  Same arithmetic, in the same order, as
-// k_sipg_lines.  DOT (operator form): also the block's part of x.y in
-// partial[blockIdx.x] (the CG's p.Ap without a second pass over p and Ap).
+// All cells of a 3D Q3 level (NP = 4: a cell's 16 lines are 16 lanes of one wave):
+//   y = M_z (M_y z_0 + M_x z_1) + M_y M_x z_2,  z_d = line operator along d.
+// Every lane loads seven rows at once -- its line of the cell and the row at the same
+// position in each of the six face neighbours (absent neighbours read the cell itself
+// and are zeroed by selection) -- and takes the other rows of a neighbour plane from
+// the lanes that loaded them: those of a y-plane are the lanes of its quad (DPP
+// broadcast), those of a z-plane sit 4 lanes apart (staged in LDS, laid out as the
+// neighbour cell).  The 1D tables indexed by a lane-varying row (mass, face coupling,
+// boundary-dependent cell matrices) are read from LDS.  DOT (operator form): also the
+// block's part of x.y in partial[blockIdx.x] (the CG's p.Ap without a second pass over
+// p and Ap).  64^3: FP32 46 us, FP64 96 us (k_sipg_cells 49 / 97 us, whose strided
+// neighbour lines cost more than its fewer products save at this degree).
 template<typename VT, typename CT, bool RESIDUAL, bool DOT = false>
 __global__ void __launch_bounds__(256, 4)
 k_sipg_lines_q3(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,

@@ -52,38 +52,6 @@ struct ElastTab
   T kappa;                     // -(mu + lambda)
 };
 
-// Rows of N values moved through LDS in 16-byte chunks: chunk k of the row of lane
-// l sits at (k * LANES + l), so that the lanes' accesses are free of bank conflicts.
-template<int N, int LANES, typename T>
-struct LaneRows
-{
-  static constexpr int CW = 16 / int(sizeof(T)), NC = (N + CW - 1) / CW;
-  static constexpr int SIZE = NC * LANES * CW;
-  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
-  static __device__ __forceinline__ void put(T *buf, int lane, const T *v)
-  {
-#pragma unroll
-    for(int k = 0; k < NC; ++k)
-    {
-      vec w;
-#pragma unroll
-      for(int e = 0; e < CW; ++e) w[e] = k * CW + e < N ? v[k * CW + e] : T(0);
-      reinterpret_cast<vec *>(buf)[k * LANES + lane] = w;
-    }
-  }
-  static __device__ __forceinline__ void get(const T *buf, int lane, T *v)
-  {
-#pragma unroll
-    for(int k = 0; k < NC; ++k)
-    {
-      const vec w = reinterpret_cast<const vec *>(buf)[k * LANES + lane];
-#pragma unroll
-      for(int e = 0; e < CW; ++e)
-        if(k * CW + e < N) v[k * CW + e] = w[e];
-    }
-  }
-};
-
 template<int DIM, int NP>
 constexpr int elasticity_cells_per_block()
 {
