@@ -165,14 +165,19 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
       // eight equal shares of blocks, one per XCD
       const unsigned grid = (blocks_for(count, moved_cells_per_block<DIM, NP>()) + 7) / 8 * 8;
       const VT ipg = VT(lv->ip * double(NP - 1) * NP);
-      auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, s, x, y, b, lv->d_vertices.ptr, tab,
+      auto launch = [&](auto kernel, unsigned threads) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, x, y, b, lv->d_vertices.ptr, tab,
                            lv->n, ipg, cells, count);
       };
       if constexpr(DIM == 3)
-        b ? launch(k_sipg_moved<NP, VT, true>) : launch(k_sipg_moved<NP, VT, false>);
+      {
+        if(grid <= kMovedSplitMaxWaves)
+          b ? launch(k_sipg_moved<NP, VT, true, true>, 256) : launch(k_sipg_moved<NP, VT, false, true>, 256);
+        else
+          b ? launch(k_sipg_moved<NP, VT, true, false>, 64) : launch(k_sipg_moved<NP, VT, false, false>, 64);
+      }
       else
-        b ? launch(k_sipg_moved_2d<NP, VT, true>) : launch(k_sipg_moved_2d<NP, VT, false>);
+        b ? launch(k_sipg_moved_2d<NP, VT, true>, 64) : launch(k_sipg_moved_2d<NP, VT, false>, 64);
       TPSS_HIP(hipGetLastError());
     });
     return;

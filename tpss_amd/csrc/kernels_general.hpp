@@ -69,6 +69,9 @@ constexpr int moved_cells_per_block()
   return 64 / cpow(NP, DIM - 1);
 }
 
+// launches of at most this many waves run the split form (a GPU has 1024 SIMDs)
+constexpr int kMovedSplitMaxWaves = 1024;
+
 // 1/a: the hardware reciprocal, in FP64 refined by two Newton steps (within an ulp
 // or two of the correctly rounded quotient)
 __device__ __forceinline__ float fast_recip(float a) { return __builtin_amdgcn_rcpf(a); }
@@ -79,8 +82,11 @@ __device__ __forceinline__ double fast_recip(double a)
   return fma(r, fma(-a, r, 1.0), r);
 }
 
-template<int NP, typename VT, bool RESIDUAL>
-__global__ void __launch_bounds__(64, (std::is_same<VT, float>::value ? 3 : 2))
+// SPLIT: four waves per block of cells, one for the cell term and one per direction of
+// the faces, for launches that leave most of the GPU idle otherwise (the time of a
+// launch is then that of one wave: a color of a 6^3 Q4 FP64 level 27 us unsplit).
+template<int NP, typename VT, bool RESIDUAL, bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? 256 : 64, (SPLIT ? 1 : std::is_same<VT, float>::value ? 3 : 2))
 k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
              const double *__restrict__ vert, const GeneralTab<NP, VT> tab, const int n,
              const VT ipg, const uint32_t *__restrict__ cells, const int64_t count)
@@ -94,8 +100,10 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
   __shared__ T A_[CSL][8][3];            // map coefficients
   __shared__ T N_[CSL][6][4][3];         // normal columns of the neighbours' maps on the faces
   __shared__ __align__(16) T L1[CSL][NDC], L2[CSL][NDC];  // y- and z-face contributions
+  __shared__ __align__(16) T L0[SPLIT ? CSL : 1][NDC];     // x-face contributions of a split block
 
-  const int t = threadIdx.x, cs = t / NL, q = t % NL;
+  const int part = SPLIT ? __builtin_amdgcn_readfirstlane(int(threadIdx.x)) / 64 : 0;
+  const int t = threadIdx.x % 64, cs = t / NL, q = t % NL;
   const int q0 = q % NP, q1 = q / NP;
   const int64_t per = int64_t(gridDim.x) / 8;  // the grid is a multiple of eight blocks
   const int64_t slot = (int64_t(blockIdx.x % 8) * per + blockIdx.x / 8) * CPB + cs;
@@ -113,7 +121,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
       ra[1][r] = 4 * (cs * NL + q0 + NP * ((q1 + r) % NP));
     }
 
-  for(int i = t; i < NTAB; i += 64) tl[i] = reinterpret_cast<const T *>(&tab)[i];
+  for(int i = threadIdx.x; i < NTAB; i += SPLIT ? 256 : 64) tl[i] = reinterpret_cast<const T *>(&tab)[i];
   // ---- loads: lines of the cell and of its face neighbours, vertices
   const T *xc = x + cell * NDC;
   const int at[3] = {NP * q, q0 + NL * q1, q};      // the lane's line along d in a cell
@@ -122,6 +130,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
 #pragma unroll
   for(int d = 0; d < 3; ++d)
   {
+    if(SPLIT && part != d + 1 && !(d == 0 && part == 0)) continue;
     const int64_t shift = (d == 0 ? int64_t(1) : d == 1 ? int64_t(n) : int64_t(n) * n) * NDC;
     const T *pl = xc + at[d] - (cc[d] > 0 ? shift : 0), *pr = xc + at[d] + (cc[d] < n - 1 ? shift : 0);
     if(d == 0)
@@ -143,7 +152,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
     // vertex c < 8: corner c; else the corner of the neighbour across face
     // f = (c - 8) / 4 opposite face corner (c - 8) % 4 (absent neighbour: any vertex)
     const int v1 = n + 1, v2 = v1 * v1, vb = cc[0] + v1 * cc[1] + v2 * cc[2];
-    for(int c = q; c < 32; c += NL)
+    for(int c = q + NL * part; c < 32; c += SPLIT ? 4 * NL : NL)
     {
       const int f = (c - 8) >> 2, d = f >> 1, side = f & 1;
       int o0 = c & 1, o1 = (c >> 1) & 1, o2 = c >> 2;
@@ -170,6 +179,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
 #pragma unroll
     for(int side = 0; side < 2; ++side)
     {
+      if(SPLIT && part != d + 1) continue;
       const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
       T dd = 0, dn = 0;
 #pragma unroll
@@ -185,7 +195,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
     }
   // ---- map coefficients, formed in FP64: item (coordinate a) of the cell, then of
   // the six neighbours' normal columns
-  for(int it = q; it < 21; it += NL)
+  for(int it = q + NL * part; it < 21; it += SPLIT ? 4 * NL : NL)
   {
     const int a = it % 3, f = it / 3 - 1;
     if(f < 0)
@@ -251,6 +261,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
     for(int j = 0; j < NP; ++j) acc[d][j] = 0;
 
   // ---------------- cell term
+  if(!SPLIT || part == 0)
   {
     T F0[NP], F1[NP], F2[NP];
     T g0[NP], g1[NP], g2[NP];
@@ -335,6 +346,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
 #pragma unroll
   for(int d = 0; d < 3; ++d)
   {
+    if(SPLIT && part != d + 1) continue;
     const int bd = 1 << d, b1 = d == 0 ? 2 : 1, b2 = d == 2 ? 2 : 4, b12 = b1 | b2;
     T jd[3];
 #pragma unroll
@@ -438,14 +450,19 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
 #pragma unroll
   for(int j = 0; j < NP; ++j)
   {
-    L1[cs][at[1] + j * st[1]] = acc[1][j];
-    L2[cs][at[2] + j * st[2]] = acc[2][j];
+    if(SPLIT && part == 1) L0[cs][at[0] + j] = acc[0][j];
+    if(!SPLIT || part == 2) L1[cs][at[1] + j * st[1]] = acc[1][j];
+    if(!SPLIT || part == 3) L2[cs][at[2] + j * st[2]] = acc[2][j];
   }
   __syncthreads();
-  if(!act) return;
+  if(!act || part != 0) return;
   T out[NP];
 #pragma unroll
-  for(int j = 0; j < NP; ++j) out[j] = acc[0][j] + L1[cs][NP * q + j] + L2[cs][NP * q + j];
+  for(int j = 0; j < NP; ++j)
+  {
+    out[j] = acc[0][j] + L1[cs][NP * q + j] + L2[cs][NP * q + j];
+    if(SPLIT) out[j] += L0[cs][NP * q + j];
+  }
   if(RESIDUAL)
   {
     T bv[NP];
