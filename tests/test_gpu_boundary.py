@@ -108,7 +108,7 @@ def test_nonfinite_check_of_the_residual_free_passes(dim, p, n):
     """The residual-free color passes check the values they store themselves
     (no separate pass over the output); the additive path and the accumulating
     entry points keep the pass over the output.  (3, 3, 16): colors of at most
-    512 patches run the four-wave pass."""
+    256 patches run the four-wave pass."""
     t = _tpss()
     lv, sm, ref = make(dim, p, n, t.MULTIPLICATIVE)
     N = ref.N

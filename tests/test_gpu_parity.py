@@ -419,7 +419,7 @@ def test_gmg_bf16_reaches_tolerance():
 def test_residual_free_richardson_step(dim, p, n, rev, n_steps):
     """With omega_R = 1 the multiplicative step runs as color passes on (x, b)
     without a residual update; it must match the reference's residual + sweep.
-    3D Q3: colors of up to 512 patches (n = 5) run the four-wave pass, larger
+    3D Q3: colors of up to 256 patches (n = 5) run the four-wave pass, larger
     ones (n = 24: about 760 patches per color) one wave per patch."""
     import tpss_amd as t
     lv, sm, ref = make(dim, p, n, t.MULTIPLICATIVE, reverse=rev, n_steps=n_steps)
@@ -479,8 +479,8 @@ def test_vmult_ignores_the_contents_of_dst(dim, p, n, kw, distorted):
     assert rel_err(host(d), ref.precond_vmult(src)) < 1e-12
 
 
-# 22^3: more than 512 patches per color, the fine-level color pass
-@pytest.mark.parametrize("n", [6, 7, 22])
+# 18^3 and 22^3: more than 256 patches per color, the fine-level color pass
+@pytest.mark.parametrize("n", [6, 7, 18, 22])
 def test_vmult_ignores_the_contents_of_dst_with_patch_damping(n):
     lv, sm, ref = make(3, 3, n, 1)
     omega = 0.8 + 0.4 * np.abs(o.splitmix_uniform(9, ref.P))

@@ -354,7 +354,7 @@ k_patch_mvp_bf16(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<float
 // registers.
 //
 // Bound by HBM: per color of the 64^3 level 42 us FP64 / 22 us FP32 (195 / 97.5 MB
-// compulsory, 222 / 106 MB moved), 57 / 29 us with plane-wise face products
+// compulsory, 216 / 108 MB moved), 57 / 29 us with plane-wise face products
 // (F z along the normal on every node, the masses across lines through LDS) and all
 // eigenvector matrices loaded at once (their scalar registers spilled).
 // ----------------------------------------------------------------------------

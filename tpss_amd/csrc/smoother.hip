@@ -539,11 +539,12 @@ void patch_pass(tpss_smoother *sm, const VT *src, VT *dst, CT *ubuf, int begin, 
 // FD = 1 selects the BF16-MFMA patch solve (3D, Q3)
 // colors of at most this many patches (3D, K = 8) run k_patch_mvp_split: its
 // four waves per patch shorten the pass where a color holds too few patches to
-// fill the GPU (measured per pass, FP32 / FP64: 16^3 cells, about 220 patches
-// per color, 5.1 / 6.1 us against 5.8 / 7.8 us with one wave per patch), and
-// lengthen it where the patches fill the GPU (32^3, about 1860 patches per
-// color: 12.3 / 17.2 against 7.6 / 12.1 us)
-constexpr int kSplitMaxPatches = 512;
+// fill the GPU, and lengthen it where the 256 CUs hold a patch each (sweep from
+// zero, FP32 / FP64 us, against one wave per patch: 4^3 cells FP32 60.6 against 64.0;
+// 16^3, 211 patches per color, 71.6 / 88.9 against 72.4 / 93.6; 18^3, 307 per color,
+// 84.8 / 115.3 against 79.1 / 101.6; 20^3, 429 per color, 90.0 / 126.5 against
+// 80.6 / 103.7)
+constexpr int kSplitMaxPatches = 256;
 
 template<typename VT, typename CT, int FD = 0>
 void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, int x_zero,
