@@ -307,6 +307,35 @@ def test_distorted_operator_block_edges(dim, p, n):
         assert rel_err(host(y)[:ref.N], bs - Ax) < bar
 
 
+# launches beyond the split form (3D Q1-Q3: more than 1024 blocks of 16, 7, 4 cells; 2D: more
+# than 768 blocks of 64 / (p+1) cells in FP32, fewer in FP64), each with a partial last block,
+# and 3D Q4 split at several blocks per CU
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 158), (2, 2, 128), (2, 3, 113), (2, 4, 97), (3, 1, 26),
+                                     (3, 2, 20), (3, 3, 17), (3, 4, 13)])
+def test_distorted_operator_of_large_launches(dim, p, n):
+    test_distorted_operator_block_edges(dim, p, n)
+
+
+# the same forms on lists of cells (the residual of a color, about half of the cells): on
+# uniform vertices the moved-vertex sweep equals the Cartesian one, whose color passes
+# other tests compare with the oracle; one level below and one beyond the split form each
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 20), (2, 1, 222), (2, 2, 180), (2, 3, 157), (2, 4, 21),
+                                     (2, 4, 137), (3, 1, 7), (3, 1, 34), (3, 2, 8), (3, 2, 25),
+                                     (3, 3, 9), (3, 3, 21), (3, 4, 6), (3, 4, 11)])
+def test_distorted_sweep_on_uniform_vertices(dim, p, n):
+    t = _tpss()
+    V = o.uniform_vertices(dim, n)
+    for prec, dt, bar in ((t.F64, np.float64, 1e-12), (t.F32, np.float32, 2e-5)):
+        out = []
+        for vertices in (V, None):
+            lv = t.Level(dim, p, n, ip_factor=2.0, vertices=vertices, precision=prec)
+            sm = t.SchwarzSmoother(lv, t.MULTIPLICATIVE, relaxation=0.9)
+            d = dev(np.full(lv.n_dofs, 7.0, dt), prec)
+            sm.vmult(d, dev(o.splitmix_uniform(6, lv.n_dofs).astype(dt), prec))
+            out.append(host(d))
+        assert rel_err(out[0], out[1]) < bar
+
+
 @pytest.mark.parametrize("dim,p,n,variant", [(2, 3, 6, 0), (3, 3, 4, 0), (3, 2, 5, 1), (3, 4, 3, 0)])
 def test_distorted_smoother_parity(dim, p, n, variant):
     V = o.distorted_vertices(dim, n, 0.15, seed=3)

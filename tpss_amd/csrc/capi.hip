@@ -151,19 +151,21 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
       }
       for(int f = 0; f < 2; ++f)
         for(int i = 0; i < NP; ++i) tab.fd[f][i] = VT(bs.fgrad[i * 2 + f]);
+      const int64_t count = cells ? n_list : lv->ncell;
+      if(count == 0) return;
+      // eight equal shares of blocks, one per XCD
+      const unsigned grid = (blocks_for(count, moved_cells_per_block<DIM, NP>()) + 7) / 8 * 8;
+      const bool split = grid <= moved_split_max_blocks<DIM, NP, VT>();
+      const bool rotated = !(split && moved_row_gathers<NP, true>());
       for(int q = 0; q < NP; ++q)
         for(int r = 0; r < NP; ++r)
         {
-          const int i = (q + r) % NP, at = q * NP + r;
+          const int i = rotated ? (q + r) % NP : r, at = q * NP + r;
           tab.R[0][at] = tab.V[q * NP + i];
           tab.R[1][at] = tab.Dv[q * NP + i];
           tab.R[2][at] = tab.V[i * NP + q];
           tab.R[3][at] = tab.Dv[i * NP + q];
         }
-      const int64_t count = cells ? n_list : lv->ncell;
-      if(count == 0) return;
-      // eight equal shares of blocks, one per XCD
-      const unsigned grid = (blocks_for(count, moved_cells_per_block<DIM, NP>()) + 7) / 8 * 8;
       const VT ipg = VT(lv->ip * double(NP - 1) * NP);
       auto launch = [&](auto kernel, unsigned threads) {
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, s, x, y, b, lv->d_vertices.ptr, tab,
@@ -171,13 +173,15 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
       };
       if constexpr(DIM == 3)
       {
-        if(grid <= kMovedSplitMaxWaves)
+        if(split)
           b ? launch(k_sipg_moved<NP, VT, true, true>, 256) : launch(k_sipg_moved<NP, VT, false, true>, 256);
-        else
+        else if constexpr(NP < 5)
           b ? launch(k_sipg_moved<NP, VT, true, false>, 64) : launch(k_sipg_moved<NP, VT, false, false>, 64);
       }
+      else if(split)
+        b ? launch(k_sipg_moved_2d<NP, VT, true, true>, 320) : launch(k_sipg_moved_2d<NP, VT, false, true>, 320);
       else
-        b ? launch(k_sipg_moved_2d<NP, VT, true>, 64) : launch(k_sipg_moved_2d<NP, VT, false>, 64);
+        b ? launch(k_sipg_moved_2d<NP, VT, true, false>, 64) : launch(k_sipg_moved_2d<NP, VT, false, false>, 64);
       TPSS_HIP(hipGetLastError());
     });
     return;

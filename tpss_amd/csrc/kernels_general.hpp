@@ -16,8 +16,8 @@
 // in registers; products along a lane index take the other lines' values from the
 // lanes that hold them, rotated (lane (q + r) mod NP with coefficient row q of the
 // matrix started at column q), for NP = 4 by DPP (in 3D a cell is a DPP row, its
-// quads the first lane index) and by ds_bpermute otherwise; only the contributions
-// of the y- and z-faces pass through LDS once.
+// quads the first lane index), by ds_bpermute for NP < 4, and for NP = 5 in order through
+// a row in LDS; the contributions of the faces of other directions pass through LDS once.
 //
 // Geometry from the map coefficients A_S.  The two cells of a face share its
 // tangents t1, t2; with w = t1 x t2, a normal-direction Jacobian column J_d of
@@ -29,7 +29,7 @@
 //
 // Bound by VALU issue (3D Q3 FP32: 2471 VALU instructions per wave of four cells).
 // 64^3 Q3 apply: FP32 221 us, FP64 412 us (590 / 1240 us with one thread per node
-// and every product through LDS); 40^3 Q4 283 / 576 us (296 / 640), 60^3 Q2
+// and every product through LDS); 40^3 Q4 217 / 414 us (296 / 640), 60^3 Q2
 // 132 / 244 us (326 / 618), 80^3 Q1 155 / 237 us (578 / 1039).  2D: 300^2 Q3 FP64
 // 17 us (123), 700^2 Q1 FP32 21 us (292).
 #pragma once
@@ -49,9 +49,39 @@ struct GeneralTab
   T Dv[NP * NP];  // Dv[q*NP + i] = phi_i'(x_q)
   T qx[NP], qw[NP];
   T fd[2][NP];    // phi_i'(0), phi_i'(1)
-  // rows of V, Dv and of their transposes rotated to start at the diagonal:
-  // R[m][q*NP + r] = entry (q, (q + r) mod NP)
+  // rows of V, Dv and of their transposes in the order of the lanes' gathers: rotated
+  // to start at the diagonal, R[m][q*NP + r] = entry (q, (q + r) mod NP), or entry (q, r)
+  // where GatherRows serves them (moved_row_gathers)
   T R[4][NP * NP];
+};
+
+// The values of five lanes in order, through a row of a wave's own LDS buffer (a wave's
+// LDS accesses run in order: no barrier).  The rows cost a write and the reads of five
+// values; the four (FP64: eight) ds_bpermute instructions of a rotation, about 8 cycles
+// of the CU's LDS each, bounded the split Q4 form: 9^3 FP64 13.5 -> 9.9 us, 48^3 FP64 1018 ->
+// 712, FP32 503 -> 372.
+template<int ROWS, typename T>
+struct GatherRows
+{
+  static constexpr int W = 16 / int(sizeof(T)), STRIDE = sizeof(T) == 4 ? 8 : 6;  // rows of 16-byte chunks
+  static constexpr int SIZE = ROWS * STRIDE;
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  static __device__ __forceinline__ void gather(T *buf, int row, int at, T v, T *o)
+  {
+    // volatile: the row is read as its five lanes have written it
+    typedef volatile __attribute__((address_space(3))) T *ptr;
+    typedef volatile __attribute__((address_space(3))) vec *vptr;
+    ptr p = (ptr)buf + row * STRIDE;
+    p[at] = v;
+#pragma unroll
+    for(int k = 0; k < 4 / W; ++k)
+    {
+      const vec w = ((vptr)p)[k];
+#pragma unroll
+      for(int e = 0; e < W; ++e) o[W * k + e] = w[e];
+    }
+    o[4] = p[4];
+  }
 };
 
 template<typename T>
@@ -69,8 +99,31 @@ constexpr int moved_cells_per_block()
   return 64 / cpow(NP, DIM - 1);
 }
 
-// launches of at most this many waves run the split form (a GPU has 1024 SIMDs)
-constexpr int kMovedSplitMaxWaves = 1024;
+// Launches of at most this many blocks run the split form (several waves per block of
+// cells, below), whose launch takes as long as its longest wave while the GPU holds all of
+// them at once.  Applies in us, split against one wave per block of cells:
+//   3D Q1-Q3, a wave per SIMD: 24^3 Q1 (864 blocks) FP64 12.6 / 11.3, FP32 8.1 / 9.5; 18^3 Q2
+//   (834) 14.1 / 13.6, 9.4 / 10.5; 22^3 Q2 (1522) 19.8 / 18.6, 11.9 / 12.5; 18^3 Q3 (1458)
+//   16.1 / 17.1, 10.9 / 11.9; 22^3 Q3 (2662) 27.1 / 24.4, 16.5 / 15.7;
+//   3D Q4 always: 12^3 17.2 / 28.8, 10.9 / 16.5; 48^3 712 / 976, 372 / 484 (the one-wave form
+//   spills 36 registers in FP64);
+//   2D FP64: 96^2 Q2 (439) 5.4 / 7.0, 128^2 Q2 (781) 9.3 / 7.5; 64^2 Q3 (256) 4.8 / 5.7, 72^2
+//   Q3 (324) 6.9 / 5.8; 64^2 Q4 (342) 9.1 / 10.3, 80^2 Q4 (534) 12.4 / 11.0;
+//   2D FP32: 96^2 Q3 (576) 4.8 / 4.8, 128^2 Q3 (1024) 5.4 / 4.9; 96^2 Q4 (768) 6.0 / 7.1,
+//   128^2 Q4 (1366) 10.7 / 8.7.
+template<int DIM, int NP, typename VT>
+constexpr unsigned moved_split_max_blocks()
+{
+  if(DIM == 3) return NP == 5 ? ~0u : 1024;
+  return std::is_same<VT, float>::value ? 768 : NP == 4 ? 256 : 512;
+}
+
+// whether the products across lanes take their values in order from GatherRows
+template<int NP, bool SPLIT>
+constexpr bool moved_row_gathers()
+{
+  return NP == 5 && SPLIT;
+}
 
 // 1/a: the hardware reciprocal, in FP64 refined by two Newton steps (within an ulp
 // or two of the correctly rounded quotient)
@@ -82,11 +135,21 @@ __device__ __forceinline__ double fast_recip(double a)
   return fma(r, fma(-a, r, 1.0), r);
 }
 
+// Waves per SIMD the register allocation must allow.  Split FP64 Q4 takes 271 registers
+// unbounded: 12^3 30.7 us with one wave per SIMD, 24.1 with two (both with ds_bpermute).
+template<int NP, typename VT, bool SPLIT>
+constexpr int moved_min_waves()
+{
+  constexpr bool F32 = std::is_same<VT, float>::value;
+  if(SPLIT) return NP < 5 ? 1 : F32 ? 3 : 2;
+  return F32 ? 3 : 2;
+}
+
 // SPLIT: four waves per block of cells, one for the cell term and one per direction of
 // the faces, for launches that leave most of the GPU idle otherwise (the time of a
-// launch is then that of one wave: a color of a 6^3 Q4 FP64 level 27 us unsplit).
+// launch is then that of one wave: 6^3 Q4 FP64 22.2 us unsplit, 7.5 split).
 template<int NP, typename VT, bool RESIDUAL, bool SPLIT>
-__global__ void __launch_bounds__(SPLIT ? 256 : 64, (SPLIT ? 1 : std::is_same<VT, float>::value ? 3 : 2))
+__global__ void __launch_bounds__(SPLIT ? 256 : 64, (moved_min_waves<NP, VT, SPLIT>()))
 k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
              const double *__restrict__ vert, const GeneralTab<NP, VT> tab, const int n,
              const VT ipg, const uint32_t *__restrict__ cells, const int64_t count)
@@ -101,6 +164,10 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
   __shared__ T N_[CSL][6][4][3];         // normal columns of the neighbours' maps on the faces
   __shared__ __align__(16) T L1[CSL][NDC], L2[CSL][NDC];  // y- and z-face contributions
   __shared__ __align__(16) T L0[SPLIT ? CSL : 1][NDC];     // x-face contributions of a split block
+  static_assert(SPLIT || NP < 5, "3D Q4 runs the split form");
+  constexpr bool ROWS = moved_row_gathers<NP, SPLIT>();
+  using GR = GatherRows<CSL * NP, T>;
+  __shared__ __align__(16) T G[ROWS ? 4 * GR::SIZE : 1];
 
   const int part = SPLIT ? __builtin_amdgcn_readfirstlane(int(threadIdx.x)) / 64 : 0;
   const int t = threadIdx.x % 64, cs = t / NL, q = t % NL;
@@ -112,14 +179,27 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
   const int64_t cell = cells ? int64_t(cells[sl]) : sl;
   const int ci = int(cell);
   const int cc[3] = {ci % n, (ci / n) % n, ci / (n * n)};
-  int ra[2][NP];  // ds_bpermute addresses of the rotations (NP != 4)
-  if constexpr(NP != 4)
+  int ra[2][NP];  // ds_bpermute addresses of the rotations (NP < 4)
+  if constexpr(NP < 4)
 #pragma unroll
     for(int r = 0; r < NP; ++r)
     {
       ra[0][r] = 4 * (cs * NL + (q0 + r) % NP + NP * q1);
       ra[1][r] = 4 * (cs * NL + q0 + NP * ((q1 + r) % NP));
     }
+
+  auto gather0 = [&](T v, T *o) {
+    if constexpr(ROWS)
+      GR::gather(G + part * GR::SIZE, cs * NP + q1, q0, v, o);
+    else
+      lane_gather<NP, 0>(v, ra[0], o);
+  };
+  auto gather1 = [&](T v, T *o) {
+    if constexpr(ROWS)
+      GR::gather(G + part * GR::SIZE, cs * NP + q0, q1, v, o);
+    else
+      lane_gather<NP, 1>(v, ra[1], o);
+  };
 
   for(int i = threadIdx.x; i < NTAB; i += SPLIT ? 256 : 64) tl[i] = reinterpret_cast<const T *>(&tab)[i];
   // ---- loads: lines of the cell and of its face neighbours, vertices
@@ -209,7 +289,7 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
         for(int S = 0; S < 8; ++S)
           if((S >> e) & 1) c[S] -= c[S ^ (1 << e)];
 #pragma unroll
-      for(int S = 0; S < 8; ++S) A_[cs][S][a] = T(c[S]);
+      for(int S = 1; S < 8; ++S) A_[cs][S][a] = T(c[S]);
       continue;
     }
     const int d = f >> 1, side = f & 1;
@@ -234,21 +314,29 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
   __syncthreads();
   // For NP >= 4 the lanes' rows of the tables and the map coefficients are read from
   // LDS again for every face (a compiler fence keeps them from staying in registers,
-  // where they spill: 64^3 Q3 FP64 556 us kept, 412 us re-read); shorter lines keep
-  // them (60^3 Q2 FP64 244 us kept, 300 us re-read)
+  // where they spill: 64^3 Q3 FP64 556 us kept, 412 us re-read), in the split form the
+  // transposed rows only ahead of the projections (12^3 Q4 FP32 14.3 -> 13.4 us, FP64 without
+  // its 16 spilled registers); shorter lines keep them (60^3 Q2 FP64 244 us kept, 300 re-read)
   auto rows = [&](int m, int q_, T *o) {
 #pragma unroll
     for(int r = 0; r < NP; ++r) o[r] = tl[2 * NL + 4 * NP + m * NL + q_ * NP + r];
   };
   T A[8][3], Va[NP], Da[NP], VaT[NP], DaT[NP], Vb[NP], Db[NP], VbT[NP], DbT[NP];
+  constexpr bool LATE = SPLIT && NP >= 4;
+  auto fetch_t = [&]() {
+    if(LATE) asm volatile("" ::: "memory");
+    rows(2, q0, VaT), rows(3, q0, DaT);
+    rows(2, q1, VbT), rows(3, q1, DbT);
+  };
   auto fetch = [&]() {
     asm volatile("" ::: "memory");
 #pragma unroll
     for(int S = 1; S < 8; ++S)
 #pragma unroll
       for(int a = 0; a < 3; ++a) A[S][a] = A_[cs][S][a];
-    rows(0, q0, Va), rows(1, q0, Da), rows(2, q0, VaT), rows(3, q0, DaT);
-    rows(0, q1, Vb), rows(1, q1, Db), rows(2, q1, VbT), rows(3, q1, DbT);
+    rows(0, q0, Va), rows(1, q0, Da);
+    rows(0, q1, Vb), rows(1, q1, Db);
+    if constexpr(!LATE) fetch_t();
   };
   fetch();
   const T p0 = tl[2 * NL + q0], p1 = tl[2 * NL + q1];                  // points along the lane indices
@@ -275,13 +363,13 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
         v += tab.V[i * NP + j] * ol[0][j];
         g += tab.Dv[i * NP + j] * ol[0][j];
       }
-      lane_gather<NP, 0>(v, ra[0], rv);
-      lane_gather<NP, 0>(g, ra[0], rg);
-      lane_gather<NP, 1>(dotn<NP>(Va, rg), ra[1], r2);
+      gather0(v, rv);
+      gather0(g, rg);
+      gather1(dotn<NP>(Va, rg), r2);
       g0[i] = dotn<NP>(Vb, r2);
-      lane_gather<NP, 1>(dotn<NP>(Da, rv), ra[1], r2);
+      gather1(dotn<NP>(Da, rv), r2);
       g1[i] = dotn<NP>(Vb, r2);
-      lane_gather<NP, 1>(dotn<NP>(Va, rv), ra[1], r2);
+      gather1(dotn<NP>(Va, rv), r2);
       g2[i] = dotn<NP>(Db, r2);
     }
     // Jacobian columns: J_0 constant along the line, J_1 and J_2 linear in x
@@ -324,17 +412,18 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
       F1[i] = R1[0] * h[0] + R1[1] * h[1] + R1[2] * h[2];
       F2[i] = R2[0] * h[0] + R2[1] * h[1] + R2[2] * h[2];
     }
+    if constexpr(LATE) fetch_t();
 #pragma unroll
     for(int i = 0; i < NP; ++i)
     {
       T r0[NP], r1[NP], r2[NP];
-      lane_gather<NP, 1>(F0[i], ra[1], r0);
-      lane_gather<NP, 1>(F1[i], ra[1], r1);
-      lane_gather<NP, 1>(F2[i], ra[1], r2);
+      gather1(F0[i], r0);
+      gather1(F1[i], r1);
+      gather1(F2[i], r2);
       const T z0 = dotn<NP>(VbT, r0), z1 = dotn<NP>(VbT, r1), z2 = dotn<NP>(DbT, r2);
-      lane_gather<NP, 0>(z0, ra[0], r0);
-      lane_gather<NP, 0>(z1, ra[0], r1);
-      lane_gather<NP, 0>(z2, ra[0], r2);
+      gather0(z0, r0);
+      gather0(z1, r1);
+      gather0(z2, r2);
       const T a0 = dotn<NP>(VaT, r0), a1 = dotn<NP>(DaT, r1) + dotn<NP>(VaT, r2);
 #pragma unroll
       for(int j = 0; j < NP; ++j) acc[0][j] += tab.Dv[i * NP + j] * a0 + tab.V[i * NP + j] * a1;
@@ -362,26 +451,26 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
       T r0[NP], r1[NP], jump, go[3], gn[3];
       {
         T m[NP];
-        lane_gather<NP, 0>(vo[d][side], ra[0], r0);
-        lane_gather<NP, 0>(vn[d][side], ra[0], r1);
+        gather0(vo[d][side], r0);
+        gather0(vn[d][side], r1);
         const T Vo = dotn<NP>(Va, r0), Vn = dotn<NP>(Va, r1);
         const T Do = dotn<NP>(Da, r0), Dn = dotn<NP>(Da, r1);
-        lane_gather<NP, 0>(go_[d][side], ra[0], r0);
-        lane_gather<NP, 0>(gn_[d][side], ra[0], r1);
+        gather0(go_[d][side], r0);
+        gather0(gn_[d][side], r1);
         const T No = dotn<NP>(Va, r0), Nn = dotn<NP>(Va, r1);
-        lane_gather<NP, 1>(Vo, ra[1], r0);
-        lane_gather<NP, 1>(Vn, ra[1], r1);
+        gather1(Vo, r0);
+        gather1(Vn, r1);
         go[2] = dotn<NP>(Db, r0);
         gn[2] = dotn<NP>(Db, r1);
 #pragma unroll
         for(int r = 0; r < NP; ++r) m[r] = r0[r] - r1[r];
         jump = dotn<NP>(Vb, m);
-        lane_gather<NP, 1>(Do, ra[1], r0);
-        lane_gather<NP, 1>(Dn, ra[1], r1);
+        gather1(Do, r0);
+        gather1(Dn, r1);
         go[1] = dotn<NP>(Vb, r0);
         gn[1] = dotn<NP>(Vb, r1);
-        lane_gather<NP, 1>(No, ra[1], r0);
-        lane_gather<NP, 1>(Nn, ra[1], r1);
+        gather1(No, r0);
+        gather1(Nn, r1);
         go[0] = dotn<NP>(Vb, r0);
         gn[0] = dotn<NP>(Vb, r1);
       }
@@ -431,16 +520,17 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
                                                     kn[0] * gn[0] + kn[1] * gn[1] + kn[2] * gn[2]);
       const T hj = -hf * jump;
       // projections on the tangential test functions
+      if constexpr(LATE) fetch_t();
       T ra_[NP], rb[NP], rc[NP];
-      lane_gather<NP, 1>(pa, ra[1], ra_);
-      lane_gather<NP, 1>(hj * ko[2], ra[1], rb);
+      gather1(pa, ra_);
+      gather1(hj * ko[2], rb);
       const T sa = dotn<NP>(VbT, ra_) + dotn<NP>(DbT, rb);
-      lane_gather<NP, 1>(hj * ko[1], ra[1], rb);
-      lane_gather<NP, 1>(hj * ko[0], ra[1], rc);
+      gather1(hj * ko[1], rb);
+      gather1(hj * ko[0], rc);
       const T sb = dotn<NP>(VbT, rb), sc = dotn<NP>(VbT, rc);
-      lane_gather<NP, 0>(sa, ra[0], ra_);
-      lane_gather<NP, 0>(sb, ra[0], rb);
-      lane_gather<NP, 0>(sc, ra[0], rc);
+      gather0(sa, ra_);
+      gather0(sb, rb);
+      gather0(sc, rc);
       const T pv = dotn<NP>(VaT, ra_) + dotn<NP>(DaT, rb), pd = dotn<NP>(VaT, rc);
 #pragma unroll
       for(int j = 0; j < NP; ++j) acc[d][j] += tab.fd[side][j] * pd;
@@ -473,9 +563,10 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
   store_row<NP>(y + cell * NDC + NP * q, out);
 }
 
-// the 2D form: a cell is NP lanes, 64 / NP cells per block
-template<int NP, typename VT, bool RESIDUAL>
-__global__ void __launch_bounds__(64, 2)
+// the 2D form: a cell is NP lanes, 64 / NP cells per block; SPLIT: five waves per block of
+// cells, one for the cell term and one per face
+template<int NP, typename VT, bool RESIDUAL, bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? 320 : 64, (SPLIT ? 1 : 2))
 k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
                 const double *__restrict__ vert, const GeneralTab<NP, VT> tab, const int n,
                 const VT ipg, const uint32_t *__restrict__ cells, const int64_t count)
@@ -486,9 +577,13 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
   __shared__ double X[CSL][12][2];         // corners; far corners of the face neighbours
   __shared__ T A_[CSL][4][2];              // map coefficients
   __shared__ T N_[CSL][4][2][2];           // normal columns of the neighbours' maps on the faces
-  __shared__ __align__(16) T L1[CSL][NDC];  // y-face contributions
+  __shared__ __align__(16) T L1[SPLIT ? 4 : 1][CSL][NDC];  // contributions of the y-faces (SPLIT: of each face)
+  constexpr bool ROWS = moved_row_gathers<NP, SPLIT>();
+  using GR = GatherRows<CSL, T>;
+  __shared__ __align__(16) T G[ROWS ? 5 * GR::SIZE : 1];
 
-  const int t = threadIdx.x, cs = t / NP, q = t % NP;
+  const int part = SPLIT ? __builtin_amdgcn_readfirstlane(int(threadIdx.x)) / 64 : 0;
+  const int t = threadIdx.x % 64, cs = t / NP, q = t % NP;
   const int64_t per = int64_t(gridDim.x) / 8;  // the grid is a multiple of eight blocks
   const int64_t slot = (int64_t(blockIdx.x % 8) * per + blockIdx.x / 8) * CPB + cs;
   const bool act = cs < CPB && slot < count;
@@ -498,12 +593,18 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
   int ra[NP];  // ds_bpermute addresses of the rotations (NP != 4)
 #pragma unroll
   for(int r = 0; r < NP; ++r) ra[r] = 4 * (cs * NP + (q + r) % NP);
+  auto gather = [&](T v, T *o) {
+    if constexpr(ROWS)
+      GR::gather(G + part * GR::SIZE, cs, q, v, o);
+    else
+      lane_gather<NP, 0>(v, ra, o);
+  };
 
   {
     // vertex c < 4: corner c; else the corner of the neighbour across face
     // f = (c - 4) / 2 opposite face corner (c - 4) % 2 (absent neighbour: any vertex)
     const int vb = cc[0] + (n + 1) * cc[1];
-    for(int c = q; c < 12; c += NP)
+    for(int c = q + NP * part; c < 12; c += SPLIT ? 5 * NP : NP)
     {
       const int f = (c - 4) >> 1, d = f >> 1, side = f & 1;
       int o0 = c & 1, o1 = c >> 1;
@@ -525,6 +626,7 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
 #pragma unroll
   for(int d = 0; d < 2; ++d)
   {
+    if(SPLIT && (part + 1) / 2 != d + 1 && !(d == 0 && part == 0)) continue;
     const int at = d == 0 ? NP * q : q, st = d == 0 ? 1 : NP;
     T ol[NP];
 #pragma unroll
@@ -532,6 +634,7 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
 #pragma unroll
     for(int side = 0; side < 2; ++side)
     {
+      if(SPLIT && part != 1 + 2 * d + side) continue;
       const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
       const int64_t shift = (d == 0 ? int64_t(1) : int64_t(n)) * NDC;
       const T *pn = xc + at + (in ? (side ? shift : -shift) : 0);
@@ -568,7 +671,7 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
   __syncthreads();
   // map coefficients, formed in FP64: item (coordinate a) of the cell, then of the
   // four neighbours' normal columns
-  for(int it = q; it < 10; it += NP)
+  for(int it = q + NP * part; it < 10; it += SPLIT ? 5 * NP : NP)
   {
     const int a = it & 1, f = (it >> 1) - 1;
     if(f < 0)
@@ -606,6 +709,7 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
 #pragma unroll
   for(int j = 0; j < NP; ++j) acc[0][j] = acc[1][j] = 0;
   // ---------------- cell term
+  if(!SPLIT || part == 0)
   {
     const T c0[2] = {A[1][0] + p0 * A[3][0], A[1][1] + p0 * A[3][1]};
 #pragma unroll
@@ -618,15 +722,15 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
         v += tab.V[i * NP + j] * u[j];
         g += tab.Dv[i * NP + j] * u[j];
       }
-      lane_gather<NP, 0>(g, ra, r0);
-      lane_gather<NP, 0>(v, ra, r1);
+      gather(g, r0);
+      gather(v, r1);
       const T g0 = dotn<NP>(Va, r0), g1 = dotn<NP>(Da, r1);
       const T c1[2] = {A[2][0] + tab.qx[i] * A[3][0], A[2][1] + tab.qx[i] * A[3][1]};
       const T det = c0[0] * c1[1] - c0[1] * c1[0];
       const T w = wq * tab.qw[i] * fast_recip(fabs(det));
       const T h0 = w * (c1[1] * g0 - c0[1] * g1), h1 = w * (c0[0] * g1 - c1[0] * g0);
-      lane_gather<NP, 0>(c1[1] * h0 - c1[0] * h1, ra, r0);
-      lane_gather<NP, 0>(c0[0] * h1 - c0[1] * h0, ra, r1);
+      gather(c1[1] * h0 - c1[0] * h1, r0);
+      gather(c0[0] * h1 - c0[1] * h0, r1);
       const T a0 = dotn<NP>(VaT, r0), a1 = dotn<NP>(DaT, r1);
 #pragma unroll
       for(int j = 0; j < NP; ++j) acc[0][j] += tab.Dv[i * NP + j] * a0 + tab.V[i * NP + j] * a1;
@@ -639,18 +743,19 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
 #pragma unroll
     for(int side = 0; side < 2; ++side)
     {
+      if(SPLIT && part != 1 + 2 * d + side) continue;
       const int f = 2 * d + side, bd = 1 << d, b1 = 2 >> d;
       const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
       T r0[NP], r1[NP], m[NP], go[2], gn[2];
-      lane_gather<NP, 0>(vo[d][side], ra, r0);
-      lane_gather<NP, 0>(vn[d][side], ra, r1);
+      gather(vo[d][side], r0);
+      gather(vn[d][side], r1);
 #pragma unroll
       for(int r = 0; r < NP; ++r) m[r] = r0[r] - r1[r];
       const T jump = dotn<NP>(Va, m);
       go[1] = dotn<NP>(Da, r0);
       gn[1] = dotn<NP>(Da, r1);
-      lane_gather<NP, 0>(go_[d][side], ra, r0);
-      lane_gather<NP, 0>(gn_[d][side], ra, r1);
+      gather(go_[d][side], r0);
+      gather(gn_[d][side], r1);
       go[0] = dotn<NP>(Va, r0);
       gn[0] = dotn<NP>(Va, r1);
       T t1[2], jd[2], jn[2];
@@ -677,22 +782,30 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
       const T pa = sigma * (nw * wq) * jump -
                    hf * (ko[0] * go[0] + ko[1] * go[1] + kn[0] * gn[0] + kn[1] * gn[1]);
       const T hj = -hf * jump;
-      lane_gather<NP, 0>(pa, ra, r0);
-      lane_gather<NP, 0>(hj * ko[1], ra, r1);
+      gather(pa, r0);
+      gather(hj * ko[1], r1);
       const T pv = dotn<NP>(VaT, r0) + dotn<NP>(DaT, r1);
-      lane_gather<NP, 0>(hj * ko[0], ra, r0);
+      gather(hj * ko[0], r0);
       const T pd = dotn<NP>(VaT, r0);
 #pragma unroll
       for(int j = 0; j < NP; ++j) acc[d][j] += tab.fd[side][j] * pd;
       acc[d][side ? P : 0] += pv;
     }
 #pragma unroll
-  for(int j = 0; j < NP; ++j) L1[cs][q + j * NP] = acc[1][j];
+  for(int j = 0; j < NP; ++j)
+  {
+    if(SPLIT && (part == 1 || part == 2)) L1[part - 1][cs][NP * q + j] = acc[0][j];
+    if(!SPLIT || part > 2) L1[SPLIT ? part - 1 : 0][cs][q + j * NP] = acc[1][j];
+  }
   __syncthreads();
-  if(!act) return;
+  if(!act || part != 0) return;
   T out[NP];
 #pragma unroll
-  for(int j = 0; j < NP; ++j) out[j] = acc[0][j] + L1[cs][NP * q + j];
+  for(int j = 0; j < NP; ++j)
+  {
+    out[j] = acc[0][j] + L1[0][cs][NP * q + j];
+    if constexpr(SPLIT) out[j] += L1[1][cs][NP * q + j] + L1[2][cs][NP * q + j] + L1[3][cs][NP * q + j];
+  }
   if(RESIDUAL)
   {
     T bv[NP];
