@@ -2,6 +2,8 @@
 Tvmult_add (schwarz_preconditioner.h:185-194), the multiplicative sweep with
 the tiled 2^dim colors, and the error paths of the C ABI (non-finite output,
 collapsed cells, CG without convergence)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -171,3 +173,49 @@ def test_collapsed_cell_is_singular():
     with pytest.raises(t.TPSSError) as e:
         t.GMGSolver(2, 2, 2, 2, vertices=V.reshape(-1, 2))
     assert e.value.code == t.E_SINGULAR
+
+
+@pytest.mark.parametrize("variant,distorted", [(0, False), (1, True)])
+def test_step_after_vmult_allocates_nothing(variant, distorted):
+    """vmult from zero needs neither a residual nor a correction vector, but leaves them
+    allocated: a caller may capture the launches of a step on the same handle"""
+    t = _tpss()
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime that the library has loaded
+    p = ctypes.byref
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        t.synchronize()
+        assert hip.hipMemGetInfo(p(free), p(total)) == 0
+        return free.value
+
+    n = 28  # vectors of 4.7 MB, beyond the granularity of a device allocation
+    V = o.distorted_vertices(3, n, 0.1, seed=3) if distorted else None
+    lv = t.Level(3, 2, n, ip_factor=2.0, vertices=V)
+    x0 = o.splitmix_uniform(4, lv.n_dofs)
+    src, x, y = dev(o.splitmix_uniform(3, lv.n_dofs)), dev(x0), dev(x0)
+    sm = t.SchwarzSmoother(lv, variant, relaxation=0.5)
+    sm.vmult(x, src)
+    before = free_bytes()
+    sm.step(y, src)
+    assert free_bytes() == before
+    eager = host(y)
+    # captured right after a vmult on a fresh handle, and replayed between eager steps
+    sm = t.SchwarzSmoother(lv, variant, relaxation=0.5)
+    sm.vmult(x, src)
+    t.synchronize()
+    stream, graph, ex = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreate(p(stream)) == 0
+    assert hip.hipStreamBeginCapture(stream, 0) == 0
+    sm.step(x, src, stream=stream.value)
+    assert hip.hipStreamEndCapture(stream, p(graph)) == 0
+    assert hip.hipGraphInstantiate(p(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        x.upload(x0)
+        assert hip.hipGraphLaunch(ex, stream) == 0
+        np.testing.assert_array_equal(host(x), eager)
+        x.upload(x0)
+        sm.step(x, src)
+        np.testing.assert_array_equal(host(x), eager)
+    assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(stream) == 0

@@ -970,7 +970,11 @@ void smoother_step_any(tpss_smoother *sm, void *dst, const void *src, hipStream_
     if(sm->pass_flag) sm->pass_checked = true;
     return;
   }
+  // the vectors of a step from a given x, also where this call starts from zero and needs
+  // none: a later step on the handle, whose launches a caller may capture, allocates nothing
   const size_t bytes = size_t(lv->N) * elem_size(lv->vec_prec);
+  sm->rich_r.resize(bytes);
+  if(sm->desc.variant == TPSS_MULTIPLICATIVE) sm->tmp2.resize(bytes);
   for(int k = 0; k < sm->desc.n_steps; ++k)
   {
     // from zero the Richardson residual is b itself and, with omega_R = 1, the step
@@ -987,7 +991,6 @@ void smoother_step_any(tpss_smoother *sm, void *dst, const void *src, hipStream_
     {
       // the Richardson residual b - A x is timed with the residual updates
       SectionTimer t(sm, 0, s);
-      sm->rich_r.resize(bytes);
       operator_apply_any(lv, sm->rich_r.ptr, dst, src, nullptr, 0, s);
       r = sm->rich_r.ptr;
     }
