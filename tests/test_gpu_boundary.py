@@ -105,12 +105,13 @@ def test_nonfinite_output_is_reported():
     assert e.value.code == t.E_NONFINITE
 
 
-@pytest.mark.parametrize("dim,p,n", [(3, 3, 6), (3, 2, 4), (3, 3, 16)])
+@pytest.mark.parametrize("dim,p,n", [(3, 3, 6), (3, 2, 4), (3, 3, 16), (3, 3, 19), (3, 1, 5), (3, 4, 3),
+                                     (2, 3, 7), (2, 1, 9), (2, 4, 5)])
 def test_nonfinite_check_of_the_residual_free_passes(dim, p, n):
     """The residual-free color passes check the values they store themselves
-    (no separate pass over the output); the additive path and the accumulating
-    entry points keep the pass over the output.  (3, 3, 16): colors of at most
-    256 patches run the four-wave pass."""
+    (no separate pass over the output); the accumulating entry points keep the
+    pass over the output.  3D Q3: colors of at most 256 patches (n = 6, 16) run
+    the four-wave pass, larger ones (n = 19) one wave per patch."""
     t = _tpss()
     lv, sm, ref = make(dim, p, n, t.MULTIPLICATIVE)
     N = ref.N
@@ -144,6 +145,42 @@ def test_nonfinite_check_of_the_residual_free_passes(dim, p, n):
     sm.precond_vmult(dst, dev(src))
     sm.finite_status()
     assert rel_err(host(dst), ref.precond_vmult(src)) < 1e-12
+
+
+@pytest.mark.parametrize("dim,p,n,ras", [(2, 3, 5, 0), (2, 1, 6, 1), (2, 2, 5, 2), (3, 2, 4, 0), (3, 4, 3, 0),
+                                         (3, 3, 4, 1), (3, 1, 5, 2)])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_nonfinite_check_of_the_additive_slot_sum(dim, p, n, ras, prec):
+    """The additive slot sum checks the values it stores (no separate pass over
+    the output), also where it accumulates into dst."""
+    t = _tpss()
+    dt = np.float32 if prec else np.float64
+    lv = t.Level(dim, p, n, precision=prec)
+    N = lv.n_dofs
+    src = o.splitmix_uniform(3, N).astype(dt)
+
+    def reported(sm, call, x, b):
+        call(dev(x, prec), dev(b, prec))
+        try:
+            sm.finite_status()
+        except t.TPSSError as e:
+            assert e.code == t.E_NONFINITE
+            return True
+        return False
+
+    zero = np.zeros(N, dt)
+    for kw in ({}, dict(n_steps=2), dict(damping_factor=0.8)):
+        sm = t.SchwarzSmoother(lv, t.ADDITIVE, ras=ras, relaxation=0.2, **kw)
+        calls = [sm.precond_vmult, sm.vmult_add, sm.Tvmult, sm.vmult, sm.step]
+        for call in calls:
+            assert not reported(sm, call, zero, src)
+            for at, value in ((0, np.nan), (N // 2, np.inf), (N - 1, -np.inf)):
+                bad = src.copy()
+                bad[at] = value
+                assert reported(sm, call, zero, bad)
+                assert not reported(sm, call, zero, src)
+                if call == sm.vmult_add:  # already in dst
+                    assert reported(sm, call, bad, src)
 
 
 def test_gmg_solve_reports_nonfinite_and_no_convergence():
