@@ -541,6 +541,11 @@ def test_color_pass_block_edges(dim, p, n, vec, loc, relax):
     assert (got[ref.N:] == 7.0).all()
 
 
+# FP32 solves of FP64 vectors in the one-wave 3D Q3 pass (more than 256 patches per color)
+def test_color_pass_with_fp32_solves_of_fp64_vectors_on_a_fine_level():
+    test_color_pass_block_edges(3, 3, 18, 0, 1, 0.9)
+
+
 # patch solves with a scatter at the edges of their blocks: 128 / K^2 patches per block
 # (3D), 64 / K (2D), two blocks of threads for FP64 Q4; additive and residual-update
 # multiplicative, FP64, FP32 and FP32 solves of FP64 vectors

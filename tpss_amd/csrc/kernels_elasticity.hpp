@@ -59,8 +59,11 @@ constexpr int elasticity_cells_per_block()
 }
 
 // Waves per SIMD the register allocation must allow (64^3 Q2: FP32 129 us unbounded,
-// 106 us with 3; FP64 290 us unbounded, 231 us with 2).  Longer lines would spill:
-// 3D Q3 FP32 24^3 15.1 us unbounded, 15.8 us with 3.
+// 106 us with 3; FP64 290 us unbounded, 231 us with 2; in FP64 the 31 KB of LDS per block hold
+// it at 1.25).  Three would spill Q3 FP32 (24^3 15.1 us unbounded, 15.8 us with 3).  Q3 FP64
+// spills with 2 (3D 30 registers, 2D 16) and gains from it as soon as the launch fills the
+// GPU: with 2 against 1, 3D 44^3 199 / 210 us, 24^3 41.3 / 43.4, 16^3 15.4 / 13.7; 2D 500^2
+// 47.3 / 52.8, 100^2 6.1 / 5.3.  Q4 FP64 keeps one.
 template<int NP, typename T>
 constexpr int elasticity_min_waves()
 {

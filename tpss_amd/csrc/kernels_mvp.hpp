@@ -367,8 +367,18 @@ struct MvpTab
   CT sigma;
 };
 
+// Waves per SIMD the register allocation must allow.  FP32 solves of FP64 vectors hold
+// FP64 rows beside them and spill 6 registers with six (64^3 sweep 725 us, with five 578,
+// with four 575; with FP64 solves 655).
 template<typename VT, typename CT>
-__global__ void __launch_bounds__(64, (std::is_same<CT, float>::value ? 6 : 2))
+constexpr int mvp_q3_min_waves()
+{
+  if(std::is_same<CT, double>::value) return 2;
+  return std::is_same<VT, float>::value ? 6 : 5;
+}
+
+template<typename VT, typename CT>
+__global__ void __launch_bounds__(64, (mvp_q3_min_waves<VT, CT>()))
 k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<4, CT> tab,
                const uint32_t *__restrict__ vtx, const uint32_t *__restrict__ fac,
                const CT *__restrict__ S_tab, const CT *__restrict__ lam_tab,
