@@ -307,6 +307,25 @@ def test_distorted_operator_block_edges(dim, p, n):
         assert rel_err(host(y)[:ref.N], bs - Ax) < bar
 
 
+# a cell whose edges shrink by 1e-5 from one face to the other: the tangents of the short
+# face have to come from the vertices (in FP32 a sum of two map coefficients, rounded at the
+# long edge's size, turns them by 1e-2); large launches take the one-wave forms
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 4), (2, 3, 4), (2, 4, 4), (2, 2, 128), (3, 1, 4), (3, 2, 4),
+                                     (3, 3, 4), (3, 4, 4), (3, 3, 17)])
+def test_distorted_operator_f32_of_tapered_cells(dim, p, n):
+    t = _tpss()
+    V = o.uniform_vertices(dim, n).reshape((n + 1,) * dim + (dim,))
+    h = 1.0 / n
+    V[..., 1, 2, :2] = [h * (1 + 1e-5), h * (1 + 0.5e-5)]  # vertex (2, 1) next to (1, 1)
+    V = V.reshape(-1, dim)
+    ref = o.Smoother(dim, p, n, ip=2.0, vertices=V)
+    x = o.splitmix_uniform(3, ref.N).astype(np.float32)
+    lv = t.Level(dim, p, n, ip_factor=2.0, vertices=V, precision=t.F32)
+    y = dev(np.zeros(ref.N, np.float32))
+    lv.vmult(y, dev(x))
+    assert rel_err(host(y), ref.operator(x.astype(np.float64))) < 1e-5
+
+
 # launches beyond the split form (3D Q1-Q3: more than 1024 blocks of 16, 7, 4 cells; 2D: more
 # than 768 blocks of 64 / (p+1) cells in FP32, fewer in FP64), each with a partial last block,
 # and 3D Q4 split at several blocks per CU

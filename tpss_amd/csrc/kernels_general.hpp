@@ -118,6 +118,16 @@ constexpr unsigned moved_split_max_blocks()
   return std::is_same<VT, float>::value ? 768 : NP == 4 ? 256 : 512;
 }
 
+// On a face x_d = 0 the tangents are map coefficients of the cell, on x_d = 1 sums of two.
+// In FP32 those are formed in FP64 from the vertices too, like every coefficient: sums of
+// rounded coefficients differ from the neighbour's tangents of the same face (FP32 error of a
+// sweep, 16^2 Q4 5.4e-7 with the sums, 3.2e-7 without; 30^3 Q1 1.02e-7, 0.92e-7).
+template<typename T>
+constexpr bool face_tangents_staged()
+{
+  return std::is_same<T, float>::value;
+}
+
 // whether the products across lanes take their values in order from GatherRows
 template<int NP, bool SPLIT>
 constexpr bool moved_row_gathers()
@@ -161,6 +171,8 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
   __shared__ __align__(16) T tl[NTAB];
   __shared__ double X[CSL][32][3];       // corners; far corners of the face neighbours
   __shared__ T A_[CSL][8][3];            // map coefficients
+  constexpr bool FT = face_tangents_staged<T>();
+  __shared__ T F_[FT ? CSL : 1][3][3][3];  // tangents of the faces x_d = 1
   __shared__ T N_[CSL][6][4][3];         // normal columns of the neighbours' maps on the faces
   __shared__ __align__(16) T L1[CSL][NDC], L2[CSL][NDC];  // y- and z-face contributions
   __shared__ __align__(16) T L0[SPLIT ? CSL : 1][NDC];     // x-face contributions of a split block
@@ -296,20 +308,27 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
     const int m1 = d == 0 ? 2 : 1, m2 = d == 2 ? 2 : 4;  // corner bits along e1, e2
     const bool in = side ? cc[0] * (d == 0) + cc[1] * (d == 1) + cc[2] * (d == 2) < n - 1
                          : cc[0] * (d == 0) + cc[1] * (d == 1) + cc[2] * (d == 2) > 0;
-    double e[4];
+    double e[4], c[4];
 #pragma unroll
     for(int cp = 0; cp < 4; ++cp)
     {
       const int cy = (side << d) | ((cp & 1) ? m1 : 0) | ((cp >> 1) ? m2 : 0);
       // absent neighbour: the cell's own edge (finite; its products are multiplied by 0)
       const double far = in ? X[cs][8 + 4 * f + cp][a] : X[cs][cy ^ (1 << d)][a];
-      const double ed = far - X[cs][cy][a];
+      c[cp] = X[cs][cy][a];
+      const double ed = far - c[cp];
       e[cp] = (side == 1) == in ? ed : -ed;
     }
     N_[cs][f][0][a] = T(e[0]);
     N_[cs][f][1][a] = T(e[1] - e[0]);
     N_[cs][f][2][a] = T(e[2] - e[0]);
     N_[cs][f][3][a] = T(e[3] - e[2] - e[1] + e[0]);
+    if(FT && side == 1)
+    {
+      F_[cs][d][0][a] = T(c[1] - c[0]);
+      F_[cs][d][1][a] = T(c[2] - c[0]);
+      F_[cs][d][2][a] = T(c[3] - c[2] - c[1] + c[0]);
+    }
   }
   __syncthreads();
   // For NP >= 4 the lanes' rows of the tables and the map coefficients are read from
@@ -479,9 +498,15 @@ k_sipg_moved(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
 #pragma unroll
       for(int a = 0; a < 3; ++a)
       {
-        const T s = side ? A[b12][a] + A[7][a] : A[b12][a];
-        t1[a] = (side ? A[b1][a] + A[bd | b1][a] : A[b1][a]) + p1 * s;
-        t2[a] = (side ? A[b2][a] + A[bd | b2][a] : A[b2][a]) + p0 * s;
+        T a1 = A[b1][a], a2 = A[b2][a], a12 = A[b12][a];
+        if(side)
+        {
+          a1 = FT ? F_[cs][d][0][a] : a1 + A[bd | b1][a];
+          a2 = FT ? F_[cs][d][1][a] : a2 + A[bd | b2][a];
+          a12 = FT ? F_[cs][d][2][a] : a12 + A[7][a];
+        }
+        t1[a] = a1 + p1 * a12;
+        t2[a] = a2 + p0 * a12;
         jn[a] = N_[cs][f][0][a] + p0 * N_[cs][f][1][a] + p1 * (N_[cs][f][2][a] + p0 * N_[cs][f][3][a]);
       }
 #pragma unroll
@@ -576,6 +601,8 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
   constexpr int CSL = (64 + NP - 1) / NP;  // cell slots, idle lanes included
   __shared__ double X[CSL][12][2];         // corners; far corners of the face neighbours
   __shared__ T A_[CSL][4][2];              // map coefficients
+  constexpr bool FT = face_tangents_staged<T>();
+  __shared__ T F_[FT ? CSL : 1][2][2];     // tangents of the faces x_d = 1
   __shared__ T N_[CSL][4][2][2];           // normal columns of the neighbours' maps on the faces
   __shared__ __align__(16) T L1[SPLIT ? 4 : 1][CSL][NDC];  // contributions of the y-faces (SPLIT: of each face)
   constexpr bool ROWS = moved_row_gathers<NP, SPLIT>();
@@ -685,18 +712,20 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
     const int d = f >> 1, side = f & 1, m1 = d == 0 ? 2 : 1;
     const int cd = d == 0 ? cc[0] : cc[1];
     const bool in = side ? cd < n - 1 : cd > 0;
-    double e[2];
+    double e[2], c[2];
 #pragma unroll
     for(int cp = 0; cp < 2; ++cp)
     {
       const int cy = (side << d) | (cp ? m1 : 0);
       // absent neighbour: the cell's own edge (finite; its products are multiplied by 0)
       const double far = in ? X[cs][4 + 2 * f + cp][a] : X[cs][cy ^ (1 << d)][a];
-      const double ed = far - X[cs][cy][a];
+      c[cp] = X[cs][cy][a];
+      const double ed = far - c[cp];
       e[cp] = (side == 1) == in ? ed : -ed;
     }
     N_[cs][f][0][a] = T(e[0]);
     N_[cs][f][1][a] = T(e[1] - e[0]);
+    if(FT && side == 1) F_[cs][d][a] = T(c[1] - c[0]);
   }
   __syncthreads();
   T A[4][2];
@@ -762,7 +791,7 @@ k_sipg_moved_2d(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restri
 #pragma unroll
       for(int a = 0; a < 2; ++a)
       {
-        t1[a] = side ? A[b1][a] + A[3][a] : A[b1][a];
+        t1[a] = !side ? A[b1][a] : FT ? F_[cs][d][a] : A[b1][a] + A[3][a];
         jd[a] = A[bd][a] + p0 * A[3][a];
         jn[a] = N_[cs][f][0][a] + p0 * N_[cs][f][1][a];
       }
