@@ -774,82 +774,30 @@ __device__ __forceinline__ CT eig_scale(CT s, CT w, CT lam)
 }
 
 // o = S^T r (forward) and r = S o (backward) along one line, S[a * K + i] =
-// component a of eigenvector i.  even_odd: the first K/2 eigenvectors are
-// symmetric, the last K/2 antisymmetric under the reversal a -> K-1-a (the 1D
-// problems of patches whose two cells have equal lengths and no boundary
-// face), so each product takes two (K/2 x K/2) blocks of S on the folded line
-// r_a +- r_{K-1-a}: half the multiply-adds.  (A compile-time choice: a
-// run-time one keeps the line arrays out of registers.)
-template<int K, bool EVEN_ODD, typename CT>
+// component a of eigenvector i
+template<int K, typename CT>
 __device__ __forceinline__ void s_forward(const CT *S, const CT *r, CT *o)
 {
-  constexpr int P = K / 2;
-  if constexpr(EVEN_ODD)
+#pragma unroll
+  for(int i = 0; i < K; ++i)
   {
-    CT rp[P], rm[P];
+    CT s = 0;
 #pragma unroll
-    for(int a = 0; a < P; ++a)
-    {
-      rp[a] = r[a] + r[K - 1 - a];
-      rm[a] = r[a] - r[K - 1 - a];
-    }
-#pragma unroll
-    for(int k = 0; k < P; ++k)
-    {
-      CT sp = 0, sm = 0;
-#pragma unroll
-      for(int a = 0; a < P; ++a)
-      {
-        sp += S[a * K + k] * rp[a];
-        sm += S[a * K + P + k] * rm[a];
-      }
-      o[k] = sp;
-      o[P + k] = sm;
-    }
-  }
-  else
-  {
-#pragma unroll
-    for(int i = 0; i < K; ++i)
-    {
-      CT s = 0;
-#pragma unroll
-      for(int a = 0; a < K; ++a) s += S[a * K + i] * r[a];
-      o[i] = s;
-    }
+    for(int a = 0; a < K; ++a) s += S[a * K + i] * r[a];
+    o[i] = s;
   }
 }
 
-template<int K, bool EVEN_ODD, typename CT>
+template<int K, typename CT>
 __device__ __forceinline__ void s_backward(const CT *S, const CT *o, CT *r)
 {
-  constexpr int P = K / 2;
-  if constexpr(EVEN_ODD)
+#pragma unroll
+  for(int a = 0; a < K; ++a)
   {
+    CT s = 0;
 #pragma unroll
-    for(int a = 0; a < P; ++a)
-    {
-      CT sp = 0, sm = 0;
-#pragma unroll
-      for(int k = 0; k < P; ++k)
-      {
-        sp += S[a * K + k] * o[k];
-        sm += S[a * K + P + k] * o[P + k];
-      }
-      r[a] = sp + sm;
-      r[K - 1 - a] = sp - sm;
-    }
-  }
-  else
-  {
-#pragma unroll
-    for(int a = 0; a < K; ++a)
-    {
-      CT s = 0;
-#pragma unroll
-      for(int i = 0; i < K; ++i) s += S[a * K + i] * o[i];
-      r[a] = s;
-    }
+    for(int i = 0; i < K; ++i) s += S[a * K + i] * o[i];
+    r[a] = s;
   }
 }
 
@@ -858,6 +806,11 @@ __device__ __forceinline__ void s_backward(const CT *S, const CT *o, CT *r)
 // to the compiler: without that it loads the matrices of all stages at once, which
 // exceeds the scalar registers (in the FP64 K = 8 solve 440 of 1300 VALU instructions
 // saved and restored them).
+// EVEN_ODD: the first K/2 eigenvectors are symmetric, the last K/2 antisymmetric under
+// the reversal a -> K-1-a (the 1D problems of patches whose two cells have equal lengths
+// and no boundary face), so each product takes two (K/2 x K/2) blocks of S on the folded
+// line r_a +- r_{K-1-a}: half the multiply-adds.  (A compile-time choice: a run-time one
+// keeps the line arrays out of registers.)
 template<typename CT>
 __device__ __forceinline__ auto scalar_rows(const CT *p)
 {
@@ -924,27 +877,28 @@ __device__ __forceinline__ void s_backward_scalar(const CT *S, const CT *o, CT *
 //   u = (S_2 x S_1 x S_0) diag(w / (lam_0 + lam_1 + lam_2)) (S_2^T x S_1^T x S_0^T) r.
 // The line direction rotates x -> y -> z -> y -> x through the patch's LDS
 // buffer B (entry (x, y, z) at x + SY y + SZ z: padded strides keep the
-// transposes free of LDS bank conflicts); EO: even-odd products in every
-// direction; SCALAR: the matrices are wave-uniform in global memory.
+// transposes free of LDS bank conflicts); SCALAR: the matrices are wave-uniform in
+// global memory; EO (with SCALAR): even-odd products in every direction.
 // Contains __syncthreads (every thread of the block must call it).
 template<int DIM, int K, typename CT, int SY = K, int SZ = K * K, bool EO = false, bool SCALAR = false>
 __device__ __forceinline__ void fd_lines(CT *r, CT *o, CT *B, const CT *S0, const CT *S1,
                                          const CT *S2, const CT *l0, const CT *l1, const CT *l2,
                                          const CT w, const int t, const bool owner)
 {
+  static_assert(SCALAR || !EO, "even-odd products take the matrices as scalar operands");
   const int ty = DIM > 1 ? t % K : 0;
   const int tz = DIM > 2 ? t / K : 0;
   auto fwd = [](const CT *S, const CT *in, CT *out) {
     if constexpr(SCALAR)
       s_forward_scalar<K, EO>(S, in, out);
     else
-      s_forward<K, EO>(S, in, out);
+      s_forward<K>(S, in, out);
   };
   auto bwd = [](const CT *S, const CT *in, CT *out) {
     if constexpr(SCALAR)
       s_backward_scalar<K, EO>(S, in, out);
     else
-      s_backward<K, EO>(S, in, out);
+      s_backward<K>(S, in, out);
   };
   fwd(S0, r, o);
   if(DIM == 2)
@@ -1130,7 +1084,7 @@ struct PatchFdShape
 // 3D is bound by LDS reads of the matrices and the slot buffer's traffic, 2D by latency.
 // Additive steps (patches, slot sum, check), with one line a lane, staging loops and a
 // separate check in brackets: 48^3 Q4 moved FP32 397 us (537), 64^3 Q3 FP32 338 (491),
-// FP64 713 (848), 128^2 Q3 FP64 12.5 (18.0); 64^3 elastic Q2 FP32 sweep 1697 -> 1493.
+// FP64 713 (848), 128^2 Q3 FP64 12.5 (18.0); 64^3 elastic Q2 FP32 sweep 1724 -> 1534.
 template<int DIM, int K, typename VT, typename CT, int MODE>
 __global__ void __launch_bounds__((PatchFdShape<DIM, K, CT>::THREADS))
 k_patch_fd(const VT *__restrict__ src, VT *__restrict__ dst, CT *__restrict__ ubuf,

@@ -353,10 +353,11 @@ k_patch_mvp_bf16(const VT *__restrict__ b, VT *__restrict__ x, const OpTab<float
 // pass through LDS once to the lanes of the x-lines, which take their M_x product in
 // registers.
 //
-// Bound by HBM: per color of the 64^3 level 42 us FP64 / 22 us FP32 (195 / 97.5 MB
-// compulsory, 216 / 108 MB moved), 57 / 29 us with plane-wise face products
-// (F z along the normal on every node, the masses across lines through LDS) and all
-// eigenvector matrices loaded at once (their scalar registers spilled).
+// Per color of the 64^3 level, mean of a step from a given x: 42.8 us FP64 / 26.2 us FP32
+// (195 / 97.5 MB compulsory, 216 / 108 MB moved: 5.0 / 4.1 TB/s, a large copy reaches 4.85);
+// FP64 is bound by HBM, FP32 by latency and issue as well.  57 / 31 us with plane-wise
+// face products (F z along the normal on every node, the masses across lines through
+// LDS) and all eigenvector matrices loaded at once (their scalar registers spilled).
 // ----------------------------------------------------------------------------
 template<int NP, typename CT>
 struct MvpTab
@@ -546,6 +547,7 @@ k_patch_mvp_q3(const VT *__restrict__ b, VT *__restrict__ x, const MvpTab<4, CT>
 // for the y- and z-faces).  Every global load of the pass is issued before the first
 // wait.  K = 6, 10: one patch per block, the eigenvector matrices as scalar operands;
 // K = 4: four patches per wave, matrices staged in LDS.
+// Q4 spills 100 scalar registers in FP64 and 26 in FP32 (tables, pointers and matrix rows).
 // Sweeps: 48^3 Q4 FP64 759 us (2246 with staging loops, plane-wise face products and a
 // branch per neighbour), 27^3 Q4 FP64 268 (534), 64^3 Q2 FP32 290 (404), 33^3 Q2 FP64 142
 // (181), 100^3 Q1 FP32 408 (472).

@@ -535,8 +535,6 @@ void patch_pass(tpss_smoother *sm, const VT *src, VT *dst, CT *ubuf, int begin, 
   });
 }
 
-// residual-free multiplicative color pass (Cartesian mesh, red-black colors);
-// FD = 1 selects the BF16-MFMA patch solve (3D, Q3)
 // colors of at most this many patches (3D, K = 8) run k_patch_mvp_split: its
 // four waves per patch shorten the pass where a color holds too few patches to
 // fill the GPU, and lengthen it where the 256 CUs hold a patch each (sweep from
@@ -546,6 +544,8 @@ void patch_pass(tpss_smoother *sm, const VT *src, VT *dst, CT *ubuf, int begin, 
 // 80.6 / 103.7)
 constexpr int kSplitMaxPatches = 256;
 
+// residual-free multiplicative color pass (Cartesian mesh, red-black colors);
+// FD = 1 selects the BF16-MFMA patch solve (3D, Q3)
 template<typename VT, typename CT, int FD = 0>
 void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, int x_zero,
                     hipStream_t s)
@@ -559,20 +559,24 @@ void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, i
   const CT relax = CT(sm->desc.relaxation);
   dispatch_dim_np(ls.dim, ls.np, [&](auto D, auto NPc) {
     constexpr int DIM = decltype(D)::value, NP = decltype(NPc)::value, K = 2 * NP;
-    OpTab<CT, NP> tab;
     const Operator1D &op = sm->level->op1d;
-    for(int e = 0; e < NP * NP; ++e)
-    {
-      tab.M[e] = CT(op.M[e]);
-      tab.Fpm[e] = CT(op.Fpm[e]);
-      tab.Fmp[e] = CT(op.Fmp[e]);
-      for(int c = 0; c < 4; ++c) tab.D[c][e] = CT(op.D[c][e]);
-    }
+    // the table of the kernels with plane-wise face products
+    auto op_tab = [&]() {
+      OpTab<CT, NP> tab;
+      for(int e = 0; e < NP * NP; ++e)
+      {
+        tab.M[e] = CT(op.M[e]);
+        tab.Fpm[e] = CT(op.Fpm[e]);
+        tab.Fmp[e] = CT(op.Fmp[e]);
+        for(int c = 0; c < 4; ++c) tab.D[c][e] = CT(op.D[c][e]);
+      }
+      return tab;
+    };
     if constexpr(FD == 1)
     {
       if constexpr(DIM == 3 && K == 8 && std::is_same<CT, float>::value)
         hipLaunchKernelGGL((k_patch_mvp_bf16<VT>), dim3(blocks_for(end - begin, 2)), dim3(128), 0, s,
-                           b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax, begin, end, ls.n,
+                           b, x, op_tab(), ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax, begin, end, ls.n,
                            x_zero);
       else
         throw Error(TPSS_E_UNSUPPORTED, "BF16-MFMA patch solves are built for 3D Q3 (k = 8)");
@@ -584,7 +588,7 @@ void mvp_fused_pass(tpss_smoother *sm, const VT *b, VT *x, int begin, int end, i
         {
           // few patches (coarse levels): one patch over four waves
           hipLaunchKernelGGL((k_patch_mvp_split<VT, CT>), dim3(unsigned(end - begin)), dim3(256),
-                             0, s, b, x, tab, ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax,
+                             0, s, b, x, op_tab(), ls.d_vtx.ptr, ls.d_fac.ptr, S, lam, om, relax,
                              begin, ls.n, x_zero, sm->pass_flag);
           TPSS_HIP(hipGetLastError());
           return;
@@ -706,7 +710,7 @@ void resolve_timings(tpss_smoother *sm)
 // If it is color 0 and color 1 follows on an even number of cells, the two colors'
 // patches tile the mesh like a chessboard: color 1 reads only cells that color 0 has
 // written, and every cell is written before a later color reads it, so x need not be
-// cleared first (64^3 Q3: 22 us of a 914 us FP64 sweep).  Otherwise cells that no
+// cleared first (64^3 Q3 FP64: 22 us beside a sweep of 655).  Otherwise cells that no
 // earlier color reached are read as neighbours and must hold zeros.
 bool chessboard_start(const tpss_smoother *sm, const std::vector<int> &seq)
 {
