@@ -589,7 +589,7 @@ def test_patch_solve_block_edges(dim, p, n, vec, loc):
 # than a block, cells with boundary faces on both sides of a direction; all cells and
 # (tiled colors, whose sweep updates the residual color by color) lists of them
 @pytest.mark.parametrize("dim,p,n", [(2, 1, 2), (2, 1, 9), (2, 2, 5), (2, 3, 8), (2, 4, 7), (3, 1, 2),
-                                     (3, 1, 5), (3, 2, 2), (3, 2, 6), (3, 3, 5), (3, 4, 2), (3, 4, 5)])
+                                     (3, 1, 5), (3, 1, 9), (3, 2, 2), (3, 2, 6), (3, 3, 5), (3, 4, 2), (3, 4, 5)])
 def test_cartesian_operator_block_edges(dim, p, n):
     t = _tpss()
     ref = o.Smoother(dim, p, n, ip=2.0)

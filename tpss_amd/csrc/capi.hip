@@ -208,12 +208,13 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
     const auto tab = make_line_tab<VT, NP>(lv->op1d);
     const int64_t count = cells ? n_list : lv->ncell;
     const unsigned grid = (blocks_for(count, line_cells_per_block<DIM, NP>()) + 7) / 8 * 8;
-    if(b)
-      hipLaunchKernelGGL((k_sipg_cells<DIM, NP, VT, true>), dim3(grid), dim3(64), 0, s, x, y, b, tab,
-                         lv->n, cells, count);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, s, x, y, b, tab, lv->n, cells, count);
+    };
+    if constexpr(DIM == 3 && NP == 2)
+      b ? launch(k_sipg_cells_q1<VT, true>) : launch(k_sipg_cells_q1<VT, false>);
     else
-      hipLaunchKernelGGL((k_sipg_cells<DIM, NP, VT, false>), dim3(grid), dim3(64), 0, s, x, y, b, tab,
-                         lv->n, cells, count);
+      b ? launch(k_sipg_cells<DIM, NP, VT, true>) : launch(k_sipg_cells<DIM, NP, VT, false>);
     TPSS_HIP(hipGetLastError());
   });
 }

@@ -17,6 +17,9 @@
 
 namespace tpss
 {
+template<int V>
+using ic = std::integral_constant<int, V>;
+
 constexpr __host__ __device__ int cpow(int b, int e) { return e == 0 ? 1 : b * cpow(b, e - 1); }
 
 // ----------------------------------------------------------------------------
@@ -238,8 +241,7 @@ struct LaneRows
 // on one XCD, so that neighbours in y and z are mostly found in its L2.
 // Bound by LDS and instruction issue.  In brackets the forms with a thread per node or
 // the neighbour planes' rows in every lane: 33^3 Q2 FP64 residual 9.8 us (12.7), 64^3 Q2
-// FP64 46 (61), 40^3 Q4 FP64 71 (137), 100^3 Q1 FP32 32 (40), 500^2 Q3 FP64 16 (42), 300^2
-// Q4 FP32 9 (25).
+// FP64 46 (61), 40^3 Q4 FP64 71 (137), 500^2 Q3 FP64 16 (42), 300^2 Q4 FP32 9 (25).
 // ----------------------------------------------------------------------------
 template<int NP, typename T>
 struct LineTab
@@ -471,6 +473,142 @@ k_sipg_cells(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict_
 #pragma unroll
     for(int i = 0; i < NP; ++i) out[i] = bv[i] - out[i];
   store_row<NP>(y + cell * NDC + NP * q, out);
+}
+
+// The same operator for 3D Q1: a cell is a quad of lanes, lane (q0, q1) = (l & 1, l >> 1) holds
+// the x-line (y, z) = (q0, q1), the y-face points (x, z) = (q0, q1) and the z-face points
+// (x, y) = (q0, q1), so every exchange is a quad permutation and nothing passes through LDS.
+// With the exchanges through LDS (its 7 KB a wave held FP64 at 5.6 waves per SIMD) FP64 levels
+// of 35 to 52 cells took 4 to 9 % longer than with whole neighbour planes in every lane.
+// Apply in us, planes / LDS / here: 46^3 FP64 6.7 / 7.2 / 6.6, 37^3 FP64 5.0 / 5.2 / 5.0, 110^3
+// FP64 74 / - / 57, FP32 52 / - / 37.
+template<int S0, int S1, int S2, int S3, typename T>
+__device__ __forceinline__ T quad_perm(T v)
+{
+  constexpr int CTRL = S0 | (S1 << 2) | (S2 << 4) | (S3 << 6);
+  if constexpr(sizeof(T) == 4)
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+  else
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true));
+}
+
+template<typename VT, bool RESIDUAL>
+__global__ void __launch_bounds__(64)
+k_sipg_cells_q1(const VT *__restrict__ x, VT *__restrict__ y, const VT *__restrict__ b,
+                const LineTab<2, VT> tab, const int n, const uint32_t *__restrict__ cells,
+                const int64_t count)
+{
+  using T = VT;
+  constexpr int NDC = 8;
+  // values of lane (j, q1), of lane (q0, j), of lane (q1, j) and of lane (j, q0)
+  auto at_y = [](auto J, T v) { constexpr int j = decltype(J)::value; return quad_perm<j, j, 2 + j, 2 + j>(v); };
+  auto at_z = [](auto J, T v) { constexpr int j = decltype(J)::value; return quad_perm<2 * j, 2 * j + 1, 2 * j, 2 * j + 1>(v); };
+  auto at_yz = [](auto J, T v) { constexpr int j = decltype(J)::value; return quad_perm<2 * j, 2 * j, 2 * j + 1, 2 * j + 1>(v); };
+  auto at_xy = [](auto J, T v) { constexpr int j = decltype(J)::value; return quad_perm<j, j + 2, j, j + 2>(v); };
+
+  const int q = threadIdx.x % 4, q0 = q & 1, q1 = q >> 1;
+  const int64_t per = int64_t(gridDim.x) / 8;  // the grid is a multiple of eight blocks
+  const int64_t slot = (int64_t(blockIdx.x % 8) * per + blockIdx.x / 8) * 16 + threadIdx.x / 4;
+  const bool act = slot < count;
+  const int64_t sl = act ? slot : 0;
+  const int64_t cell = cells ? int64_t(cells[sl]) : sl;
+  const int ci = int(cell);
+  const int cc[3] = {ci % n, (ci / n) % n, ci / (n * n)};
+  const T *xc = x + cell * NDC;
+  // the line of the cell and of its x-neighbours; the y- and z-neighbours' lines at the
+  // lane's face points (an absent neighbour: the cell's own line, reversed)
+  T u[2], nb[3][2][2], bv[2];
+  load_row<2>(xc + 2 * q, u);
+#pragma unroll
+  for(int d = 0; d < 3; ++d)
+#pragma unroll
+    for(int side = 0; side < 2; ++side)
+    {
+      const bool in = side ? cc[d] < n - 1 : cc[d] > 0;
+      const int64_t shift = (d == 0 ? int64_t(1) : d == 1 ? int64_t(n) : int64_t(n) * n) * NDC;
+      const int st = 1 << d, at = d == 0 ? 2 * q : d == 1 ? q0 + 4 * q1 : q;
+      const T *src = xc + (in ? (side ? shift : -shift) : 0) + at;
+      const T r0 = src[0], r1 = src[st];
+      nb[d][side][0] = in ? r0 : -r1;
+      nb[d][side][1] = in ? r1 : -r0;
+    }
+  if constexpr(RESIDUAL) load_row<2>(b + cell * NDC + 2 * q, bv);
+  // lane-indexed rows of the tables
+  const bool odd0 = q0 != 0, odd1 = q1 != 0;
+  T M0[2], M1[2], L0[2], L1[2], g0[2], g1[2];
+#pragma unroll
+  for(int j = 0; j < 2; ++j)
+  {
+    M0[j] = odd0 ? tab.M[2 + j] : tab.M[j];
+    M1[j] = odd1 ? tab.M[2 + j] : tab.M[j];
+    L0[j] = odd0 ? tab.L[2 + j] : tab.L[j];
+    L1[j] = odd1 ? tab.L[2 + j] : tab.L[j];
+    g0[j] = odd0 ? tab.g[j][1] : tab.g[j][0];
+    g1[j] = odd1 ? tab.g[j][1] : tab.g[j][0];
+  }
+  // traces (v, P) of the neighbours' lines; w: the cell's own value on the face
+  T v[3][2], jp[3][2];
+  auto trace = [&](int d, int side, T w) {
+    const T *r = nb[d][side];
+    const T dn = tab.g[1 - side][0] * r[0] + tab.g[1 - side][1] * r[1];
+    v[d][side] = side ? r[0] : r[1];
+    jp[d][side] = (side ? T(-0.5) : T(0.5)) * dn + tab.sigma * (w - v[d][side]);
+  };
+  trace(0, 0, u[0]);
+  trace(0, 1, u[1]);
+  // (every lane takes part in the permutations, the selection follows; scalars: a selection
+  // between entries of an array would move the array out of registers)
+  const T y00 = at_y(ic<0>{}, u[0]), y01 = at_y(ic<0>{}, u[1]);
+  const T y10 = at_y(ic<1>{}, u[0]), y11 = at_y(ic<1>{}, u[1]);
+  const T z00 = at_yz(ic<0>{}, u[0]), z01 = at_yz(ic<0>{}, u[1]);
+  const T z10 = at_yz(ic<1>{}, u[0]), z11 = at_yz(ic<1>{}, u[1]);
+  trace(1, 0, odd0 ? y01 : y00);
+  trace(1, 1, odd0 ? y11 : y10);
+  trace(2, 0, odd0 ? z01 : z00);
+  trace(2, 1, odd0 ? z11 : z10);
+  // y stage: masses and L along y of the lines, masses of the x-face traces
+  T My[2], Ly[2], Mv[2], Mp[2], Zv[2], Zp[2];
+#pragma unroll
+  for(int i = 0; i < 2; ++i)
+  {
+    const T r0 = i ? y01 : y00, r1 = i ? y11 : y10;
+    My[i] = M0[0] * r0 + M0[1] * r1;
+    Ly[i] = L0[0] * r0 + L0[1] * r1;
+    Mv[i] = M0[0] * at_y(ic<0>{}, v[0][i]) + M0[1] * at_y(ic<1>{}, v[0][i]);
+    Mp[i] = M0[0] * at_y(ic<0>{}, jp[0][i]) + M0[1] * at_y(ic<1>{}, jp[0][i]);
+    // z-face traces contracted along y by the lanes (x, y) = (q0, q1)
+    Zv[i] = M1[0] * at_z(ic<0>{}, v[2][i]) + M1[1] * at_z(ic<1>{}, v[2][i]);
+    Zp[i] = M1[0] * at_z(ic<0>{}, jp[2][i]) + M1[1] * at_z(ic<1>{}, jp[2][i]);
+  }
+  T tz[2] = {T(0), T(0)};
+#pragma unroll
+  for(int side = 0; side < 2; ++side)
+  {
+    const T es = odd0 == (side == 1) ? T(1) : T(0), cv = (side ? T(0.5) : T(-0.5)) * g0[side];
+    Ly[0] += cv * at_y(ic<0>{}, v[1][side]) + es * at_y(ic<0>{}, jp[1][side]);
+    Ly[1] += cv * at_y(ic<1>{}, v[1][side]) + es * at_y(ic<1>{}, jp[1][side]);
+    const T ez = odd1 == (side == 1) ? T(1) : T(0), cz = (side ? T(0.5) : T(-0.5)) * g1[side];
+    tz[0] += cz * at_xy(ic<0>{}, Zv[side]) + ez * at_xy(ic<0>{}, Zp[side]);
+    tz[1] += cz * at_xy(ic<1>{}, Zv[side]) + ez * at_xy(ic<1>{}, Zp[side]);
+  }
+  // x products, then z
+  T out[2];
+#pragma unroll
+  for(int i = 0; i < 2; ++i)
+  {
+    const T zm = T(0.5) * (tab.g[1][i] * Mv[1] - tab.g[0][i] * Mv[0]) + Mp[i] + tab.L[2 * i] * My[0] +
+                 tab.L[2 * i + 1] * My[1] + tab.M[2 * i] * Ly[0] + tab.M[2 * i + 1] * Ly[1];
+    const T zl = tab.M[2 * i] * My[0] + tab.M[2 * i + 1] * My[1];
+    out[i] = tab.M[2 * i] * tz[0] + tab.M[2 * i + 1] * tz[1];
+    out[i] += M1[0] * at_z(ic<0>{}, zm) + L1[0] * at_z(ic<0>{}, zl);
+    out[i] += M1[1] * at_z(ic<1>{}, zm) + L1[1] * at_z(ic<1>{}, zl);
+  }
+  if(!act) return;
+  if constexpr(RESIDUAL)
+#pragma unroll
+    for(int i = 0; i < 2; ++i) out[i] = bv[i] - out[i];
+  store_row<2>(y + cell * NDC + 2 * q, out);
 }
 
 // All cells of a 3D Q3 level (NP = 4: a cell's 16 lines are 16 lanes of one wave):

@@ -11,9 +11,6 @@
 
 namespace tpss
 {
-template<int V>
-using ic = std::integral_constant<int, V>;
-
 // calls f(ic<dim>, ic<np>) for the supported (dim, p+1) pairs
 template<typename F>
 void dispatch_dim_np(int dim, int np, F &&f)
