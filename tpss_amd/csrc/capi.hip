@@ -59,7 +59,7 @@ template<int NP, typename T>
 ElastTab<NP, T> make_elast_tab(const tpss_level *lv)
 {
   ElastTab<NP, T> tab;
-  const Basis1D bs = make_basis(NP - 1);
+  const Basis1D &bs = lv->basis;
   const double h = lv->h, mu = lv->mu, la = lv->lambda;
   const int p = NP - 1;
   const double sigma = lv->ip * (p == 0 ? 1.0 : double(p) * (p + 1)) / h;
@@ -138,7 +138,7 @@ void operator_apply(const tpss_level *lv, VT *y, const VT *x, const VT *b, const
       constexpr int DIM = decltype(D)::value, NP = decltype(NPc)::value;
       constexpr int NDC = cpow(NP, DIM);
       GeneralTab<NP, VT> tab;
-      const Basis1D bs = make_basis(NP - 1);
+      const Basis1D &bs = lv->basis;
       for(int q = 0; q < NP; ++q)
       {
         tab.qx[q] = VT(bs.qx[q]);
@@ -406,6 +406,7 @@ int tpss_level_create(const tpss_level_desc *desc, tpss_level **out)
       lv->distorted = true;
     }
     lv->op1d = make_operator_1d(lv->p, lv->h, lv->ip);
+    lv->basis = make_basis(lv->p);
     *out = lv.release();
   });
 }

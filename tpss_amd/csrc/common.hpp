@@ -188,4 +188,5 @@ struct tpss_level
   std::vector<double> vertices;            // host copy ((n+1)^dim * dim)
   tpss::DeviceArray<double> d_vertices;
   tpss::Operator1D op1d;
+  tpss::Basis1D basis;  // of degree p, for the operators' tables of every launch
 };

@@ -27,7 +27,7 @@
 // dS = |w|: one reciprocal per cell side and one square root.  At a cell point the
 // reference flux is C^T C grad / |det J| with the adjugate C of J.
 //
-// Bound by VALU issue (3D Q3 FP32: 2471 VALU instructions per wave of four cells).
+// Bound by VALU issue (3D Q3 FP32: 2571 VALU instructions per wave of four cells).
 // 64^3 Q3 apply: FP32 221 us, FP64 412 us (590 / 1240 us with one thread per node
 // and every product through LDS); 40^3 Q4 217 / 414 us (296 / 640), 60^3 Q2
 // 132 / 244 us (326 / 618), 80^3 Q1 155 / 237 us (578 / 1039).  2D: 300^2 Q3 FP64
